@@ -28,14 +28,24 @@
 //   * fp32 accumulation across the whole K in MFMA order.
 //
 // attn_prefill_kernel: causal GQA attention of T query rows at positions pos0 .. pos0+T-1 over
-// the fp16 cache rows [0, pos0 + t] (the chunk's own rows written by attn_prep before it). A
-// work-group takes one kv head and 64 / GQA rows; its 4 waves each own 16 (row, q head) columns
-// of the MFMA and walk the same keys, 64 per iteration staged once in LDS for all of them (K as
-// rows, V transposed so that the P.V operand of 4 keys of one dimension is one 8-byte read).
-// Per 16-key group the decode kernel's per-wave flash step (csrc/attn.hip): S^T = K Q^T with q
-// as f16 high + low parts, the online softmax per column in fp32, O^T += V^T P^T with P as f16
-// high + low parts, so the result is fp32-accurate attention; keys past a row's position are
-// -inf. Every wave covers every key its rows need, so no merge across waves is needed.
+// the cache rows [0, pos0 + t] (the chunk's own rows written by attn_prep before it), f16 or the
+// rotated int8 form. A work-group takes one kv head and the rows whose (row, q head) pairs fill its
+// matrix columns, 16 per tile; its waves walk the same keys, 32 per step, staged in LDS for all of
+// them: S^T = K Q^T with q as f16 high + low parts, an online softmax per column in fp32, O^T += V^T
+// P^T with P as f16 high + low parts, so the result is fp32-accurate attention; keys past a row's
+// position are -inf. What bounds it is the matrix cores and the softmax's vector instructions in
+// turn (two waves per SIMD overlap them in part), at rows of 256 also the LDS reads:
+//   * both products are 16x16x32: P V takes two 16-key score tiles as one operand (the order of
+//     its 32 keys is free), with V^T from LDS rows through the transposing reads;
+//   * at rows of 128 a wave has two column tiles on one set of LDS reads (rows of 256: one, two
+//     would leave one wave per SIMD: 777 rows over 3778 int8 keys 128 -> 200 us);
+//   * a step's keys are loaded two iterations ahead into registers and written to the other LDS
+//     buffer after the products: one barrier per iteration, no wait for the load's latency;
+//   * the accumulators follow the running maximum only when it has risen by more than 2^8, the
+//     f16 parts come from v_cvt_pk_f16_f32 and v_fma_mix_f32.
+// Measured (MI355X, 40 / 8 heads of 128, 2048 rows): 180 -> 86 us, 500 TFLOP/s of attention products
+// or 1.0 PFLOP/s with the low parts (45 % of the matrix cores' time at 98 us, counters); 16 / 2 heads of 256,
+// int8, 777 rows at position 3001: 375 -> 126 us; one step per 16 keys on 16x16x16 products before.
 #include <algorithm>
 #include <string>
 
@@ -437,7 +447,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const uint32_t* __rest
 // ---------------------------------------------------------------------------------------------
 // the chunk's causal attention
 // ---------------------------------------------------------------------------------------------
-typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
 
 struct PrefillAttnArgs {
   const float* attn_q;  // [T][q_heads][HD] fp32
@@ -469,240 +478,400 @@ __device__ __forceinline__ u4_t widen_i8x8(uint32_t x0, uint32_t x1) {
               h2_bits(as_h2(__builtin_amdgcn_perm(hi, x1, 0x04030402u)) - bias)};
 }
 
+// The max over the four lanes l % 16 + 16 k that hold one column's scores: v_permlane16_swap and
+// v_permlane32_swap of x with a copy of itself leave rows (0, 0, 2, 2) / (1, 1, 3, 3) and halves
+// (lo, lo) / (hi, hi) in the two registers (no LDS round trip; assembly as in csrc/attn_dma.h).
+__device__ __forceinline__ void swap16(float& a0, float& a1) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a0), "+v"(a1));
+}
+__device__ __forceinline__ void swap32(float& a0, float& a1) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a0), "+v"(a1));
+}
+// (v_maximum3_f32: fmaxf would quieten each operand first, an instruction per operand)
+__device__ __forceinline__ float max3(float x, float y, float z) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y), z);
+}
+__device__ __forceinline__ float col_max(float x) {
+  float a0 = x, a1 = x;
+  swap16(a0, a1);
+  float b0 = __builtin_elementwise_maximum(a0, a1), b1 = b0;
+  swap32(b0, b1);
+  return __builtin_elementwise_maximum(b0, b1);
+}
+
+// two fp32 values as f16 pairs, high and low parts (v_cvt_pk_f16_f32 rounds to nearest; the
+// remainder v - h is exact in fp32: one v_fma_mix_f32 with neg1 = -1, which the compiler may not
+// know to be -1 - it would make the fma a conversion and a subtraction)
+__device__ __forceinline__ void split_pair(float v0, float v1, float neg1, uint32_t& hi, uint32_t& lo) {
+  const h2_t h = __builtin_convertvector((f2_t{v0, v1}), h2_t);
+  const float l0 = __builtin_fmaf((float)h.x, neg1, v0), l1 = __builtin_fmaf((float)h.y, neg1, v1);
+  hi = h2_bits(h);
+  lo = h2_bits(__builtin_convertvector((f2_t{l0, l1}), h2_t));
+}
+
+// 8 consecutive elements of a cache row as loaded, and as f16
+template <int KV8>
+struct KvPiece {
+  typedef u4_t type;
+  static __device__ __forceinline__ u4_t f16(u4_t v) { return v; }
+};
+template <>
+struct KvPiece<1> {
+  typedef u2_t type;
+  static __device__ __forceinline__ u4_t f16(u2_t v) { return widen_i8x8(v.x, v.y); }
+};
+
 // KV8: the K and V rows are int8 with one fp16 scale per (position, kv head), the attn_prep_kv8
 // form (kv8.cl): the rows are widened exactly to f16 in LDS, a score is scaled by its key's K
-// scale and a weight by its key's V scale before P V (the decode reader's order), and the
-// output stays in the rotated basis (un-rotated by unrotate_rows_kernel).
-template <int HD, int GQA, int KV8>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(PrefillAttnArgs a) {
+// scale and a weight by its key's V scale before P V (the decode reader's order); the output goes
+// to out_rot in the rotated basis and, un-rotated (FWHT(s * y) / 16, kv8.cl:814-860), to attn_out.
+//
+// CT: 16-column tiles per wave, which share every LDS read of K and V; NS: 4 NS waves, wave w
+// taking the column tiles of w % 4 and the keys 32 (w / 4) .. of each 32 NS-key iteration (the NS
+// partial results of a column merge through LDS at the end, in ascending key part).
+template <int HD, int GQA, int KV8, int NC, int CT, int NS>
+__global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_prefill_kernel(PrefillAttnArgs a) {
   constexpr uint32_t KK = HD / 32, NT = HD / 16;
-  constexpr uint32_t RB = 64 / GQA;          // rows per work-group
-  constexpr uint32_t KB = 64;                // keys per iteration
-  constexpr uint32_t KROW = HD + 8;          // padded K row in LDS (f16)
-  constexpr uint32_t ROWB = HD * 2;          // K row bytes
-  constexpr uint32_t VTP = KB + 4;           // V^T row (one dimension over the 64 keys), padded
-  constexpr uint32_t DPT = HD / 8;           // dimensions per staging thread of a key pair
-  __shared__ __align__(16) uint16_t sK[KB * KROW];
-  __shared__ __align__(16) uint16_t sVt[HD * VTP];
-  __shared__ float sKs[KV8 ? KB : 1], sVs[KV8 ? KB : 1];
+  constexpr uint32_t COLS = 16 * CT * NC, RB = COLS / GQA;  // columns and rows per work-group
+  constexpr uint32_t KB = 32 * NS;                      // keys per iteration
+  constexpr uint32_t KROW = HD + 8;   // K row in LDS (f16): 16 rows' 16-byte reads fall on distinct banks
+  constexpr uint32_t VROW = HD + 16;  // V row: the transposing reads of 16 rows' 32 bytes likewise
+  constexpr uint32_t TPR = 2 * NC, CH = HD / (8 * TPR);  // staging threads per row, pieces of 8 elements per thread
+  struct Stage {
+    uint16_t k[KB * KROW];
+    uint16_t v[KB * VROW];
+    float ks[KV8 ? KB : 4], vs[KV8 ? KB : 4];
+  };
+  __shared__ __align__(16) union {
+    Stage st[2];
+    struct {
+      float acc[CT * NT * 4][64], m[CT][64], l[CT][64];
+    } part[NS > 1 ? NC * (NS - 1) : 1];
+  } sm;
   // the last row blocks see the most keys: they are dispatched first, so the short blocks fill
   // the tail of the grid
   const uint32_t j = blockIdx.x, t0 = (gridDim.y - 1u - blockIdx.y) * RB;
-  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, cw = wave % NC, ks = wave / NC;
   const uint32_t qi = lane & 15u, qq = lane >> 4;
-  // this lane's column: pair p = 16 wave + qi -> row t0 + p / GQA, q head j GQA + p % GQA
-  const uint32_t p = 16u * wave + qi, prow = p / GQA, ph = j * GQA + p % GQA;
-  const bool col_live = prow < RB && t0 + prow < a.T;
   const uint32_t rows_here = min(RB, a.T - t0);
   const uint32_t kend = a.pos0 + t0 + rows_here;  // keys [0, kend) cover every row of the block
-  const uint32_t lim = col_live ? a.pos0 + t0 + prow : kend - 1u;  // last key this column sees
-
-  // q as the B operand (f16 high and low parts): column qi, k = 32 kk + 8 qq + e
-  h8_t qh[KK], ql[KK];
-#pragma unroll
-  for (uint32_t kk = 0; kk < KK; ++kk) {
-    float v[8];
-    if (col_live) {
-      const float* qp = a.attn_q + ((size_t)(t0 + prow) * a.q_heads + ph) * HD + 32u * kk + 8u * qq;
-      const f4_t q0 = *reinterpret_cast<const f4_t*>(qp);
-      const f4_t q1 = *reinterpret_cast<const f4_t*>(qp + 4);
-      v[0] = q0.x; v[1] = q0.y; v[2] = q0.z; v[3] = q0.w;
-      v[4] = q1.x; v[5] = q1.y; v[6] = q1.z; v[7] = q1.w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = 0.f;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const half_t h = (half_t)v[e];
-      qh[kk][e] = h;
-      ql[kk][e] = (half_t)(v[e] - (float)h);
-    }
-  }
-
-  float m_run = -INFINITY, l_run = 0.f;
-  f4_t acc[NT];
-#pragma unroll
-  for (uint32_t tt = 0; tt < NT; ++tt) acc[tt] = f4_t{0.f, 0.f, 0.f, 0.f};
-  const size_t hoff = (size_t)j * a.head_stride;
-  // staging: thread t loads key row t >> 2, quarter t & 3 of its K row (f16 bytes in LDS), and
-  // dimensions DPT (t & 7) .. + DPT - 1 of the key pair 2 (t >> 3), 2 (t >> 3) + 1 of V, which it
-  // writes transposed (V^T[dimension][key], a u32 per dimension holding both keys) so that the
-  // A operand of the P.V product (4 consecutive keys of one dimension) is one 8-byte read
-  constexpr uint32_t QB = ROWB / 4u;  // f16 bytes per quarter row
-  const uint32_t srow = t >> 2, squart = t & 3u;
-  const uint32_t vpair = t >> 3, vd0 = DPT * (t & 7u);
-  auto cache_row = [&](uint32_t key) -> size_t {
+  // staging: TPR threads per key row, each its 8-element pieces TPR apart; the next
+  // iteration's rows are in flight in registers while this one's are multiplied, and go to the
+  // other LDS buffer afterwards. A key past kend re-reads the last one (its scores are -inf).
+  const uint32_t srow = t / TPR, sch = t % TPR;
+  auto cache_row = [&](uint32_t kb) -> size_t {
+    const uint32_t key = min(kb + srow, kend - 1u);
     return a.pages ? (size_t)a.pages[key / a.page] * a.page + key % a.page : (size_t)key;
   };
-  for (uint32_t kb = 0; kb < kend; kb += KB) {
-    {
-      const uint32_t key = kb + srow;
-      const bool live = key < kend;
-      const size_t crow = live ? cache_row(key) : 0;
-      const uint32_t vk0 = kb + 2u * vpair;
-      const bool vlive0 = vk0 < kend, vlive1 = vk0 + 1u < kend;
-      const size_t vrow0 = vlive0 ? cache_row(vk0) : 0, vrow1 = vlive1 ? cache_row(vk0 + 1u) : 0;
-      uint16_t vt0[DPT], vt1[DPT];  // dimensions vd0 .. of the pair's two keys (f16 bits)
-      if constexpr (KV8 == 0) {
-        const unsigned char* kp =
-            static_cast<const unsigned char*>(a.kv_k) + (crow * a.row_stride + hoff) * 2u + squart * QB;
+  constexpr uint32_t EB = KV8 ? 1u : 2u;  // bytes per cache element
+  const size_t hoff = (size_t)j * a.head_stride;
+  typename KvPiece<KV8>::type kr[CH], vr[CH];
+  uint16_t ksr = 0, vsr = 0;
+  auto load_tile = [&](size_t crow) {
+    const size_t off = (crow * a.row_stride + hoff) * EB + 8u * EB * sch;
 #pragma unroll
-        for (uint32_t i = 0; i < QB / 16u; ++i) {
-          const u4_t kv = live ? *reinterpret_cast<const u4_t*>(kp + 16u * i) : u4_t{0u, 0u, 0u, 0u};
-          *reinterpret_cast<u4_t*>(reinterpret_cast<unsigned char*>(sK + srow * KROW) + squart * QB + 16u * i) = kv;
-        }
-        const uint16_t* v0 = static_cast<const uint16_t*>(a.kv_v) + vrow0 * a.row_stride + hoff + vd0;
-        const uint16_t* v1 = static_cast<const uint16_t*>(a.kv_v) + vrow1 * a.row_stride + hoff + vd0;
-#pragma unroll
-        for (uint32_t i = 0; i < DPT / 8u; ++i) {
-          const u4_t x0 = vlive0 ? *reinterpret_cast<const u4_t*>(v0 + 8u * i) : u4_t{0u, 0u, 0u, 0u};
-          const u4_t x1 = vlive1 ? *reinterpret_cast<const u4_t*>(v1 + 8u * i) : u4_t{0u, 0u, 0u, 0u};
-#pragma unroll
-          for (uint32_t e = 0; e < 4; ++e) {
-            vt0[8u * i + 2u * e] = (uint16_t)(x0[e] & 0xFFFFu);
-            vt0[8u * i + 2u * e + 1u] = (uint16_t)(x0[e] >> 16);
-            vt1[8u * i + 2u * e] = (uint16_t)(x1[e] & 0xFFFFu);
-            vt1[8u * i + 2u * e + 1u] = (uint16_t)(x1[e] >> 16);
-          }
-        }
-      } else {
-        const unsigned char* kp = static_cast<const unsigned char*>(a.kv_k) + crow * a.row_stride + hoff + squart * (QB / 2u);
-#pragma unroll
-        for (uint32_t i = 0; i < QB / 32u; ++i) {  // 16 int8 -> 32 bytes of f16
-          const u4_t kv = live ? *reinterpret_cast<const u4_t*>(kp + 16u * i) : u4_t{0u, 0u, 0u, 0u};
-          unsigned char* kd = reinterpret_cast<unsigned char*>(sK + srow * KROW) + squart * QB + 32u * i;
-          *reinterpret_cast<u4_t*>(kd) = widen_i8x8(kv.x, kv.y);
-          *reinterpret_cast<u4_t*>(kd + 16) = widen_i8x8(kv.z, kv.w);
-        }
-        const unsigned char* v0 = static_cast<const unsigned char*>(a.kv_v) + vrow0 * a.row_stride + hoff + vd0;
-        const unsigned char* v1 = static_cast<const unsigned char*>(a.kv_v) + vrow1 * a.row_stride + hoff + vd0;
-#pragma unroll
-        for (uint32_t i = 0; i < DPT / 16u; ++i) {  // 16 int8 per load
-          const u4_t x0 = vlive0 ? *reinterpret_cast<const u4_t*>(v0 + 16u * i) : u4_t{0u, 0u, 0u, 0u};
-          const u4_t x1 = vlive1 ? *reinterpret_cast<const u4_t*>(v1 + 16u * i) : u4_t{0u, 0u, 0u, 0u};
-          const u4_t w0[2] = {widen_i8x8(x0.x, x0.y), widen_i8x8(x0.z, x0.w)};
-          const u4_t w1[2] = {widen_i8x8(x1.x, x1.y), widen_i8x8(x1.z, x1.w)};
-#pragma unroll
-          for (uint32_t h = 0; h < 2; ++h)
-#pragma unroll
-            for (uint32_t e = 0; e < 4; ++e) {
-              vt0[16u * i + 8u * h + 2u * e] = (uint16_t)(w0[h][e] & 0xFFFFu);
-              vt0[16u * i + 8u * h + 2u * e + 1u] = (uint16_t)(w0[h][e] >> 16);
-              vt1[16u * i + 8u * h + 2u * e] = (uint16_t)(w1[h][e] & 0xFFFFu);
-              vt1[16u * i + 8u * h + 2u * e + 1u] = (uint16_t)(w1[h][e] >> 16);
-            }
-        }
-        if (squart == 0) {
-          const size_t so = crow * a.sc_row_stride + (size_t)j * a.sc_head_stride;
-          sKs[srow] = live ? h2f(a.k_scale[so]) : 0.f;
-          sVs[srow] = live ? h2f(a.v_scale[so]) : 0.f;
-        }
-      }
-#pragma unroll
-      for (uint32_t d = 0; d < DPT; ++d)
-        *reinterpret_cast<uint32_t*>(sVt + (vd0 + d) * VTP + 2u * vpair) = (uint32_t)vt0[d] | ((uint32_t)vt1[d] << 16);
+    for (uint32_t i = 0; i < CH; ++i) {
+      kr[i] = *reinterpret_cast<const typename KvPiece<KV8>::type*>(static_cast<const unsigned char*>(a.kv_k) + off + 8u * TPR * EB * i);
+      vr[i] = *reinterpret_cast<const typename KvPiece<KV8>::type*>(static_cast<const unsigned char*>(a.kv_v) + off + 8u * TPR * EB * i);
     }
-    lds_barrier();
+    if constexpr (KV8 == 1) {  // (all 8 threads of a row: one address)
+      const size_t so = crow * a.sc_row_stride + (size_t)j * a.sc_head_stride;
+      ksr = a.k_scale[so];
+      vsr = a.v_scale[so];
+    }
+  };
+  auto store_tile = [&](Stage& s) {
 #pragma unroll
-    for (uint32_t grp = 0; grp < KB / 16u; ++grp) {
-      const uint32_t g0 = kb + 16u * grp;
-      if (g0 >= kend) break;  // uniform
-      // scores S^T[key g0 + 4 qq + r][column qi]
-      f4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (uint32_t kk = 0; kk < KK; ++kk) {
-        const h8_t kh = *reinterpret_cast<const h8_t*>(sK + (16u * grp + qi) * KROW + 32u * kk + 8u * qq);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[kk], d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[kk], d, 0, 0, 0);
+    for (uint32_t i = 0; i < CH; ++i) {
+      const uint32_t e = 8u * (sch + TPR * i);
+      *reinterpret_cast<u4_t*>(s.k + srow * KROW + e) = KvPiece<KV8>::f16(kr[i]);
+      *reinterpret_cast<u4_t*>(s.v + srow * VROW + e) = KvPiece<KV8>::f16(vr[i]);
+    }
+    if constexpr (KV8 == 1) {
+      if (sch == 0) {
+        s.ks[srow] = h2f(ksr);
+        s.vs[srow] = h2f(vsr);
       }
-      float sc[4];
-      float mx = -INFINITY;
+    }
+  };
+
+  // the first rows and the page table's entries of the next two iterations go out before q
+  size_t crow = cache_row(KB);
+  const size_t crow2 = cache_row(2u * KB);
+  load_tile(cache_row(0));
+  // a weight is 2^(c s - m) with s the unscaled score: one fma per key, m the running max of c s
+  // (c > 0: a negative scale's sign goes to q; a zero scale keeps -inf times c at -inf)
+  const float sl = a.scale * 1.4426950408889634f, sgn = sl < 0.f ? -1.f : 1.f;
+  const float c = sl == 0.f ? 1e-37f : fabsf(sl);
+  const bool computes = 16u * CT * cw < rows_here * GQA;  // a wave without a live column only stages
+  float neg1 = -1.f;
+  asm("" : "+s"(neg1));
+  // this lane's columns: pair p = 16 (CT cw + ct) + qi -> row t0 + p / GQA, q head j GQA + p % GQA
+  uint32_t prow[CT], ph[CT], lim[CT];
+  bool live[CT];
+  h8_t qh[CT][KK], ql[CT][KK];  // q as the B operand (f16 high and low parts): k = 32 kk + 8 qq + e
 #pragma unroll
-      for (uint32_t r = 0; r < 4; ++r) {
-        const uint32_t key = g0 + 4u * qq + r;
-        float rs = a.scale;
-        if constexpr (KV8 == 1) rs = a.scale * sKs[16u * grp + 4u * qq + r];
-        sc[r] = key <= lim ? d[r] * rs : -INFINITY;
-        mx = fmaxf(mx, sc[r]);
+  for (uint32_t ct = 0; ct < CT; ++ct) {
+    const uint32_t p = 16u * (CT * cw + ct) + qi;
+    prow[ct] = p / GQA;
+    ph[ct] = j * GQA + p % GQA;
+    live[ct] = prow[ct] < rows_here;
+    lim[ct] = live[ct] ? a.pos0 + t0 + prow[ct] : kend - 1u;  // the last key the column sees
+    // (a dead column reads the first row's q and is never written)
+    const float* qp = a.attn_q + ((size_t)(t0 + (live[ct] ? prow[ct] : 0u)) * a.q_heads + ph[ct]) * HD + 8u * qq;
+#pragma unroll
+    for (uint32_t kk = 0; kk < KK; ++kk) {
+      const f4_t q0 = *reinterpret_cast<const f4_t*>(qp + 32u * kk) * sgn;
+      const f4_t q1 = *reinterpret_cast<const f4_t*>(qp + 32u * kk + 4) * sgn;
+      u4_t h, l;
+      uint32_t hh, ll;
+      split_pair(q0.x, q0.y, neg1, hh, ll); h.x = hh; l.x = ll;
+      split_pair(q0.z, q0.w, neg1, hh, ll); h.y = hh; l.y = ll;
+      split_pair(q1.x, q1.y, neg1, hh, ll); h.z = hh; l.z = ll;
+      split_pair(q1.z, q1.w, neg1, hh, ll); h.w = hh; l.w = ll;
+      qh[ct][kk] = __builtin_bit_cast(h8_t, h);
+      ql[ct][kk] = __builtin_bit_cast(h8_t, l);
+    }
+  }
+
+  // m_run: the column's reference exponent. It is raised to the largest c s seen only when that
+  // exceeds it by more than kSlack (weights up to 2^kSlack lose nothing in fp32 or in the f16 high
+  // and low parts), so after a few keys the accumulators are hardly ever rescaled and the maximum
+  // over the column's four lanes hardly ever formed
+  constexpr float kNoKey = -1e30f, kSlack = 8.f;
+  float m_run[CT], l_run[CT];
+  f4_t acc[CT][NT];
+#pragma unroll
+  for (uint32_t ct = 0; ct < CT; ++ct) {
+    m_run[ct] = kNoKey;
+    l_run[ct] = 0.f;
+#pragma unroll
+    for (uint32_t tt = 0; tt < NT; ++tt) acc[ct][tt] = f4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  store_tile(sm.st[0]);
+  load_tile(crow);
+  crow = crow2;
+  lds_barrier();
+  for (uint32_t kb = 0, it = 0; kb < kend; kb += KB, ++it) {
+    const Stage& s = sm.st[it & 1u];
+    const uint32_t g0 = kb + 32u * ks;  // this wave's 32 keys
+    if (computes && (NS == 1 || g0 < kend)) {  // uniform per wave
+      // scores S^T[key g0 + 16 g + 4 qq + r][column qi]
+      f4_t d[CT][2];
+#pragma unroll
+      for (uint32_t ct = 0; ct < CT; ++ct) d[ct][0] = d[ct][1] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (uint32_t kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (uint32_t g = 0; g < 2; ++g) {
+          const h8_t kh = *reinterpret_cast<const h8_t*>(s.k + (32u * ks + 16u * g + qi) * KROW + 32u * kk + 8u * qq);
+#pragma unroll
+          for (uint32_t ct = 0; ct < CT; ++ct) d[ct][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[ct][kk], d[ct][g], 0, 0, 0);
+#pragma unroll
+          for (uint32_t ct = 0; ct < CT; ++ct) d[ct][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[ct][kk], d[ct][g], 0, 0, 0);
+        }
+      f4_t kscale[2], vscale[2];
+      if constexpr (KV8 == 1) {
+#pragma unroll
+        for (uint32_t g = 0; g < 2; ++g) {
+          kscale[g] = *reinterpret_cast<const f4_t*>(s.ks + 32u * ks + 16u * g + 4u * qq);
+          vscale[g] = *reinterpret_cast<const f4_t*>(s.vs + 32u * ks + 16u * g + 4u * qq);
+        }
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run, mx);  // finite: key 0 <= lim for every column
-      const float alpha = expf(m_run - m_new);
-      float w[4];
+      const bool masked = g0 + 31u > a.pos0 + t0;  // uniform: some column does not see every key
+      u4_t bh[CT], bl[CT];
 #pragma unroll
-      for (uint32_t r = 0; r < 4; ++r) w[r] = expf(sc[r] - m_new);
-      l_run = __builtin_fmaf(l_run, alpha, (w[0] + w[1]) + (w[2] + w[3]));
-      m_run = m_new;
-      if (__ballot(alpha != 1.0f)) {
+      for (uint32_t ct = 0; ct < CT; ++ct) {
+        float w[8];
 #pragma unroll
-        for (uint32_t tt = 0; tt < NT; ++tt) acc[tt] *= alpha;
+        for (uint32_t e = 0; e < 8; ++e) {
+          w[e] = d[ct][e / 4][e % 4];
+          if constexpr (KV8 == 1) w[e] *= kscale[e / 4][e % 4];
+        }
+        if (masked) {
+#pragma unroll
+          for (uint32_t e = 0; e < 8; ++e)
+            w[e] = g0 + 16u * (e / 4) + 4u * qq + e % 4 <= lim[ct] ? w[e] : -INFINITY;
+        }
+        const float mx = max3(max3(w[0], w[1], w[2]), max3(w[3], w[4], w[5]), max3(w[6], w[7], w[7])) * c;
+        if (__ballot(mx > m_run[ct] + kSlack)) {
+          const float m_new = fmaxf(m_run[ct], col_max(mx));
+          const float alpha = __builtin_amdgcn_exp2f(m_run[ct] - m_new);
+          m_run[ct] = m_new;
+          l_run[ct] *= alpha;
+#pragma unroll
+          for (uint32_t tt = 0; tt < NT; ++tt) acc[ct][tt] *= alpha;
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(w[e], c, -m_run[ct]));
+        l_run[ct] += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+        if constexpr (KV8 == 1) {
+#pragma unroll
+          for (uint32_t e = 0; e < 8; ++e) w[e] *= vscale[e / 4][e % 4];
+        }
+        uint32_t hh, ll;
+        split_pair(w[0], w[1], neg1, hh, ll); bh[ct].x = hh; bl[ct].x = ll;
+        split_pair(w[2], w[3], neg1, hh, ll); bh[ct].y = hh; bl[ct].y = ll;
+        split_pair(w[4], w[5], neg1, hh, ll); bh[ct].z = hh; bl[ct].z = ll;
+        split_pair(w[6], w[7], neg1, hh, ll); bh[ct].w = hh; bl[ct].w = ll;
       }
-      h4_t bh, bl;
-#pragma unroll
-      for (uint32_t r = 0; r < 4; ++r) {
-        float wv = w[r];
-        if constexpr (KV8 == 1) wv *= sVs[16u * grp + 4u * qq + r];
-        const half_t h = (half_t)wv;
-        bh[r] = h;
-        bl[r] = (half_t)(wv - (float)h);
-      }
+      // O^T += V^T P^T: the products' 32 k are the keys 4 qq + e of the two groups, which is how
+      // the lanes hold the weights; V^T of 4 keys comes from one transposing read (lane 4 jj + h
+      // of a 16-lane group supplies key 4 qq + jj, dims 4 h ..; lane i receives dim i of 4 keys)
+      typedef short v4s_t __attribute__((ext_vector_type(4)));
+      typedef v4s_t __attribute__((address_space(3)))* v4s_lds;
+      const uint16_t* vb = s.v + (32u * ks + 4u * qq + (qi >> 2)) * VROW + 4u * (qi & 3u);
 #pragma unroll
       for (uint32_t tt = 0; tt < NT; ++tt) {
-        const h4_t av = *reinterpret_cast<const h4_t*>(sVt + (16u * tt + qi) * VTP + 16u * grp + 4u * qq);
-        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bh, acc[tt], 0, 0, 0);
-        acc[tt] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bl, acc[tt], 0, 0, 0);
+        const v4s_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_lds)(vb + 16u * tt));
+        const v4s_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s_lds)(vb + 16u * VROW + 16u * tt));
+        const h8_t av = __builtin_bit_cast(h8_t, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (uint32_t ct = 0; ct < CT; ++ct) {
+          acc[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(h8_t, bh[ct]), acc[ct][tt], 0, 0, 0);
+          acc[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(h8_t, bl[ct]), acc[ct][tt], 0, 0, 0);
+        }
       }
     }
-    lds_barrier();  // every wave is done with this iteration's keys before they are replaced
+    // (the other buffer was last read before the previous barrier)
+    if (kb + KB < kend) {
+      store_tile(sm.st[(it + 1u) & 1u]);
+      if (kb + 2u * KB < kend) {
+        load_tile(crow);
+        crow = cache_row(kb + 3u * KB);
+      }
+    }
+    lds_barrier();
   }
-  float l = l_run + __shfl_xor(l_run, 16, 64);
-  l = l + __shfl_xor(l, 32, 64);
-  if (col_live) {
-    if constexpr (KV8 == 1) {
-      float* op = a.out_rot + ((size_t)(t0 + prow) * a.q_heads + ph) * HD;
+
+  float l[CT];
 #pragma unroll
-      for (uint32_t tt = 0; tt < NT; ++tt)
+  for (uint32_t ct = 0; ct < CT; ++ct) {
+    float a0 = l_run[ct], a1 = l_run[ct];
+    swap16(a0, a1);
+    float b0 = a0 + a1, b1 = b0;
+    swap32(b0, b1);
+    l[ct] = b0 + b1;
+  }
+  if constexpr (NS > 1) {
+    // the key parts 1 .. NS - 1 hand their state over through LDS (the staged keys are done with)
+    if (ks) {
+      auto& pt = sm.part[NC * (ks - 1u) + cw];
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) op[16u * tt + 4u * qq + r] = acc[tt][r] / l;
-    } else {
-      uint16_t* op = a.attn_out + (size_t)(t0 + prow) * a.q_heads * HD + (size_t)ph * HD;
+      for (uint32_t ct = 0; ct < CT; ++ct) {
+        pt.m[ct][lane] = m_run[ct];
+        pt.l[ct][lane] = l[ct];
 #pragma unroll
-      for (uint32_t tt = 0; tt < NT; ++tt)
+        for (uint32_t tt = 0; tt < NT; ++tt)
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) op[16u * tt + 4u * qq + r] = f2h(acc[tt][r] / l);
+          for (uint32_t r = 0; r < 4; ++r) pt.acc[(ct * NT + tt) * 4u + r][lane] = acc[ct][tt][r];
+      }
+    }
+    lds_barrier();
+    if (ks) return;
+#pragma unroll
+    for (uint32_t q = 0; q + 1u < NS; ++q) {
+      const auto& pt = sm.part[NC * q + cw];
+#pragma unroll
+      for (uint32_t ct = 0; ct < CT; ++ct) {
+        // (a part without a key of the column: kNoKey, weight 0)
+        const float mq = pt.m[ct][lane], m = fmaxf(m_run[ct], mq);
+        const float f0 = __builtin_amdgcn_exp2f(m_run[ct] - m), f1 = __builtin_amdgcn_exp2f(mq - m);
+        m_run[ct] = m;
+        l[ct] = __builtin_fmaf(pt.l[ct][lane], f1, l[ct] * f0);
+#pragma unroll
+        for (uint32_t tt = 0; tt < NT; ++tt)
+#pragma unroll
+          for (uint32_t r = 0; r < 4; ++r)
+            acc[ct][tt][r] = __builtin_fmaf(pt.acc[(ct * NT + tt) * 4u + r][lane], f1, acc[ct][tt][r] * f0);
+      }
     }
   }
-}
-
-// grid (q_heads, T), 256 lanes: attn_reduce_v2_kv8's un-rotation (kv8.cl:814-860) of one
-// (row, head) output, head_dim 256: unrotate(y) = FWHT(s * y) / 16, then f16
-__global__ __launch_bounds__(256) void unrotate_rows_kernel(const float* __restrict__ in, uint16_t* __restrict__ out,
-                                                            uint32_t q_heads) {
-  __shared__ float xch[256];
-  const uint32_t h = blockIdx.x, row = blockIdx.y, d = threadIdx.x;
-  const size_t off = ((size_t)row * q_heads + h) * 256u;
-  float v1[1] = {kv8_flip(in[off + d], kv8_sign_neg(d))};
-  fwht256<1>(v1, d, xch);
-  out[off + d] = f2h(v1[0] * 0.0625f);
+#pragma unroll
+  for (uint32_t ct = 0; ct < CT; ++ct) {
+    // the lane holds dims 16 tt + 4 qq + r of its column
+    const float inv = 1.0f / l[ct];
+    const size_t o = ((size_t)(t0 + prow[ct]) * a.q_heads + ph[ct]) * HD + 4u * qq;
+#pragma unroll
+    for (uint32_t tt = 0; tt < NT; ++tt) acc[ct][tt] *= inv;
+    if constexpr (KV8 == 1) {
+      if (live[ct]) {
+#pragma unroll
+        for (uint32_t tt = 0; tt < NT; ++tt) *reinterpret_cast<f4_t*>(a.out_rot + o + 16u * tt) = acc[ct][tt];
+      }
+      // FWHT(s * y): the stages h = 1 .. 128 in order, the pair (i, i + h) becoming (a + c, a - c):
+      // h = 1, 2 inside the four values, 4 and 8 across the lane groups, 16 .. 128 across the tiles
+#pragma unroll
+      for (uint32_t tt = 0; tt < NT; ++tt) {
+        f4_t y;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) y[r] = kv8_flip(acc[ct][tt][r], kv8_sign_neg(16u * tt + 4u * qq + r));
+        const f4_t y1 = {y[0] + y[1], y[0] - y[1], y[2] + y[3], y[2] - y[3]};
+        f4_t y2 = {y1[0] + y1[2], y1[1] + y1[3], y1[0] - y1[2], y1[1] - y1[3]};
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+          float a0 = y2[r], a1 = y2[r];
+          swap16(a0, a1);
+          float b0 = (qq & 1u) ? a0 - a1 : a0 + a1, b1 = b0;
+          swap32(b0, b1);
+          y2[r] = (qq & 2u) ? b0 - b1 : b0 + b1;
+        }
+        acc[ct][tt] = y2;
+      }
+#pragma unroll
+      for (uint32_t h = 1; h < NT; h *= 2)
+#pragma unroll
+        for (uint32_t tt = 0; tt < NT; ++tt)
+          if (!(tt & h)) {
+            const f4_t u = acc[ct][tt], v = acc[ct][tt + h];
+            acc[ct][tt] = u + v;
+            acc[ct][tt + h] = u - v;
+          }
+#pragma unroll
+      for (uint32_t tt = 0; tt < NT; ++tt) acc[ct][tt] *= 0.0625f;
+    }
+    if (live[ct]) {
+#pragma unroll
+      for (uint32_t tt = 0; tt < NT; ++tt) {
+        const u2_t w = {(uint32_t)f2h(acc[ct][tt][0]) | ((uint32_t)f2h(acc[ct][tt][1]) << 16),
+                        (uint32_t)f2h(acc[ct][tt][2]) | ((uint32_t)f2h(acc[ct][tt][3]) << 16)};
+        *reinterpret_cast<u2_t*>(a.attn_out + o + 16u * tt) = w;
+      }
+    }
+  }
 }
 
 template <int HD, int GQA, int KV8>
-void launch_prefill_gqa(const PrefillAttnArgs& a, uint32_t kv_heads, hipStream_t st) {
-  constexpr uint32_t RB = 64 / GQA;
-  attn_prefill_kernel<HD, GQA, KV8><<<dim3(kv_heads, (a.T + RB - 1) / RB), 256, 0, st>>>(a);
+void launch_prefill_gqa(const PrefillAttnArgs& a, uint32_t kv_heads, uint32_t cus, hipStream_t st) {
+  // Measured (40 / 8 heads of 128 or 16 / 2 of 256; us): two column tiles per wave where they still give
+  // every CU a work-group (2048 rows: 86 against 97 at one tile); below that the keys in two parts,
+  // which doubles the waves, until one part fills the CUs (777 rows over 3778 int8 keys: 133 against
+  // 175 in one part; 333 rows over 1333: 32 / 44), but not for 64 keys or fewer (64 rows at position
+  // 0: 6.6 / 7.4, int8 12.4 / 14.9); up to 32 columns at rows of 128 two column tiles and the keys in
+  // four parts (3 rows over 8003: 77 / 131; 6 over 506: 11.1 / 13.5).
+  constexpr int CT = HD == 128 ? 2 : 1;
+  constexpr uint32_t RB = 64 * CT / GQA, R1 = 64 / GQA;
+  const uint32_t wide = kv_heads * ((a.T + RB - 1) / RB), narrow = kv_heads * ((a.T + R1 - 1) / R1);
+  if (CT > 1 && wide > cus)
+    attn_prefill_kernel<HD, GQA, KV8, 4, CT, 1><<<dim3(kv_heads, (a.T + RB - 1) / RB), 256, 0, st>>>(a);
+  else if (narrow > cus || a.pos0 + a.T <= 64)
+    attn_prefill_kernel<HD, GQA, KV8, 4, 1, 1><<<dim3(kv_heads, (a.T + R1 - 1) / R1), 256, 0, st>>>(a);
+  else if (HD == 128 && a.T * GQA <= 32)
+    attn_prefill_kernel<HD, GQA, KV8, 2, 1, (HD == 128 ? 4 : 2)><<<dim3(kv_heads, 1), (HD == 128 ? 512 : 256), 0, st>>>(a);
+  else
+    attn_prefill_kernel<HD, GQA, KV8, 4, 1, 2><<<dim3(kv_heads, (a.T + R1 - 1) / R1), 512, 0, st>>>(a);
 }
 
 template <int HD, int KV8>
-int launch_prefill_attn(const PrefillAttnArgs& a, uint32_t gqa, uint32_t kv_heads, hipStream_t st) {
+int launch_prefill_attn(const PrefillAttnArgs& a, uint32_t gqa, uint32_t kv_heads, uint32_t cus, hipStream_t st) {
   switch (gqa) {
-    case 1: launch_prefill_gqa<HD, 1, KV8>(a, kv_heads, st); return 0;
-    case 2: launch_prefill_gqa<HD, 2, KV8>(a, kv_heads, st); return 0;
-    case 4: launch_prefill_gqa<HD, 4, KV8>(a, kv_heads, st); return 0;
-    case 5: launch_prefill_gqa<HD, 5, KV8>(a, kv_heads, st); return 0;
-    case 6: launch_prefill_gqa<HD, 6, KV8>(a, kv_heads, st); return 0;
-    case 8: launch_prefill_gqa<HD, 8, KV8>(a, kv_heads, st); return 0;
+    case 1: launch_prefill_gqa<HD, 1, KV8>(a, kv_heads, cus, st); return 0;
+    case 2: launch_prefill_gqa<HD, 2, KV8>(a, kv_heads, cus, st); return 0;
+    case 4: launch_prefill_gqa<HD, 4, KV8>(a, kv_heads, cus, st); return 0;
+    case 5: launch_prefill_gqa<HD, 5, KV8>(a, kv_heads, cus, st); return 0;
+    case 6: launch_prefill_gqa<HD, 6, KV8>(a, kv_heads, cus, st); return 0;
+    case 8: launch_prefill_gqa<HD, 8, KV8>(a, kv_heads, cus, st); return 0;
     default: return -1;
   }
 }
@@ -819,6 +988,15 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t* __restr
 
 using namespace mi;
 
+// the CUs of the current device, which the launch rules fill
+static int cu_count(uint32_t* cus, const char* name) {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return mi_hip((int)hipGetLastError(), name);
+  *cus = n > 0 ? (uint32_t)n : 1u;
+  return 0;
+}
+
 // The work-group tile of the GEMM. Every tile sums a column over the k-groups in the same MFMA
 // order, so the choice changes the speed only, never a bit of the result. For N a multiple of
 // 256 the tile is a row of 4 waves of R x 64 (R = 128, 96 or 64): the larger R, the less
@@ -840,12 +1018,11 @@ static int launch_gemm(const char* name, const uint32_t* qweight, const uint16_t
   // the packed weights stay below 2 GiB
   if (((uint64_t)T + 128u) * K * 2u >= (1ull << 31) || (uint64_t)K * N / 2u >= (1ull << 31))
     return mi_fail(MI_ERR_SHAPE, (std::string(name) + ": x or qweight beyond 2 GiB").c_str());
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return mi_hip((int)hipGetLastError(), name);
+  uint32_t cus = 0;
+  if (int e = cu_count(&cus, name)) return e;
   hipStream_t st = (hipStream_t)stream;
   if (N % 256u == 0) {
-    const uint64_t C = (uint64_t)(cus > 0 ? cus : 1);
+    const uint64_t C = cus;
     auto cost = [&](uint32_t R, uint64_t rate) {  // rows on the busiest CU x 100 / rate (percent)
       const uint64_t wg = (uint64_t)(N / 256u) * ((T + R - 1u) / R);
       return (wg + C - 1u) / C * R * 10000u / rate;
@@ -931,8 +1108,10 @@ int mi_attn_prefill(const float* attn_q, const uint16_t* kv_k, const uint16_t* k
   PrefillAttnArgs a{attn_q, kv_k, kv_v, pages, attn_out, row_stride, head_stride, page, T, pos0,
                     shape->q_heads, shape->scale, nullptr, nullptr, 0, 0, nullptr};
   hipStream_t st = (hipStream_t)stream;
-  const int r = HD == 128 ? launch_prefill_attn<128, 0>(a, gqa, shape->kv_heads, st)
-                          : launch_prefill_attn<256, 0>(a, gqa, shape->kv_heads, st);
+  uint32_t cus = 0;
+  if (int e = cu_count(&cus, "attn_prefill")) return e;
+  const int r = HD == 128 ? launch_prefill_attn<128, 0>(a, gqa, shape->kv_heads, cus, st)
+                          : launch_prefill_attn<256, 0>(a, gqa, shape->kv_heads, cus, st);
   if (r) return mi_fail(MI_ERR_SHAPE, "attn_prefill: unsupported GQA");
   return mi_hip((int)hipGetLastError(), "attn_prefill");
 }
@@ -955,12 +1134,11 @@ int mi_attn_prefill_kv8(const float* attn_q, const int8_t* kv_k, const int8_t* k
   PrefillAttnArgs a{attn_q, kv_k, kv_v, pages, attn_out, row_stride, head_stride, page, T, pos0,
                     shape->q_heads, shape->scale, k_scale, v_scale, sc_row_stride, sc_head_stride, out_rot};
   hipStream_t st = (hipStream_t)stream;
-  if (launch_prefill_attn<256, 1>(a, gqa, shape->kv_heads, st))
+  uint32_t cus = 0;
+  if (int e = cu_count(&cus, "attn_prefill_kv8")) return e;
+  if (launch_prefill_attn<256, 1>(a, gqa, shape->kv_heads, cus, st))
     return mi_fail(MI_ERR_SHAPE, "attn_prefill_kv8: unsupported GQA");
-  int e = (int)hipGetLastError();
-  if (e) return mi_hip(e, "attn_prefill_kv8");
-  unrotate_rows_kernel<<<dim3(shape->q_heads, T), 256, 0, st>>>(out_rot, attn_out, shape->q_heads);
-  return mi_hip((int)hipGetLastError(), "attn_prefill_kv8 unrotate");
+  return mi_hip((int)hipGetLastError(), "attn_prefill_kv8");
 }
 
 int mi_attn_prep_rows(const float* qkv, uint32_t T, uint32_t pos0, const mi_attn_shape* shape, const float* q_norm,

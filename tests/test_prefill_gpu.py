@@ -168,6 +168,85 @@ def test_attn_prefill_vs_fp64(QH, KVH, HD, T, pos0):
     assert cos.min() >= 0.99999
 
 
+def unrotate64():
+    """y -> H_256 diag(s) y / 16 as an fp64 matrix (the int8 cache's rotation, kv8.h:1-26)."""
+    words = (0xA197D809, 0xA6850592, 0xB205A73E, 0x20AFA769, 0x45C2CF64, 0xBEAEAACB, 0x75F39ADD, 0x2385A70C)
+    sign = np.array([-1.0 if words[j // 32] >> (j % 32) & 1 else 1.0 for j in range(256)])
+    h = np.ones((1, 1))
+    for _ in range(8):
+        h = np.block([[h, h], [h, -h]])
+    return h * sign[None, :] / 16
+
+
+# each work-group shape of the launch rule on a 256-CU part: 32 columns or fewer with the keys in four
+# parts (1..6 rows at GQA 5) around its 128-key iteration, 64 keys in one part against 65 in two, 64
+# columns with the keys in two parts, 64 and 128 columns in one; key counts around the iterations' edges
+@pytest.mark.parametrize("QH,KVH,HD,T,pos0,int8", [
+    (40, 8, 128, 6, 122, 0), (40, 8, 128, 6, 123, 0), (40, 8, 128, 1, 64, 0), (40, 8, 128, 64, 0, 0),
+    (40, 8, 128, 65, 0, 0), (40, 8, 128, 7, 185, 0), (40, 8, 128, 400, 33, 0), (40, 8, 128, 810, 0, 0),
+    (12, 2, 128, 3, 500, 0), (16, 2, 256, 5, 59, 0), (16, 2, 256, 33, 95, 0), (16, 2, 256, 1030, 0, 0),
+    (16, 2, 256, 1, 0, 1), (16, 2, 256, 9, 119, 1), (16, 2, 256, 1030, 31, 1), (24, 4, 256, 37, 290, 1)])
+def test_attn_prefill_work_group_shapes_vs_fp64(QH, KVH, HD, T, pos0, int8):
+    """Scores that grow along the keys (the running maximum keeps rising, so the accumulators are
+    rescaled again and again) and span about 2^30, against fp64 causal attention; the last cache row
+    holds what no row may read."""
+    sh = O.attn_shape(QH, KVH, HD)
+    Lm = pos0 + T + 1
+    rng = np.random.default_rng(QH + T + pos0)
+    q = 2 * rng.standard_normal((T, QH, HD)).astype(np.float32)
+    ramp = np.linspace(0.3, 1.5, Lm)[None, :, None]
+    k = ramp * rng.standard_normal((KVH, Lm, HD))
+    if int8:
+        s16 = O.f32_to_f16_bits((np.abs(k).max(-1) / 127).astype(np.float32))
+        k8 = np.clip(np.rint(k / O.f16_bits_to_f32(s16)[..., None]), -127, 127).astype(np.int8)
+        v8 = rng.integers(-127, 128, size=(KVH, Lm, HD)).astype(np.int8)
+        vs = O.f32_to_f16_bits(rng.uniform(0.005, 0.05, (KVH, Lm)).astype(np.float32))
+        s16[:, -1] = vs[:, -1] = 0x7E00  # NaN scales in the row past the last
+        kf = k8 * O.f16_bits_to_f32(s16).astype(np.float64)[..., None]
+        vf = v8 * O.f16_bits_to_f32(vs).astype(np.float64)[..., None]
+    else:
+        k16, v16 = O.f32_to_f16_bits(k.astype(np.float32)), O.f32_to_f16_bits(rng.standard_normal(k.shape).astype(np.float32))
+        k16[:, -1] = v16[:, -1] = 0x7E00
+        kf, vf = O.f16_bits_to_f32(k16).astype(np.float64), O.f16_bits_to_f32(v16).astype(np.float64)
+    print(f"attn_prefill {QH}/{KVH}x{HD} T={T} pos0={pos0} int8={int8}", flush=True)
+    if int8:
+        keep = [dev(a) for a in (q, k8, v8, s16, vs)]
+        rot, out = empty((T, QH, HD), np.float32), empty((T, QH * HD), np.uint16)
+        mi.call("mi_attn_prefill_kv8", *[ptr(a) for a in keep], HD, Lm * HD, 1, Lm, None, 0, T, pos0, mi.shape_ref(sh),
+                ptr(rot), ptr(out), stream())
+        sync()
+        got = host(out, np.uint16)
+    else:
+        got = prefill_attention(sh, q, k16, v16, T, pos0)
+    g = O.f16_bits_to_f32(got).astype(np.float64).reshape(T, QH, HD)
+    keys = pos0 + T
+    hidden = np.arange(keys)[None, :] > pos0 + np.arange(T)[:, None]
+    for h in range(QH):
+        s = q[:, h].astype(np.float64) @ kf[h // (QH // KVH), :keys].T * float(sh.scale)
+        s[hidden] = -np.inf
+        w = np.exp(s - s.max(-1, keepdims=True))
+        w /= w.sum(-1, keepdims=True)
+        kh, vh = kf[h // (QH // KVH), :keys], vf[h // (QH // KVH), :keys]
+        want = w @ vh
+        # a score's error: 2^-21 sum |q k| scale (q in two f16 parts is good to 2^-22, the fp32 sums of
+        # its products to about as much); a weight's is that of its own and of the largest score; the
+        # weights' parts and the sums over the keys add 2^-20. The parts are f16 values down to 2^-24, so
+        # a weight (int8: times its V scale) is also off by up to 2^-25 of the largest one, whatever its
+        # size: independent over the keys, 8 standard deviations of 2^-25 / sqrt(3) each
+        ds = 2.0 ** -21 * np.where(hidden, 0, np.abs(q[:, h]).astype(np.float64) @ np.abs(kh).T * float(sh.scale))
+        bound = (2 * ds.max(-1, keepdims=True) + 2.0 ** -20) * (w @ np.abs(vh))
+        vraw = v8[h // (QH // KVH), :keys].astype(np.float64) if int8 else vh
+        bound += 8 * 2.0 ** -25 / 3 ** 0.5 * np.sqrt(~hidden @ np.square(vraw))
+        if int8:
+            rot_err = np.abs(host(rot, np.float32).reshape(T, QH, HD)[:, h] - want)
+            assert np.all(rot_err <= bound), (h, (rot_err / bound).max())
+            R = unrotate64()
+            want, bound = want @ R.T, bound @ np.abs(R).T
+        err = np.abs(g[:, h] - want)
+        bound = bound + 2.0 ** -11 * np.abs(want) + 2.0 ** -25  # the f16 rounding of the output
+        assert np.all(err <= bound), (h, (err / bound).max())
+
+
 def test_attn_prefill_paged_bitwise():
     sh = O.attn_shape(40, 8, 128)
     Lm, P, T, pos0 = 512, 64, 50, 300
