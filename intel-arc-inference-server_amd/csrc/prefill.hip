@@ -8,24 +8,31 @@
 // gate||up + SiLU, down + residual + norm; the last position's head and argmax leave the control
 // block as decode's ingest of the same ids would (cur_token = the argmax, pos advanced by T).
 //
-// gemm_w4a16_kernel: out[T][N] fp32 = x[T][K] (f16) . W[K][N] (int4 GPTQ g64, layout 0). The
-// contraction is a dense GEMM here (2 T K N flops over K N / 2 weight bytes): MFMA-bound from a
-// few dozen rows, so it is tiled for the matrix cores rather than streamed like the decode GEMV.
-//   * 4 waves per work-group, each 16 RI rows x 64 columns = RI x 4 v_mfma_f32_16x16x32_f16
-//     tiles; WM waves along the rows: tiles of 128 x 256 (RI 8, one row of waves: the B words
-//     are loaded and dequantised once per work-group and serve 128 rows), 96 x 256, 64 x 256 and
-//     128 x 128 (see launch_gemm for the choice);
+// gemm_w4a16_kernel, gemm_w4a16_few_kernel: out[T][N] fp32 = x[T][K] (f16) . W[K][N] (int4 GPTQ g64,
+// layout 0). The contraction is a dense GEMM here (2 T K N flops over K N / 2 weight bytes):
+// MFMA-bound from some hundred rows, bound by the weights' stream and its latency below.
+//   * each wave has 16 RI rows x 64 columns = RI x 4 v_mfma_f32_16x16x32_f16 tiles; 4 waves side by
+//     side make tiles of 16 RI x 256 (RI 8: 128 rows per weight unpacked). Where a launch would
+//     leave CUs with one such work-group or none, RI is smaller and 8 waves split the k-groups in
+//     two parts, or (few rows) 8 waves split the k-groups of a 64-column tile (pick_gemm);
 //   * one 64-deep k-group per iteration (one scale per column). The activations go through LDS,
 //     double-buffered (the next group's rows are loaded into registers while the current group
 //     is multiplied, then written to the other buffer). The weights skip LDS: a B fragment of
 //     v_mfma_f32_16x16x32_f16 is 8 consecutive k of one column, which is exactly one int4 word,
-//     so each lane loads its own words a group ahead and dequantises them into the fragment
-//     (LDS then carries the activations only, which halves its traffic per MFMA);
+//     so each lane loads its own words two groups ahead (16 bytes: one word of each of its four
+//     column tiles) and unpacks them into the fragments, half a group at a time between the
+//     products of the half before. Every load is unconditional and stays where it is written, so
+//     the waits count exactly the loads that may still be in flight;
 //   * w = f16((q - 8) * scale): q - 8 exact in f16 (the magic-number unpack of the decode GEMV),
 //     one f16 rounding of the product (the reference's prefill rounds the same product to bf16,
 //     pf_dequant_slab.cl); the activations are permuted to the unpack's pair order
 //     (k0,k4)(k1,k5)(k2,k6)(k3,k7) inside each 8-k chunk, so the products pair up;
-//   * fp32 accumulation across the whole K in MFMA order.
+//   * fp32 accumulation in MFMA order, the k parts' sums added in ascending k. A column's order
+//     therefore depends on the shape that the rule takes, that is on T, K and N.
+// Measured at 2048 rows (MI355X, us before / now): gate||up + SwiGLU 5120 -> 34816 714 / 678 (1.08 PFLOP/s;
+// the library's plain f16 product of these sizes 1.17), q||k||v 5120 -> 7168 167 / 147, down 17408 -> 5120
+// 406 / 359; a product of the matrix cores takes twice its issue time even so, since the clock falls under
+// it (1.93 GHz at 1.0 PFLOP/s by the counters).
 //
 // attn_prefill_kernel: causal GQA attention of T query rows at positions pos0 .. pos0+T-1 over
 // the cache rows [0, pos0 + t] (the chunk's own rows written by attn_prep before it), f16 or the
@@ -68,43 +75,110 @@ __device__ __forceinline__ u4_t perm_pairs(u4_t v) {
               __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
 }
 
+// The unpack's masks and magic, in registers and opaque: (w & mask) | magic then is one v_and_or_b32
+// (known literals would become two instructions), and unlike inline assembly the scheduler can
+// place it between matrix products.
+struct DqConst {
+  uint32_t lo = 0x000F000Fu, hi = 0x00F000F0u, magic = 0x64006400u;
+  __device__ __forceinline__ DqConst() { asm("" : "+s"(lo), "+s"(hi), "+v"(magic)); }
+};
+
 // f16((q_i - 8) * s) of one word's 8 nibbles, pair order (q0,q4)(q1,q5)(q2,q6)(q3,q7)
-__device__ __forceinline__ u4_t dequant_scaled(uint32_t w, h2_t s2) {
-  const uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, magic = 0x64006400u;
+__device__ __forceinline__ u4_t dequant_scaled(uint32_t w, h2_t s2, const DqConst& c) {
   const h2_t b1032 = {(half_t)1032.0f, (half_t)1032.0f};
   const h2_t s16 = {(half_t)0.0625f, (half_t)0.0625f};
   const h2_t b72 = {(half_t)-72.0f, (half_t)-72.0f};
   const uint32_t t = w >> 8;
-  const h2_t p0 = as_h2(and_or(w, m_lo, magic)) - b1032;                               // q - 8, exact
-  const h2_t p1 = __builtin_elementwise_fma(as_h2(and_or(w, m_hi, magic)), s16, b72);  // exact
-  const h2_t p2 = as_h2(and_or(t, m_lo, magic)) - b1032;
-  const h2_t p3 = __builtin_elementwise_fma(as_h2(and_or(t, m_hi, magic)), s16, b72);
+  const h2_t p0 = as_h2((w & c.lo) | c.magic) - b1032;                               // q - 8, exact
+  const h2_t p1 = __builtin_elementwise_fma(as_h2((w & c.hi) | c.magic), s16, b72);  // exact
+  const h2_t p2 = as_h2((t & c.lo) | c.magic) - b1032;
+  const h2_t p3 = __builtin_elementwise_fma(as_h2((t & c.hi) | c.magic), s16, b72);
   return u4_t{h2_bits(p0 * s2), h2_bits(p1 * s2), h2_bits(p2 * s2), h2_bits(p3 * s2)};
 }
 
-// SILU: the columns are gate||up in the interleave16 order (gate block, up block, ...); a wave's
-// 64 columns hold two such pairs, so each lane has the gate and up value of the same output in
-// its tiles j and j + 1, and writes h [T][N/2] f16 = rne(rne(silu(rne(g))) * rne(u)) (the
-// arithmetic of prep_silu_mul, prep.cl:384) instead of the fp32 output.
-template <bool SILU, uint32_t WM, uint32_t RI, uint32_t LB>
-__global__ __launch_bounds__(256, LB) void gemm_w4a16_kernel(const uint32_t* __restrict__ qweight,
-                                                         const uint16_t* __restrict__ scales,
-                                                         const uint16_t* __restrict__ x,
-                                                         float* __restrict__ out, uint16_t* __restrict__ h_out,
-                                                         uint32_t T, uint32_t K, uint32_t N) {
-  // WM waves along the rows, 4 / WM along the columns, each wave 16 RI rows x 64 columns
-  constexpr uint32_t BM = 16u * RI * WM, BN = 256u / WM, WN = 4u / WM, AI = BM / 32u;
-  __shared__ __align__(16) uint16_t As[2][BM][GROW];
-  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  const uint32_t wm = wave / WN, wn = wave % WN;
-  const uint32_t n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
-  const uint32_t G = K / GBK;
-  const uint32_t fr = lane & 15u, fq = lane >> 4;  // fragment row/column, k chunk (8 k)
+// outputs are stored in pieces of several elements at the elements' own alignment
+typedef f4_t f4_any __attribute__((aligned(4)));
+typedef u2_t h4_any __attribute__((aligned(2)));
 
-  // activations, staged through LDS: thread t takes rows (t >> 3) + 32 i (i < BM / 32), 8-k chunk t & 7
-  const uint32_t a_row = t >> 3, a_chunk = t & 7u;
-  // buffer loads: 32-bit offsets keep the addresses out of 64-bit registers; the row sits in the
+// A wave's 64 columns: lane (fr, fq) = (l % 16, l / 16) reads word row fq of a half group's four at
+// columns 4 fr .. 4 fr + 3 (one 16-byte load), and column 4 fr + j is column fr of the wave's matrix
+// tile j: the B operand is the lane's own word, and the lane ends with four adjacent columns.
+struct BGroup {
+  u4_t w[2];  // k half ks: the word rows 4 ks + fq
+  u2_t s;     // the four columns' scales
+};
+// the operands of k half ks: four tiles' fragments
+__device__ __forceinline__ void dequant_half(const BGroup& b, uint32_t ks, const DqConst& c, h8_t (&bf)[4]) {
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j) {
+    const uint32_t sj = j < 2 ? b.s.x : b.s.y;
+    const h2_t s2 = as_h2(__builtin_amdgcn_perm(sj, sj, j & 1u ? 0x03020302u : 0x01000100u));
+    bf[j] = __builtin_bit_cast(h8_t, dequant_scaled(b.w[ks][j], s2, c));
+  }
+}
+// Fixes the place where operands are formed: ahead of the loads that refill the registers they come
+// from. (Sunk past those loads, to the products, they would make the loads take other registers,
+// and the copies back at the loop's end would wait for the loads.)
+template <uint32_t N>
+__device__ __forceinline__ void pin(h8_t (&f)[N]) {
+#pragma unroll
+  for (uint32_t j = 0; j < N; ++j) asm volatile("" : "+v"(f[j]));
+  __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ uint16_t swiglu16(float g, float u) {
+  const uint16_t g_b = f2h(g), u_b = f2h(u);
+  return f2h(h2f(f2h(silu_f32(h2f(g_b)))) * h2f(u_b));
+}
+
+// The lane's four adjacent columns ncol .. + 3 of one row. SILU: the columns are gate||up in the
+// interleave16 order, so the up values of a gate lane (fr & 4 == 0) are four lanes on; it writes h
+// [T][N/2] f16 = rne(rne(silu(rne(g))) * rne(u)) (the arithmetic of prep_silu_mul, prep.cl:384)
+// instead of the fp32 output. Every lane of the row's 16 calls it; `store`: the row and column exist.
+template <bool SILU>
+__device__ __forceinline__ void store_row4(f4_t v, bool store, float* out, uint16_t* h_out, uint32_t row, uint32_t ncol,
+                                           uint32_t N) {
+  if constexpr (SILU) {
+    uint16_t h[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) h[j] = swiglu16(v[j], dpp_f<0x104>(v[j]));  // row_shl:4
+    if (store && !(ncol & 16u)) {
+      const uint32_t n = ncol / 32u * 16u + ncol % 16u;
+      *reinterpret_cast<h4_any*>(h_out + (size_t)row * (N / 2) + n) =
+          u2_t{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+    }
+  } else {
+    if (store) *reinterpret_cast<f4_any*>(out + (size_t)row * N + ncol) = v;
+  }
+}
+
+// Tile: 16 RI rows x 256 columns, 4 waves of 16 RI x 64 per K part. KS = 2: 8 waves, waves 4 .. 7 the
+// second half of the k-groups, the halves added at the end through LDS. DA / DB: k-groups of
+// activations / weights in flight in registers ahead of the one multiplied.
+template <bool SILU, uint32_t RI, uint32_t KS, uint32_t DA>
+__global__ __launch_bounds__(256 * KS, 2) void gemm_w4a16_kernel(const uint32_t* __restrict__ qweight,
+                                                                 const uint16_t* __restrict__ scales,
+                                                                 const uint16_t* __restrict__ x,
+                                                                 float* __restrict__ out, uint16_t* __restrict__ h_out,
+                                                                 uint32_t T, uint32_t K, uint32_t N) {
+  constexpr uint32_t BM = 16u * RI, AI = (BM + 31u) / 32u;
+  __shared__ __align__(16) union {
+    uint16_t As[KS][2][BM][GROW];
+    f4_t part[KS > 1 ? 4 : 1][RI][4][64];
+  } sm;
+  // (readfirstlane: the compiler then knows that a wave's part and column block are uniform)
+  const uint32_t t = threadIdx.x % 256u, lane = t & 63u, wn = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t kp = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 256u) : 0u;
+  const uint32_t n0 = blockIdx.x * 256u, m0 = blockIdx.y * BM;
+  const uint32_t fr = lane & 15u, fq = lane >> 4;
+  const uint32_t G = K / GBK, n_it = (G + KS - 1u) / KS;  // this part's groups: g0 .. g1 - 1
+  const uint32_t g0 = kp * n_it, g1 = min(G, g0 + n_it);
+  const uint32_t ncol = n0 + 64u * wn + 4u * fr;
+  const bool col_in = n0 + 64u * wn < N;  // uniform per wave: the last tile may hold 128 columns
+
+  // activations, staged through LDS: thread t takes rows (t >> 3) + 32 i, 8-k chunk t & 7. Buffer
+  // loads: 32-bit offsets keep the addresses out of 64-bit registers; the row sits in the
   // per-thread offset, so a row at or past T lies outside the resource's T K elements and reads 0
+  const uint32_t a_row = t >> 3, a_chunk = t & 7u;
   const __amdgpu_buffer_rsrc_t x_rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, T * K * 2u, 0x00020000);
   const __amdgpu_buffer_rsrc_t w_rs =
@@ -112,33 +186,34 @@ __global__ __launch_bounds__(256, LB) void gemm_w4a16_kernel(const uint32_t* __r
   const __amdgpu_buffer_rsrc_t s_rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(scales), 0, (K / GBK) * N * 2u, 0x00020000);
   const uint32_t a_voff = ((m0 + a_row) * K + 8u * a_chunk) * 2u;
-  u4_t a_st[AI];
-  auto load_a = [&](uint32_t g) {
+  const uint32_t wcol = col_in ? ncol : 4u * fr;  // (a wave past N reads its own tile's words of column 0 ..)
+  const uint32_t w_voff = (fq * N + wcol) * 4u, s_voff = wcol * 2u;
+  u4_t a_st[DA][AI];
+  BGroup b_st[2];
+  // (a group at or past the part's end takes offsets outside the resource: zeros, so the loop needs
+  // no branch around its loads or products)
+  auto past = [&](uint32_t g) { return g < g1 ? 0u : 0x80000000u; };
+  auto load_a = [&](uint32_t g, u4_t (&st)[AI]) {
+    const uint32_t o = past(g);
+    g = min(g, G - 1u);
 #pragma unroll
     for (uint32_t i = 0; i < AI; ++i)
-      a_st[i] = __builtin_bit_cast(
-          u4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rs, a_voff + 32u * i * K * 2u, g * GBK * 2u, 0));
+      st[i] = __builtin_bit_cast(
+          u4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rs, (a_voff + 32u * i * K * 2u) | o, g * GBK * 2u, 0));
   };
-  auto store_a = [&](uint32_t buf) {
-#pragma unroll
-    for (uint32_t i = 0; i < AI; ++i)
-      *reinterpret_cast<u4_t*>(&As[buf][a_row + 32u * i][8u * a_chunk]) = perm_pairs(a_st[i]);
-  };
-  // weights, straight into registers: the B fragment of n-tile j and k half ks is one word per
-  // lane (8 k of column 16 j + fr, word row 4 ks + fq of the group), dequantised just before use
-  const uint32_t ncol = n0 + 64u * wn + fr;
-  const uint32_t w_voff = (fq * N + ncol) * 4u, s_voff = ncol * 2u;
-  uint32_t b_w[2][4];
-  uint16_t b_s[4];
-  auto load_b = [&](uint32_t g) {
+  auto load_b = [&](uint32_t g, BGroup& b) {
+    const uint32_t o = past(g);
+    g = min(g, G - 1u);
 #pragma unroll
     for (uint32_t ks = 0; ks < 2; ++ks)
+      b.w[ks] = __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rs, w_voff | o, (8u * g + 4u * ks) * N * 4u, 2));
+    b.s = __builtin_bit_cast(u2_t, __builtin_amdgcn_raw_buffer_load_b64(s_rs, s_voff | o, g * N * 2u, 0));
+  };
+  auto store_a = [&](uint32_t buf, const u4_t (&st)[AI]) {
 #pragma unroll
-      for (uint32_t j = 0; j < 4; ++j)
-        b_w[ks][j] = __builtin_amdgcn_raw_buffer_load_b32(w_rs, w_voff, ((8u * g + 4u * ks) * N + 16u * j) * 4u, 2);
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j)
-      b_s[j] = __builtin_amdgcn_raw_buffer_load_b16(s_rs, s_voff, (g * N + 16u * j) * 2u, 0);
+    for (uint32_t i = 0; i < AI; ++i)
+      if (32u * (i + 1u) <= BM || a_row + 32u * i < BM)
+        *reinterpret_cast<u4_t*>(&sm.As[kp][buf][a_row + 32u * i][8u * a_chunk]) = perm_pairs(st[i]);
   };
 
   f4_t acc[RI][4];
@@ -147,59 +222,160 @@ __global__ __launch_bounds__(256, LB) void gemm_w4a16_kernel(const uint32_t* __r
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
 
-  load_a(0);
-  load_b(0);
-  store_a(0);
+  // Each half group's products run with the next half's weights becoming fragments between them (two
+  // vector instructions hide behind each product; as phases of their own the products and the
+  // unpack would add up). A group's weight registers are refilled, two groups on, once its second
+  // half is unpacked.
+  const DqConst dq;
+  h8_t bf[2][4];
+  load_b(g0, b_st[0]);
+#pragma unroll
+  for (uint32_t u = 0; u < DA; ++u) load_a(g0 + u, a_st[u]);
+  __builtin_amdgcn_sched_barrier(0);
+  load_b(g0 + 1u, b_st[1]);
+  store_a(0, a_st[0]);
+  dequant_half(b_st[0], 0, dq, bf[0]);
+  pin(bf[0]);
   lds_barrier();
-  for (uint32_t g = 0; g < G; ++g) {
-    const uint32_t buf = g & 1u;
-    // this group's weights become fragments; the next group's loads go out
-    h8_t bf[2][4];
+  for (uint32_t it0 = 0; it0 < n_it; it0 += 2u) {
 #pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-      const h2_t s2 = as_h2((uint32_t)b_s[j] | ((uint32_t)b_s[j] << 16));
+    for (uint32_t u = 0; u < 2u; ++u) {
+      const uint32_t g = g0 + it0 + u;
+      load_a(g + DA, a_st[u % DA]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (uint32_t ks = 0; ks < 2; ++ks) bf[ks][j] = __builtin_bit_cast(h8_t, dequant_scaled(b_w[ks][j], s2));
+      for (uint32_t ks = 0; ks < 2; ++ks) {
+        h8_t af[RI];
+#pragma unroll
+        for (uint32_t i = 0; i < RI; ++i)
+          af[i] = *reinterpret_cast<const h8_t*>(&sm.As[kp][u][16u * i + fr][32u * ks + 8u * fq]);
+#pragma unroll
+        for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+          for (uint32_t j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[ks][j], acc[i][j], 0, 0, 0);
+        dequant_half(b_st[ks ? u ^ 1u : u], ks ^ 1u, dq, bf[ks ^ 1u]);
+        pin(bf[ks ^ 1u]);
+        if (ks == 0) load_b(g + 2u, b_st[u]);
+      }
+      store_a(u ^ 1u, a_st[(u + 1u) % DA]);  // the other buffer was last read before the previous barrier
+      lds_barrier();
     }
-    if (g + 1 < G) {
-      load_a(g + 1);
-      load_b(g + 1);
-    }
-#pragma unroll
-    for (uint32_t ks = 0; ks < 2; ++ks) {
-      h8_t af[RI];
-#pragma unroll
-      for (uint32_t i = 0; i < RI; ++i)
-        af[i] = *reinterpret_cast<const h8_t*>(&As[buf][16u * RI * wm + 16u * i + fr][32u * ks + 8u * fq]);
-#pragma unroll
-      for (uint32_t i = 0; i < RI; ++i)
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[ks][j], acc[i][j], 0, 0, 0);
-    }
-    if (g + 1 < G) store_a(buf ^ 1u);  // the other buffer was last read before the previous barrier
-    lds_barrier();
   }
-  // lane holds rows 4 (lane >> 4) + r of column lane & 15 of each 16 x 16 tile
+  if constexpr (KS > 1) {  // the second half's sums through LDS (the staged activations are done with)
+    if (kp) {
+#pragma unroll
+      for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) sm.part[wn][i][j][lane] = acc[i][j];
+    }
+    lds_barrier();
+    if (kp) return;
+#pragma unroll
+    for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) acc[i][j] += sm.part[wn][i][j][lane];
+  }
+  // lane holds rows 4 fq + r of columns ncol .. + 3 of each 16-row tile
 #pragma unroll
   for (uint32_t i = 0; i < RI; ++i)
 #pragma unroll
     for (uint32_t r = 0; r < 4; ++r) {
-      const uint32_t row = m0 + 16u * RI * wm + 16u * i + 4u * fq + r;
-      if (row < T) {
-        if constexpr (SILU) {
+      const uint32_t row = m0 + 16u * i + 4u * fq + r;
+      store_row4<SILU>(f4_t{acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]}, row < T && col_in, out, h_out, row,
+                       ncol, N);
+    }
+}
+
+// Few rows: 16 RI rows x 64 columns per work-group, its KW waves taking a KW-th of the k-groups
+// each. Nothing is shared, so there is no LDS staging and no barrier in the loop: a wave loads its
+// weights and its activations (in the A operand's own layout, from L2) D groups ahead. The waves'
+// sums are added through LDS in ascending k.
+template <bool SILU, uint32_t RI, uint32_t KW, uint32_t D>
+__global__ __launch_bounds__(64 * KW, KW > 8 ? 4 : 2) void gemm_w4a16_few_kernel(
+    const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ x,
+    float* __restrict__ out, uint16_t* __restrict__ h_out, uint32_t T, uint32_t K, uint32_t N) {
+  constexpr uint32_t BM = 16u * RI;
+  __shared__ f4_t red[KW][BM][16];
+  const uint32_t lane = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15u,
+                 fq = lane >> 4;
+  const uint32_t n0 = blockIdx.x * 64u, m0 = blockIdx.y * BM, ncol = n0 + 4u * fr;
+  const uint32_t G = K / GBK, g0 = w * G / KW, g1 = (w + 1u) * G / KW;
+  const __amdgpu_buffer_rsrc_t x_rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, T * K * 2u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t w_rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(qweight), 0, (K / 8u) * N * 4u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t s_rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(scales), 0, (K / GBK) * N * 2u, 0x00020000);
+  const uint32_t a_voff = ((m0 + fr) * K + 8u * fq) * 2u, w_voff = (fq * N + ncol) * 4u, s_voff = ncol * 2u;
+  const DqConst dq;
+  u4_t a_st[D][2][RI];
+  BGroup b_st[D];
+  auto load = [&](uint32_t g, uint32_t u) {
+    g = min(g, G - 1u);
 #pragma unroll
-          for (uint32_t jp = 0; jp < 2; ++jp) {
-            const uint16_t g_b = f2h(acc[i][2 * jp][r]), u_b = f2h(acc[i][2 * jp + 1][r]);
-            const uint16_t s_b = f2h(silu_f32(h2f(g_b)));
-            h_out[(size_t)row * (N / 2) + (n0 + 64u * wn) / 2 + 16u * jp + fr] = f2h(h2f(s_b) * h2f(u_b));
-          }
-        } else {
+    for (uint32_t ks = 0; ks < 2; ++ks)
+      b_st[u].w[ks] =
+          __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rs, w_voff, (8u * g + 4u * ks) * N * 4u, 2));
+    b_st[u].s = __builtin_bit_cast(u2_t, __builtin_amdgcn_raw_buffer_load_b64(s_rs, s_voff, g * N * 2u, 0));
 #pragma unroll
-          for (uint32_t j = 0; j < 4; ++j) out[(size_t)row * N + ncol + 16u * j] = acc[i][j][r];
-        }
+    for (uint32_t ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (uint32_t i = 0; i < RI; ++i)
+        a_st[u][ks][i] = __builtin_bit_cast(
+            u4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rs, a_voff + 32u * i * K, (g * GBK + 32u * ks) * 2u, 0));
+  };
+  f4_t acc[RI][4];
+#pragma unroll
+  for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (uint32_t u = 0; u < D; ++u) {
+    load(g0 + u, u);
+    __builtin_amdgcn_sched_barrier(0);  // in the loop's order (as in gemm_w4a16_kernel)
+  }
+  for (uint32_t g = g0; g < g1; g += D) {
+#pragma unroll
+    for (uint32_t u = 0; u < D; ++u) {
+      h8_t bf[2][4], af[2][RI];
+#pragma unroll
+      for (uint32_t ks = 0; ks < 2; ++ks) dequant_half(b_st[u], ks, dq, bf[ks]);
+#pragma unroll
+      for (uint32_t ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (uint32_t i = 0; i < RI; ++i) af[ks][i] = __builtin_bit_cast(h8_t, perm_pairs(a_st[u][ks][i]));
+#pragma unroll
+      for (uint32_t ks = 0; ks < 2; ++ks) {
+        pin(bf[ks]);
+        pin(af[ks]);
+      }
+      load(g + u + D, u);
+      if (g + u < g1) {  // uniform
+#pragma unroll
+        for (uint32_t ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[ks][i], bf[ks][j], acc[i][j], 0, 0, 0);
       }
     }
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r)
+      red[w][16u * i + 4u * fq + r][fr] = f4_t{acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
+  __syncthreads();
+  // (the lanes of a wave take 16 adjacent pieces of four rows at a time: BM * 16 pieces in all)
+  for (uint32_t e = threadIdx.x; e < BM * 16u; e += 64u * KW) {
+    const uint32_t row = e / 16u, c = e % 16u;
+    f4_t v = red[0][row][c];
+#pragma unroll
+    for (uint32_t q = 1; q < KW; ++q) v += red[q][row][c];
+    store_row4<SILU>(v, m0 + row < T, out, h_out, m0 + row, n0 + 4u * c, N);
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -348,6 +524,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const u4_t* __restrict__ 
   const __amdgpu_buffer_rsrc_t w_rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(wb), 0, (uint32_t)(block_u32 * 4u), 0x00020000);
   const uint32_t cb0 = (n0 + 64u * wn) / 16u;
+  const DqConst dq;
   uint32_t b_w[2][4];
   uint32_t b_s[4];
   auto load_b = [&](uint32_t g) {
@@ -377,7 +554,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const u4_t* __restrict__ 
     for (uint32_t j = 0; j < 4; ++j) {
       const h2_t s2 = as_h2(b_s[j] | (b_s[j] << 16));
 #pragma unroll
-      for (uint32_t ks = 0; ks < 2; ++ks) bf[ks][j] = __builtin_bit_cast(h8_t, dequant_scaled(b_w[ks][j], s2));
+      for (uint32_t ks = 0; ks < 2; ++ks) bf[ks][j] = __builtin_bit_cast(h8_t, dequant_scaled(b_w[ks][j], s2, dq));
     }
     if (g + 1 < G) {
       load_a(g + 1);
@@ -798,7 +975,7 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
     if constexpr (KV8 == 1) {
       if (live[ct]) {
 #pragma unroll
-        for (uint32_t tt = 0; tt < NT; ++tt) *reinterpret_cast<f4_t*>(a.out_rot + o + 16u * tt) = acc[ct][tt];
+        for (uint32_t tt = 0; tt < NT; ++tt) *reinterpret_cast<f4_any*>(a.out_rot + o + 16u * tt) = acc[ct][tt];
       }
       // FWHT(s * y): the stages h = 1 .. 128 in order, the pair (i, i + h) becoming (a + c, a - c):
       // h = 1, 2 inside the four values, 4 and 8 across the lane groups, 16 .. 128 across the tiles
@@ -836,7 +1013,7 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
       for (uint32_t tt = 0; tt < NT; ++tt) {
         const u2_t w = {(uint32_t)f2h(acc[ct][tt][0]) | ((uint32_t)f2h(acc[ct][tt][1]) << 16),
                         (uint32_t)f2h(acc[ct][tt][2]) | ((uint32_t)f2h(acc[ct][tt][3]) << 16)};
-        *reinterpret_cast<u2_t*>(a.attn_out + o + 16u * tt) = w;
+        *reinterpret_cast<h4_any*>(a.attn_out + o + 16u * tt) = w;
       }
     }
   }
@@ -997,13 +1174,43 @@ static int cu_count(uint32_t* cus, const char* name) {
   return 0;
 }
 
-// The work-group tile of the GEMM. Every tile sums a column over the k-groups in the same MFMA
-// order, so the choice changes the speed only, never a bit of the result. For N a multiple of
-// 256 the tile is a row of 4 waves of R x 64 (R = 128, 96 or 64): the larger R, the less
-// dequantisation and fewer loads per MFMA (measured relative rates 1 : 0.93 : 0.85), the
-// coarser the grid. The choice minimises the rows the busiest CU works through over that rate,
-// ceil(work-groups / CUs) R / rate: 128 rows for the qkv and gate||up linears of a long chunk,
-// 96 for o and down, 64 for short chunks. Otherwise 128 x 128 (2 x 2 waves of 64 x 64).
+// The work-group shape of the GEMM: rows per tile 16 ri, k parts ks (or the few-rows kernel). All but
+// the 128-row tile run one work-group of 8 waves per CU, so a launch takes ceil(work-groups / CUs)
+// rounds; a round's time over 80 k-groups (K = 5120), measured on a 256-CU part, is the table's
+// `cost` (us x 10), what a launch adds to it `over`. The rule takes the shape with the least sum.
+// Measured (us, the one 4-wave kernel of 64..128-row tiles before / this rule's choice; K -> N):
+//   5120 -> 7168: 8 rows 65.5 / 11.3 (few, 16 rows), 64: 66.4 / 20.9 (few, 32), 100: 67.6 / 27.5 (few, 64),
+//   200: 67.5 / 36 (32 x 256), 333: 68.6 / 41 (48), 500: 69.2 / 45 (64), 777: 83.4 / 63 (96),
+//   1500: 140 / 119 (96), 2048: 169 / 155 (128);
+//   17408 -> 5120: 8 rows 218 / 26, 64: 220 / 48, 333: 220 / 110, 777: 267 / 190, 2048: 414 / 368;
+//   12864 -> 2816: 8 rows 160 / 19, 64: 162 / 26, 1024: 168 / 101.
+// (The 128-row tile, 4 waves and two work-groups per CU, loses to the others until it needs fewer rounds.)
+struct GemmPick {
+  bool few;
+  uint32_t ri, ks;
+};
+static GemmPick pick_gemm(uint32_t T, uint32_t K, uint32_t N, uint32_t cus) {
+  static constexpr struct {
+    GemmPick p;
+    uint32_t cost, over;
+  } kShapes[] = {{{true, 1, 8}, 110, 20},  {{true, 2, 8}, 160, 20},  {{true, 4, 8}, 240, 20},
+                 {{false, 1, 2}, 270, 40}, {{false, 2, 2}, 330, 40}, {{false, 3, 2}, 390, 40},
+                 {{false, 4, 2}, 450, 40}, {{false, 6, 2}, 640, 40}, {{false, 8, 1}, 775, 40}};
+  GemmPick best{false, 8, 1};
+  uint64_t least = ~0ull;
+  for (const auto& s : kShapes) {
+    const uint64_t rows = (T + 16u * s.p.ri - 1u) / (16u * s.p.ri);
+    if (rows > 65535u) continue;  // the grid's limit
+    const uint64_t wg = rows * (s.p.few ? N / 64u : (N + 255u) / 256u);
+    const uint64_t t = (wg + cus - 1u) / cus * s.cost * (K / GBK) + 80ull * s.over;
+    if (t < least) {
+      least = t;
+      best = s.p;
+    }
+  }
+  return best;
+}
+
 template <bool SILU>
 static int launch_gemm(const char* name, const uint32_t* qweight, const uint16_t* scales, const uint16_t* x,
                        float* out, uint16_t* h, uint32_t T, uint32_t K, uint32_t N, void* stream) {
@@ -1021,26 +1228,25 @@ static int launch_gemm(const char* name, const uint32_t* qweight, const uint16_t
   uint32_t cus = 0;
   if (int e = cu_count(&cus, name)) return e;
   hipStream_t st = (hipStream_t)stream;
-  if (N % 256u == 0) {
-    const uint64_t C = cus;
-    auto cost = [&](uint32_t R, uint64_t rate) {  // rows on the busiest CU x 100 / rate (percent)
-      const uint64_t wg = (uint64_t)(N / 256u) * ((T + R - 1u) / R);
-      return (wg + C - 1u) / C * R * 10000u / rate;
-    };
-    const uint64_t c128 = cost(128u, 100u), c96 = cost(96u, 93u), c64 = cost(64u, 85u);
-    if (c128 <= c96 && c128 <= c64)
-      gemm_w4a16_kernel<SILU, 1, 8, 2><<<dim3(N / 256u, (T + 127u) / 128u), 256, 0, st>>>(qweight, scales, x, out,
-                                                                                          h, T, K, N);
-    else if (c96 <= c64)
-      gemm_w4a16_kernel<SILU, 1, 6, 2><<<dim3(N / 256u, (T + 95u) / 96u), 256, 0, st>>>(qweight, scales, x, out, h,
-                                                                                         T, K, N);
-    else
-      gemm_w4a16_kernel<SILU, 1, 4, 1><<<dim3(N / 256u, (T + 63u) / 64u), 256, 0, st>>>(qweight, scales, x, out, h,
-                                                                                         T, K, N);
-  } else {
-    gemm_w4a16_kernel<SILU, 2, 4, 1><<<dim3(N / 128u, (T + 127u) / 128u), 256, 0, st>>>(qweight, scales, x, out, h,
-                                                                                         T, K, N);
+  const GemmPick p = pick_gemm(T, K, N, cus);
+  const dim3 grid(p.few ? N / 64u : (N + 255u) / 256u, (T + 16u * p.ri - 1u) / (16u * p.ri));
+#define MI_GEMM(RI, KS, DA) \
+  gemm_w4a16_kernel<SILU, RI, KS, DA><<<grid, 256 * KS, 0, st>>>(qweight, scales, x, out, h, T, K, N)
+#define MI_GEMM_FEW(RI, D) \
+  gemm_w4a16_few_kernel<SILU, RI, 8, D><<<grid, 512, 0, st>>>(qweight, scales, x, out, h, T, K, N)
+  switch ((p.few ? 100u : 10u * p.ks) + p.ri) {
+    case 101: MI_GEMM_FEW(1, 4); break;
+    case 102: MI_GEMM_FEW(2, 4); break;
+    case 104: MI_GEMM_FEW(4, 2); break;
+    case 21: MI_GEMM(1, 2, 2); break;
+    case 22: MI_GEMM(2, 2, 2); break;
+    case 23: MI_GEMM(3, 2, 2); break;
+    case 24: MI_GEMM(4, 2, 2); break;
+    case 26: MI_GEMM(6, 2, 1); break;
+    default: MI_GEMM(8, 1, 1); break;
   }
+#undef MI_GEMM
+#undef MI_GEMM_FEW
   return mi_hip((int)hipGetLastError(), name);
 }
 

@@ -64,6 +64,47 @@ def test_gemm_vs_fp64(T, K, N):
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
 
 
+# the launch rule's work-group shapes on a 256-CU part, in its order (16, 32, 64 rows with the k-groups
+# over 8 waves; 16 .. 96 rows x 256 columns in two k parts; 128 rows): full and ragged rows, odd group
+# counts, fewer groups than waves or parts, a last tile of 128 columns
+@pytest.mark.parametrize("T,K,N", [(16, 448, 384), (5, 64, 128), (17, 576, 7296), (64, 320, 7168), (33, 64, 7168),
+                                   (100, 832, 7168), (16, 1856, 34816), (11, 2112, 34944), (30, 1856, 34816),
+                                   (48, 1856, 34816), (35, 2112, 34944), (64, 1856, 34816), (511, 1088, 7296),
+                                   (700, 1088, 7168), (673, 64, 7296), (1000, 320, 14464)])
+def test_gemm_work_group_shapes(T, K, N):
+    """Each shape against the fp64 product (test_gemm_vs_fp64's bound), and its SwiGLU form bitwise
+    mi_silu_mul of the fp32 output."""
+    qw, sc = weights(K, N, T + K)
+    x = O.f32_to_f16_bits(np.random.default_rng(T).standard_normal((T, K)).astype(np.float32))
+    print(f"gemm shapes T={T} K={K} N={N}", flush=True)
+    dq, ds, dx = dev(qw), dev(sc), dev(x)
+    out, h, hw = empty((T, N), np.float32), empty((T, N // 2), np.uint16), empty((T, N // 2), np.uint16)
+    mi.call("mi_gemm_w4a16", ptr(dq), ptr(ds), ptr(dx), ptr(out), T, K, N, stream())
+    mi.call("mi_gemm_w4a16_silu", ptr(dq), ptr(ds), ptr(dx), ptr(h), T, K, N, stream())
+    mi.call("mi_silu_mul", ptr(out), ptr(hw), T, N // 2, 1, stream())
+    sync()
+    got = host(out, np.float32)
+    w, xf = dequant16(qw, sc), O.f16_bits_to_f32(x).astype(np.float64)
+    bound = 2.0 ** -16 * (np.abs(xf) @ np.abs(w)) + 1e-30
+    over = np.abs(got - xf @ w) / bound
+    assert np.all(over <= 1), over.max()
+    assert np.array_equal(host(h, np.uint16), host(hw, np.uint16))
+
+
+def test_gemm_outputs_at_their_own_alignment():
+    """Outputs one element off 16 bytes: the same values."""
+    T, K, N = 40, 128, 384
+    qw, sc = weights(K, N, 1)
+    dq, ds = dev(qw), dev(sc)
+    dx = dev(O.f32_to_f16_bits(np.random.default_rng(0).standard_normal((T, K)).astype(np.float32)))
+    for call, dt, n in (("mi_gemm_w4a16", np.float32, N), ("mi_gemm_w4a16_silu", np.uint16, N // 2)):
+        a, b = empty(T * n + 1, dt), empty(T * n + 1, dt)
+        mi.call(call, ptr(dq), ptr(ds), ptr(dx), ptr(a), T, K, N, stream())
+        mi.call(call, ptr(dq), ptr(ds), ptr(dx), ptr(b) + dt().itemsize, T, K, N, stream())
+        sync()
+        assert np.array_equal(host(b, dt)[1:], host(a, dt)[:-1])
+
+
 @pytest.mark.parametrize("T,K,N", [(70, 512, 256), (70, 512, 384), (1000, 128, 14336), (2000, 64, 5120)])
 def test_gemm_exact_arithmetic(T, K, N):
     """Small-integer activations and scale 1/16: every product and partial sum is exact in fp32,
