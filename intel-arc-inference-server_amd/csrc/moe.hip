@@ -15,6 +15,8 @@
 // separate lanes (each is independent) and one lane per (column, slice) then adds them in
 // order from LDS: the same operations in the same order, spread over 256 lanes so the
 // expert weights stream at HBM rate instead of one lane per column walking K.
+#include <type_traits>
+
 #include "mi_common.h"
 #include "mi_capi_internal.h"
 #include "gemv_core.h"
@@ -33,90 +35,105 @@ __device__ __forceinline__ float rf(float v) { return h2f(f2h(v)); }
 // ---- router || shared-gate GEMV (gemv_bf16.cl:103-200), fp16 weights --------------------
 // grid (N/16, M), 16 * ksplit lanes: lane l of slice q sums column n_tile*16 + l over k8 in
 // [q*per, (q+1)*per), 8 products per k8 in k order; slices merge by the pairwise tree.
-// R rows per work-group (R > 1 for a prefill chunk's rows): the weights a lane loads serve all
-// R rows, each row's sum running in the same order as with R = 1.
-template <uint32_t R>
+// A chunk of up to 16 k8 blocks' weights and activations is loaded before any of it is used (one
+// memory round trip per chunk).
 __global__ __launch_bounds__(256) void gemv_f16w_kernel(const uint16_t* __restrict__ w,
                                                         const uint16_t* __restrict__ x,
                                                         float* __restrict__ out, uint32_t M, uint32_t K,
                                                         uint32_t N, uint32_t ksplit) {
-  __shared__ float red[R][16][16];
+  __shared__ float red[16][16];
   const uint32_t lane = threadIdx.x & 15u, q = threadIdx.x >> 4;
-  const uint32_t nt = blockIdx.x, m0 = blockIdx.y * R;
-  const uint32_t rows = min(R, M - m0);
+  const uint32_t nt = blockIdx.x, m = blockIdx.y;
   const uint32_t K8 = K / 8, per = K8 / ksplit;
   const uint16_t* tile = w + (size_t)nt * K8 * 128 + (size_t)q * per * 128 + lane;
-  const uint16_t* xr = x + (size_t)m0 * K + (size_t)q * per * 8;
-  float acc[R];
+  const uint16_t* xr = x + (size_t)m * K + (size_t)q * per * 8;
+  float acc = 0.f;
+  constexpr uint32_t CH = 16;
+  for (uint32_t k8 = 0; k8 < per; k8 += CH) {
+    uint16_t wv[CH][8];
+    u4_t xv[CH];
 #pragma unroll
-  for (uint32_t r = 0; r < R; ++r) acc[r] = 0.f;
-  uint32_t k8 = 0;
-  if constexpr (R == 1) {
-    // one row: a chunk of up to 16 k8 blocks' weights and activations is loaded before any of
-    // it is used (one memory round trip per chunk; the sum's order is unchanged)
-    constexpr uint32_t CH = 16;
-    for (; k8 < per; k8 += CH) {
-      uint16_t wv[CH][8];
-      u4_t xv[CH];
+    for (uint32_t u = 0; u < CH; ++u) {
+      const uint32_t kk = min(k8 + u, per - 1u);  // (past the slice: re-read, not added)
 #pragma unroll
-      for (uint32_t u = 0; u < CH; ++u) {
-        const uint32_t kk = min(k8 + u, per - 1u);  // (past the slice: re-read, not added)
+      for (uint32_t j = 0; j < 8; ++j) wv[u][j] = tile[(size_t)kk * 128 + j * 16];
+      xv[u] = *reinterpret_cast<const u4_t*>(xr + (size_t)kk * 8);
+    }
 #pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) wv[u][j] = tile[(size_t)kk * 128 + j * 16];
-        xv[u] = *reinterpret_cast<const u4_t*>(xr + (size_t)kk * 8);
-      }
+    for (uint32_t u = 0; u < CH; ++u) {
+      if (k8 + u < per) {
+        const uint32_t xw[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
 #pragma unroll
-      for (uint32_t u = 0; u < CH; ++u) {
-        if (k8 + u < per) {
-          const uint32_t xw[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
-#pragma unroll
-          for (uint32_t j = 0; j < 8; ++j)
-            acc[0] += h2f(wv[u][j]) * h2f((uint16_t)(xw[j / 2] >> (16 * (j % 2))));
-        }
+        for (uint32_t j = 0; j < 8; ++j) acc += h2f(wv[u][j]) * h2f((uint16_t)(xw[j / 2] >> (16 * (j % 2))));
       }
     }
   }
-  for (; k8 + 4 <= per; k8 += 4) {
-    uint16_t wv[4][8];
+  red[q][lane] = acc;
+  __syncthreads();
+  for (uint32_t stride = ksplit / 2; stride > 0; stride >>= 1) {
+    if (q < stride) red[q][lane] += red[q + stride][lane];
+    __syncthreads();
+  }
+  if (q == 0) out[(size_t)m * N + nt * 16 + lane] = red[0][lane];
+}
+
+// The same for a prefill chunk's rows, bit for bit: grid (ceil(N / 64), ceil(M / R)), 64 * ksplit
+// lanes: wave q sums slice q of 64 columns for R rows. A product of two f16 values is exact in fp32,
+// so one fma per product (v_fma_mix_f32 on the f16 operands) is the R = 1 kernel's multiply and add.
+// Bound by those fmas (2048 rows x 272 columns x 2048: 1.14 G, 29 us of issue at 2.4 GHz): the
+// activations are uniform in a wave and come through the scalar cache, the weights are loaded once
+// for R rows, so little else is issued (one 2-byte load per 8 fmas). Measured: 118 us as 16-lane
+// columns with the products and sums apart and 16-byte activation loads per lane, 73 us now.
+template <uint32_t R>
+__global__ __launch_bounds__(1024) void gemv_f16w_rows_kernel(const uint16_t* __restrict__ w,
+                                                              const uint16_t* __restrict__ x,
+                                                              float* __restrict__ out, uint32_t M, uint32_t K,
+                                                              uint32_t N, uint32_t ksplit) {
+  __shared__ float red[16][R][64];
+  const uint32_t lane = threadIdx.x & 63u, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n = blockIdx.x * 64u + lane, m0 = blockIdx.y * R;
+  const uint32_t K8 = K / 8, per = K8 / ksplit;
+  // (columns past N read the last tile's and are not stored; rows past M the last row's)
+  const uint32_t nt = min(n / 16u, N / 16u - 1u);
+  const uint16_t* tile = w + ((size_t)nt * K8 + (size_t)q * per) * 128 + n % 16u;
+  const uint16_t* xr = x + (size_t)q * per * 8;
+  float acc[R];
 #pragma unroll
-    for (uint32_t u = 0; u < 4; ++u)
+  for (uint32_t r = 0; r < R; ++r) acc[r] = 0.f;
+  constexpr uint32_t CH = 4;
+  auto block = [&](uint32_t k8, auto count) {
+    constexpr uint32_t C = decltype(count)::value;
+    uint16_t wv[C][8];
+#pragma unroll
+    for (uint32_t u = 0; u < C; ++u)
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) wv[u][j] = tile[(size_t)(k8 + u) * 128 + j * 16];
 #pragma unroll
     for (uint32_t r = 0; r < R; ++r) {
-      if (r < rows) {
-        u4_t xv[4];
+      const uint32_t* xw = reinterpret_cast<const uint32_t*>(xr + (size_t)min(m0 + r, M - 1u) * K + k8 * 8);
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) xv[u] = *reinterpret_cast<const u4_t*>(xr + (size_t)r * K + (k8 + u) * 8);
+      for (uint32_t u = 0; u < C; ++u)
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-          const uint32_t xw[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
-#pragma unroll
-          for (uint32_t j = 0; j < 8; ++j)
-            acc[r] += h2f(wv[u][j]) * h2f((uint16_t)(xw[j / 2] >> (16 * (j % 2))));
-        }
-      }
-    }
-  }
-  for (; k8 < per; ++k8)
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r)
-      if (r < rows)
         for (uint32_t j = 0; j < 8; ++j)
-          acc[r] += h2f(tile[(size_t)k8 * 128 + j * 16]) * h2f(xr[(size_t)r * K + k8 * 8 + j]);
+          acc[r] = __builtin_fmaf(h2f(wv[u][j]), h2f((uint16_t)(xw[4 * u + j / 2] >> (16 * (j % 2)))), acc[r]);
+    }
+  };
+  uint32_t k8 = 0;
+  for (; k8 + CH <= per; k8 += CH) block(k8, std::integral_constant<uint32_t, CH>{});
+  for (; k8 < per; ++k8) block(k8, std::integral_constant<uint32_t, 1>{});
 #pragma unroll
-  for (uint32_t r = 0; r < R; ++r) red[r][q][lane] = acc[r];
+  for (uint32_t r = 0; r < R; ++r) red[q][r][lane] = acc[r];
   __syncthreads();
+  // the pairwise tree over the slices, all rows and columns at once
   for (uint32_t stride = ksplit / 2; stride > 0; stride >>= 1) {
-    if (q < stride)
-#pragma unroll
-      for (uint32_t r = 0; r < R; ++r) red[r][q][lane] += red[r][q + stride][lane];
+    for (uint32_t e = threadIdx.x; e < stride * R * 64u; e += 64u * ksplit)
+      (&red[0][0][0])[e] += (&red[0][0][0])[e + stride * R * 64u];
     __syncthreads();
   }
-  if (q == 0)
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r)
-      if (r < rows) out[(size_t)(m0 + r) * N + nt * 16 + lane] = red[r][0][lane];
+  for (uint32_t e = threadIdx.x; e < R * 64u; e += 64u * ksplit) {
+    const uint32_t r = e / 64u, c = blockIdx.x * 64u + e % 64u;
+    if (m0 + r < M && c < N) out[(size_t)(m0 + r) * N + c] = red[0][r][e % 64u];
+  }
 }
 
 // ---- routing (moe.cl:192-262; twin moe_ref.h:62-96) ----------------------------------------
@@ -607,10 +624,14 @@ extern "C" int mi_gemv_f16w(const uint16_t* w_tiled, const uint16_t* x, float* o
     return mi_fail(MI_ERR_SHAPE, "gemv_f16w: ksplit must be a power of two <= 16 dividing K/8");
   if (reinterpret_cast<uintptr_t>(x) % 16) return mi_fail(MI_ERR_ARG, "gemv_f16w: x needs 16-byte alignment");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // 8 rows per work-group: the 2048-row router of 272 columns 73 us (4 rows 88; 16 rows 86, whose 640
+  // work-groups leave the second of two rounds a quarter full)
+  constexpr uint32_t R = 8;
   if (M >= 64)
-    gemv_f16w_kernel<8><<<dim3(N / 16, (M + 7) / 8), 16 * ksplit, 0, st>>>(w_tiled, x, out, M, K, N, ksplit);
+    gemv_f16w_rows_kernel<R><<<dim3((N + 63) / 64, (M + R - 1) / R), 64 * ksplit, 0, st>>>(w_tiled, x, out, M, K, N,
+                                                                                           ksplit);
   else
-    gemv_f16w_kernel<1><<<dim3(N / 16, M), 16 * ksplit, 0, st>>>(w_tiled, x, out, M, K, N, ksplit);
+    gemv_f16w_kernel<<<dim3(N / 16, M), 16 * ksplit, 0, st>>>(w_tiled, x, out, M, K, N, ksplit);
   return mi_hip(static_cast<int>(hipGetLastError()), "gemv_f16w launch");
 }
 

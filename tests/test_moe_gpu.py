@@ -345,6 +345,66 @@ def test_moe_prefill_matches_decode_kernels(T, bad):
     assert 1 <= n_tiles <= (P + 63) // 64 + E + 1
 
 
+# mean pairs per expert at the launch rule's edges (20 / 21 and 52 / 53: tiles of at most 32, 64 and 96
+# rows), with random routes and with every row on the same experts (whole tiles and remainders)
+@pytest.mark.parametrize("T,K,skew", [(16, 1, False), (40, 8, False), (42, 8, False), (42, 8, True), (104, 8, False),
+                                      (104, 7, True), (107, 8, False), (97, 8, True), (193, 5, True), (129, 8, True)])
+def test_moe_prefill_tile_shapes(T, K, skew):
+    """mi_moe_prefill's row tiles against the oracle of the prefill block (rel 2e-3, as
+    test_moe_prefill_matches_decode_kernels), the pairs' list the stable sort by expert."""
+    E, H, I = 16, 512, 128
+    mo = Moe(5, E=E, top_k=K, hidden=H, inter=I, router_n=32)
+    rng = np.random.default_rng(T + K)
+    x = O.f32_to_f16_bits(rng.standard_normal((T, H)).astype(np.float32))
+    resid0 = O.f32_to_f16_bits(rng.standard_normal((T, H)).astype(np.float32))
+    rt = np.zeros((T, ROUTE_WORDS), np.uint32)
+    rt[:, :K] = np.arange(K) if skew else np.argsort(rng.random((T, E)), axis=1)[:, :K]
+    w = rng.dirichlet(np.ones(K), T).astype(np.float16).astype(np.float32)
+    rt[:, 8:8 + K] = w.view(np.uint32)
+    rt[:, 16] = rng.random(T).astype(np.float16).astype(np.float32).view(np.uint32)
+    P = T * (K + 1)
+    lst, tiles, tiles_n = empty(P, np.uint32), empty(((P + 63) // 64 + E + 1) * 4, np.uint32), empty(1, np.uint32)
+    hh, dd, resid = empty((P, I), np.uint16), empty((P, H), np.uint16), dev(resid0)
+    droute, dx = dev(rt), dev(x)
+    print(f"moe_prefill tiles T={T} K={K} skew={skew}", flush=True)
+    mi.call("mi_moe_prefill", ptr(droute), ptr(dx), ptr(mo.d_gu), ptr(mo.d_dn), ptr(resid), T, E, K, H, I, ptr(lst),
+            ptr(tiles), ptr(tiles_n), ptr(hh), ptr(dd), stream())
+    sync()
+    got = O.f16_bits_to_f32(host(resid, np.uint16).reshape(T, H)).astype(np.float64)
+    orc = resid0.copy()
+    O.lib().orc_moe_prefill(O.ORC_F16, E, K, H, I, O._p(rt), O._p(x), O._p(mo.gu), O._p(mo.dn), O._p(orc), T)
+    want = O.f16_bits_to_f32(orc).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2e-3 * np.abs(want) + 2e-3 * np.abs(want).max())
+    ex = np.concatenate([rt[:, :K].astype(np.int64), np.full((T, 1), E)], axis=1).ravel()
+    assert np.array_equal(host(lst, np.uint32), np.argsort(ex, kind="stable").astype(np.uint32))
+
+
+@pytest.mark.parametrize("M,K,N,ksplit", [(64, 64, 16, 8), (65, 128, 80, 4), (71, 1088, 272, 8), (100, 576, 48, 1),
+                                          (130, 2048, 272, 16), (64, 4096, 128, 16)])
+def test_router_gemv_of_a_chunk_is_bitwise_the_short_launches(M, K, N, ksplit):
+    """64 rows and more take the kernel of 64 columns and 8 rows per work-group: every output bitwise
+    the oracle's and the launches' of fewer rows (slices of 1 .. 72 k8 blocks, ragged rows and
+    columns, a zero and the largest and smallest f16 values among the operands)."""
+    rng = np.random.default_rng(M + K)
+    w = O.f32_to_f16_bits((0.02 * rng.standard_normal((N, K))).astype(np.float32))
+    x = O.f32_to_f16_bits(rng.standard_normal((M, K)).astype(np.float32))
+    w.ravel()[::97], x.ravel()[::89], x.ravel()[5::101] = 0x0001, 0x8001, 0x8000
+    w.ravel()[3::211], x.ravel()[7::307] = 0x03FF, 0x7BFF
+    wt = np.empty(N * K, np.uint16)
+    O.lib().orc_f16w_tile(O._p(w), K, N, O._p(wt))
+    want = np.empty((M, N), np.float32)
+    O.lib().orc_gemv_f16w(F16, O._p(wt), O._p(x), M, K, N, ksplit, O._p(want))
+    dw, dx, out = dev(wt), dev(x), empty((M, N), np.float32)
+    print(f"gemv_f16w rows M={M} K={K} N={N} ksplit={ksplit}", flush=True)
+    mi.call("mi_gemv_f16w", ptr(dw), ptr(dx), ptr(out), M, K, N, ksplit, stream())
+    short = empty((63, N), np.float32)
+    mi.call("mi_gemv_f16w", ptr(dw), ptr(dx), ptr(short), 63, K, N, ksplit, stream())
+    sync()
+    got = host(out, np.uint32).reshape(M, N)
+    assert np.array_equal(got, want.view(np.uint32))
+    assert np.array_equal(got[:63], host(short, np.uint32).reshape(63, N))
+
+
 def test_moe_prefill_refuses_bad_shapes():
     with pytest.raises(mi.MiError):
         mi.call("mi_moe_prefill", 16, 16, 16, 16, 16, 2049, 256, 8, 2048, 512, 16, 16, 16, 16, 16, None)
