@@ -99,6 +99,7 @@ __device__ __forceinline__ u4_t dequant_scaled(uint32_t w, h2_t s2, const DqCons
 // outputs are stored in pieces of several elements at the elements' own alignment
 typedef f4_t f4_any __attribute__((aligned(4)));
 typedef u2_t h4_any __attribute__((aligned(2)));
+typedef u4_t h8_any __attribute__((aligned(2)));
 
 // A wave's 64 columns: lane (fr, fq) = (l % 16, l / 16) reads word row fq of a half group's four at
 // columns 4 fr .. 4 fr + 3 (one 16-byte load), and column 4 fr + j is column fr of the wave's matrix
@@ -389,54 +390,68 @@ __global__ __launch_bounds__(64 * KW, KW > 8 ? 4 : 2) void gemm_w4a16_few_kernel
 // (moe.cl:383-470's epilogue, moe_ref.h:144-152) runs per row afterwards.
 constexpr uint32_t kMoeRouteWords = 32, kMoeW = 8, kMoeSG = 16;  // the route row (moe.cl:49-56)
 constexpr uint32_t kMoeTile = 136;                                 // layout 1: 128 words + 16 f16 scales
-constexpr uint32_t kMoeRows = 64;                                  // pairs per row tile
 constexpr uint32_t kMoeMaxPairs = 2048u * 9u;                      // T <= 2048, top_k <= 8
-
-// the expert of slot s of a route row: the shared expert (index E) for s = top_k, and for an
-// id outside [0, E) (moe.hip's slot_expert)
-__device__ __forceinline__ uint32_t moe_slot_expert(const uint32_t* row, uint32_t s, uint32_t E, uint32_t top_k) {
-  if (s >= top_k) return E;
-  const uint32_t id = row[s];
-  return id < E ? id : E;
-}
 
 // One work-group, a stable counting sort of the pairs p = t (top_k + 1) + s of T rows by expert:
 // expert e's pairs go to list[off_e ..] in ascending p (the reference's (token, slot) order), its
 // row tiles to tiles[] as {e, first list index, pair count}, the tile count to tiles_n[0]. Wave w (of
 // 16) owns the pairs [w Q, (w + 1) Q): it counts them per expert, then places them 64 at a time, a
 // lane's rank among the lanes of its expert coming from a match mask built from 9 ballots (one per
-// bit of the expert index), so list[] is the same on every call.
+// bit of the expert index), so list[] is the same on every call. Latency-bound (2048 rows x 9 pairs):
+// 31 us with the offsets summed by one thread and a division per pair, 22 now.
 __global__ __launch_bounds__(1024) void moe_group_kernel(const uint32_t* __restrict__ route, uint32_t T,
-                                                        uint32_t E, uint32_t top_k, uint32_t* __restrict__ list,
+                                                        uint32_t E, uint32_t top_k, uint32_t tile_rows,
+                                                        uint32_t* __restrict__ list,
                                                         u4_t* __restrict__ tiles, uint32_t* __restrict__ tiles_n) {
   __shared__ uint16_t s_ex[kMoeMaxPairs];
   constexpr uint32_t kW = 16, kT = kW * 64;
-  __shared__ uint32_t s_wc[kW][257], s_off[257], s_toff[257], s_cnt[257];
+  __shared__ uint32_t s_wc[kW][257], s_off[257], s_toff[257], s_cnt[257], s_wsum[kW][2];
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, slots = top_k + 1, P = T * slots;
   for (uint32_t e = t; e <= E; e += kT)
     for (uint32_t w = 0; w < kW; ++w) s_wc[w][e] = 0;
-  for (uint32_t p = t; p < P; p += kT)
-    s_ex[p] = (uint16_t)moe_slot_expert(route + (size_t)(p / slots) * kMoeRouteWords, p % slots, E, top_k);
+  for (uint32_t r = t; r < T; r += kT) {  // a thread per row, its ids' loads together
+    uint32_t id[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) id[k] = route[(size_t)r * kMoeRouteWords + k];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k)
+      if (k < top_k) s_ex[r * slots + k] = (uint16_t)min(id[k], E);  // (an id outside [0, E): the shared expert)
+    s_ex[r * slots + top_k] = (uint16_t)E;
+  }
   __syncthreads();
   const uint32_t Q = (P + kW - 1u) / kW, lo = min(P, wave * Q), hi = min(P, lo + Q);
   for (uint32_t p = lo + lane; p < hi; p += 64u) atomicAdd(&s_wc[wave][s_ex[p]], 1u);  // counts only
   __syncthreads();
-  for (uint32_t e = t; e <= E; e += kT) {
-    uint32_t c = 0;
-    for (uint32_t w = 0; w < kW; ++w) c += s_wc[w][e];
-    s_cnt[e] = c;
+  // the experts' first list indices and tiles: exclusive sums over the experts, thread e expert e
+  // (the lanes of a wave by shuffles, then the waves before it; E <= 256 < kT)
+  uint32_t c = 0;
+  if (t <= E)
+    for (uint32_t w = 0; w < kW; ++w) c += s_wc[w][t];
+  const uint32_t ct = (c + tile_rows - 1u) / tile_rows;
+  uint32_t o = c, to = ct;
+#pragma unroll
+  for (uint32_t d = 1; d < 64u; d *= 2) {
+    const uint32_t po = __shfl_up(o, d, 64), pt = __shfl_up(to, d, 64);
+    if (lane >= d) {
+      o += po;
+      to += pt;
+    }
+  }
+  if (lane == 63u) {
+    s_wsum[wave][0] = o;
+    s_wsum[wave][1] = to;
   }
   __syncthreads();
-  if (t == 0) {
-    uint32_t o = 0, to = 0;
-    for (uint32_t e = 0; e <= E; ++e) {
-      s_off[e] = o;
-      s_toff[e] = to;
-      o += s_cnt[e];
-      to += (s_cnt[e] + kMoeRows - 1u) / kMoeRows;
-    }
-    tiles_n[0] = to;
+  for (uint32_t w = 0; w < wave; ++w) {
+    o += s_wsum[w][0];
+    to += s_wsum[w][1];
   }
+  if (t <= E) {
+    s_cnt[t] = c;
+    s_off[t] = o - c;
+    s_toff[t] = to - ct;
+  }
+  if (t == E) tiles_n[0] = to;
   __syncthreads();
   for (uint32_t e = t; e <= E; e += kT) {  // s_wc becomes each wave's next list index per expert
     uint32_t b = s_off[e];
@@ -467,8 +482,8 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const uint32_t* __restr
   }
   for (uint32_t e = t; e <= E; e += kT) {
     const uint32_t n = s_cnt[e];
-    for (uint32_t k = 0; k * kMoeRows < n; ++k)
-      tiles[s_toff[e] + k] = u4_t{e, s_off[e] + k * kMoeRows, min(kMoeRows, n - k * kMoeRows), 0u};
+    for (uint32_t k = 0; k * tile_rows < n; ++k)
+      tiles[s_toff[e] + k] = u4_t{e, s_off[e] + k * tile_rows, min(tile_rows, n - k * tile_rows), 0u};
   }
 }
 
@@ -477,148 +492,191 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const uint32_t* __restr
 // at j 16 + c, its f16 scale at half-word 256 + c). A row of a pair p is row p / slots of x
 // (GATE_UP) or row p of h (down). GATE_UP: N = 2 inter in interleave16 order, SwiGLU in the
 // epilogue into h[p][inter] (the dense GEMM's epilogue); down: d[p][N] rounded to f16 (the
-// combine's first rounding of a slot's value, so nothing is lost). Tile: 64 pairs x
-// 256 columns, 4 waves of 64 x 64, the dense GEMM's k loop.
-template <bool GATE_UP>
-__global__ __launch_bounds__(256) void moe_gemm_kernel(const u4_t* __restrict__ tiles,
-                                                       const uint32_t* __restrict__ tiles_n,
-                                                       const uint32_t* __restrict__ list,
-                                                       const uint32_t* __restrict__ blocks, size_t block_u32,
-                                                       const uint16_t* __restrict__ a, uint32_t a_rows,
-                                                       uint16_t* __restrict__ h_out, uint16_t* __restrict__ d_out,
-                                                       uint32_t slots, uint32_t K, uint32_t N) {
-  __shared__ __align__(16) uint16_t As[2][kMoeRows][GROW];
-  if (blockIdx.y >= tiles_n[0]) return;  // uniform: the grid is sized for the most tiles
-  const u4_t tile = tiles[blockIdx.y];
-  const uint32_t e = tile.x, first = tile.y, cnt = tile.z;
-  const uint32_t t = threadIdx.x, lane = t & 63u, wn = t >> 6;
-  const uint32_t n0 = blockIdx.x * 256u, G = K / GBK;
-  const uint32_t fr = lane & 15u, fq = lane >> 4;
+// combine's first rounding of a slot's value, so nothing is lost). Tile: up to 96 pairs x 256
+// columns, 4 waves side by side, the dense GEMM's loop for the tile's 16-row blocks (1 .. 6, uniform):
+// at top 8 of 256 experts a 2048-row chunk has 64 +- 8 pairs per expert, one tile of 4 or 5 blocks,
+// where tiles of 64 rows took a second, nearly empty one for half of the experts. Bound by the
+// products and the weights' latency (77 + 39 GFLOP over 428 MB there): gate||up 166 -> 135 us, down
+// 98 -> 85 at 2048 rows; 512 rows: the block 230 -> 178.
+struct MoeGemm {
+  const u4_t* tiles;
+  const uint32_t *tiles_n, *list, *blocks;
+  const uint16_t* a;
+  uint16_t *h_out, *d_out;
+  size_t block_u32;
+  uint32_t a_rows, slots, K, N;
+};
 
-  // activations: thread t stages pairs (t >> 3) + 32 i (i < 2), 8-k chunk t & 7; a pair past
-  // the tile's count gets an offset outside the resource and reads zeros
+template <bool GATE_UP, uint32_t RI, uint32_t ROWS>
+__device__ __forceinline__ void moe_gemm_tile(const MoeGemm& m, const u4_t& tile, uint16_t (&As)[2][ROWS][GROW]) {
+  constexpr uint32_t BM = 16u * RI, AI = (BM + 31u) / 32u;
+  const uint32_t e = tile.x, first = tile.y, cnt = tile.z, K = m.K, N = m.N, G = K / GBK;
+  const uint32_t t = threadIdx.x, lane = t & 63u, wn = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t fr = lane & 15u, fq = lane >> 4, n0 = blockIdx.x * 256u + 64u * wn;
+
+  // activations: thread t stages pairs (t >> 3) + 32 i, 8-k chunk t & 7; a pair past the tile's
+  // count gets an offset outside the resource and reads zeros
   const uint32_t a_row = t >> 3, a_chunk = t & 7u;
   const __amdgpu_buffer_rsrc_t x_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a), 0, a_rows * K * 2u, 0x00020000);
-  uint32_t a_voff[2];
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(m.a), 0, m.a_rows * K * 2u, 0x00020000);
+  uint32_t a_voff[AI];
 #pragma unroll
-  for (uint32_t i = 0; i < 2; ++i) {
-    const uint32_t r = a_row + 32u * i;
-    const uint32_t p = r < cnt ? list[first + r] : 0u;
-    const uint32_t src = GATE_UP ? p / slots : p;
-    a_voff[i] = r < cnt ? (src * K + 8u * a_chunk) * 2u : 0x80000000u;
+  for (uint32_t i = 0; i < AI; ++i) {
+    const uint32_t r = a_row + 32u * i, p = m.list[first + min(r, cnt - 1u)];
+    a_voff[i] = r < cnt ? ((GATE_UP ? p / m.slots : p) * K + 8u * a_chunk) * 2u : 0x80000000u;
   }
-  u4_t a_st[2];
-  auto load_a = [&](uint32_t g) {
+  // weights: lane (fr, fq) takes columns n0 + 4 fr .. + 3 (as in the dense GEMM): 16-column tile
+  // fr / 4 of the wave's four, word row fq of a half group's, its columns 4 (fr % 4) ..
+  const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint32_t*>(m.blocks + (size_t)e * m.block_u32), 0, (uint32_t)(m.block_u32 * 4u), 0x00020000);
+  const uint32_t t_voff = (fr >> 2) * G * kMoeTile * 4u, w_voff = t_voff + (fq * 16u + 4u * (fr & 3u)) * 4u;
+  const uint32_t s_voff = t_voff + (256u + 4u * (fr & 3u)) * 2u, base = n0 / 16u * G * kMoeTile * 4u;
+  u4_t a_st[AI];
+  BGroup b_st[2];
+  auto load_a = [&](uint32_t g) {  // (a group past the last re-reads it and is not multiplied)
+    const uint32_t so = min(g, G - 1u) * GBK * 2u;
 #pragma unroll
-    for (uint32_t i = 0; i < 2; ++i)
-      a_st[i] = __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rs, a_voff[i], g * GBK * 2u, 0));
+    for (uint32_t i = 0; i < AI; ++i)
+      a_st[i] = __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rs, a_voff[i], so, 0));
+  };
+  auto load_b = [&](uint32_t g, BGroup& b) {
+    const uint32_t so = base + min(g, G - 1u) * kMoeTile * 4u;
+#pragma unroll
+    for (uint32_t ks = 0; ks < 2; ++ks)
+      b.w[ks] = __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rs, w_voff, so + 256u * ks, 2));
+    b.s = __builtin_bit_cast(u2_t, __builtin_amdgcn_raw_buffer_load_b64(w_rs, s_voff, so, 0));
   };
   auto store_a = [&](uint32_t buf) {
 #pragma unroll
-    for (uint32_t i = 0; i < 2; ++i)
-      *reinterpret_cast<u4_t*>(&As[buf][a_row + 32u * i][8u * a_chunk]) = perm_pairs(a_st[i]);
-  };
-  // weights: column n = n0 + 64 wn + 16 j + fr sits in 16-column tile n / 16 at column fr
-  const uint32_t* wb = blocks + (size_t)e * block_u32;
-  const __amdgpu_buffer_rsrc_t w_rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(wb), 0, (uint32_t)(block_u32 * 4u), 0x00020000);
-  const uint32_t cb0 = (n0 + 64u * wn) / 16u;
-  const DqConst dq;
-  uint32_t b_w[2][4];
-  uint32_t b_s[4];
-  auto load_b = [&](uint32_t g) {
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-      const uint32_t tb = ((cb0 + j) * G + g) * kMoeTile;  // u32 index of the tile
-#pragma unroll
-      for (uint32_t ks = 0; ks < 2; ++ks)
-        b_w[ks][j] = __builtin_amdgcn_raw_buffer_load_b32(w_rs, ((4u * ks + fq) * 16u + fr) * 4u, tb * 4u, 2);
-      b_s[j] = __builtin_amdgcn_raw_buffer_load_b16(w_rs, (256u + fr) * 2u, tb * 4u, 0);
-    }
+    for (uint32_t i = 0; i < AI; ++i)
+      if (32u * (i + 1u) <= BM || a_row + 32u * i < BM)
+        *reinterpret_cast<u4_t*>(&As[buf][a_row + 32u * i][8u * a_chunk]) = perm_pairs(a_st[i]);
   };
 
-  f4_t acc[4][4];
+  f4_t acc[RI][4];
 #pragma unroll
-  for (uint32_t i = 0; i < 4; ++i)
+  for (uint32_t i = 0; i < RI; ++i)
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+  const DqConst dq;
+  h8_t bf[2][4];
+  load_b(0, b_st[0]);
   load_a(0);
-  load_b(0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_b(1, b_st[1]);
   store_a(0);
+  dequant_half(b_st[0], 0, dq, bf[0]);
+  pin(bf[0]);
   lds_barrier();
-  for (uint32_t g = 0; g < G; ++g) {
-    const uint32_t buf = g & 1u;
-    h8_t bf[2][4];
+  // (G is even: hidden a multiple of 512, inter of 128)
+  for (uint32_t g0 = 0; g0 < G; g0 += 2u) {
 #pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-      const h2_t s2 = as_h2(b_s[j] | (b_s[j] << 16));
+    for (uint32_t u = 0; u < 2u; ++u) {
+      const uint32_t g = g0 + u;
+      load_a(g + 1u);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (uint32_t ks = 0; ks < 2; ++ks) bf[ks][j] = __builtin_bit_cast(h8_t, dequant_scaled(b_w[ks][j], s2, dq));
+      for (uint32_t ks = 0; ks < 2; ++ks) {
+        h8_t af[RI];
+#pragma unroll
+        for (uint32_t i = 0; i < RI; ++i)
+          af[i] = *reinterpret_cast<const h8_t*>(&As[u][16u * i + fr][32u * ks + 8u * fq]);
+#pragma unroll
+        for (uint32_t i = 0; i < RI; ++i)
+#pragma unroll
+          for (uint32_t j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[ks][j], acc[i][j], 0, 0, 0);
+        dequant_half(b_st[ks ? u ^ 1u : u], ks ^ 1u, dq, bf[ks ^ 1u]);
+        pin(bf[ks ^ 1u]);
+        if (ks == 0) load_b(g + 2u, b_st[u]);
+      }
+      store_a(u ^ 1u);
+      lds_barrier();
     }
-    if (g + 1 < G) {
-      load_a(g + 1);
-      load_b(g + 1);
-    }
-#pragma unroll
-    for (uint32_t ks = 0; ks < 2; ++ks) {
-      h8_t af[4];
-#pragma unroll
-      for (uint32_t i = 0; i < 4; ++i)
-        af[i] = *reinterpret_cast<const h8_t*>(&As[buf][16u * i + fr][32u * ks + 8u * fq]);
-#pragma unroll
-      for (uint32_t i = 0; i < 4; ++i)
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf[ks][j], acc[i][j], 0, 0, 0);
-    }
-    if (g + 1 < G) store_a(buf ^ 1u);
-    lds_barrier();
   }
-  // lane holds pairs 4 (lane >> 4) + r of column lane & 15 of each 16 x 16 tile
+  // lane holds pairs 4 fq + r of columns n0 + 4 fr .. + 3 of each 16-row block
 #pragma unroll
-  for (uint32_t i = 0; i < 4; ++i)
+  for (uint32_t i = 0; i < RI; ++i)
 #pragma unroll
     for (uint32_t r = 0; r < 4; ++r) {
-      const uint32_t q = 16u * i + 4u * fq + r;
-      if (q < cnt) {
-        const uint32_t p = list[first + q];
-        if constexpr (GATE_UP) {
-#pragma unroll
-          for (uint32_t jp = 0; jp < 2; ++jp) {
-            const uint16_t g_b = f2h(acc[i][2 * jp][r]), u_b = f2h(acc[i][2 * jp + 1][r]);
-            const uint16_t s_b = f2h(silu_f32(h2f(g_b)));
-            h_out[(size_t)p * (N / 2) + (n0 + 64u * wn) / 2 + 16u * jp + fr] = f2h(h2f(s_b) * h2f(u_b));
-          }
-        } else {
-#pragma unroll
-          for (uint32_t j = 0; j < 4; ++j) d_out[(size_t)p * N + n0 + 64u * wn + 16u * j + fr] = f2h(acc[i][j][r]);
-        }
+      const uint32_t q = 16u * i + 4u * fq + r, p = m.list[first + min(q, cnt - 1u)];
+      const f4_t v = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
+      if constexpr (GATE_UP) {
+        store_row4<true>(v, q < cnt, nullptr, m.h_out, p, n0 + 4u * fr, N);
+      } else if (q < cnt) {
+        *reinterpret_cast<h4_any*>(m.d_out + (size_t)p * N + n0 + 4u * fr) =
+            u2_t{(uint32_t)f2h(v[0]) | ((uint32_t)f2h(v[1]) << 16), (uint32_t)f2h(v[2]) | ((uint32_t)f2h(v[3]) << 16)};
       }
     }
 }
 
+// RMAX: the most 16-row blocks of a work-group's tile. Its registers set the waves in flight, so
+// few pairs per expert, where the weights' stream is the bound, take RMAX 2: half of a 64-row tile
+// per work-group (grid z), five waves per SIMD.
+template <bool GATE_UP, uint32_t RMAX>
+__global__ __launch_bounds__(256, RMAX == 2 ? 4 : RMAX == 4 ? 3 : 2) void moe_gemm_kernel(MoeGemm m) {
+  __shared__ __align__(16) uint16_t As[2][16u * RMAX][GROW];
+  if (blockIdx.y >= m.tiles_n[0]) return;  // uniform: the grid is sized for the most tiles
+  u4_t tile = m.tiles[blockIdx.y];
+  if constexpr (RMAX == 2) {
+    const uint32_t skip = 32u * blockIdx.z;
+    if (skip >= tile.z) return;
+    tile.y += skip;
+    tile.z = min(32u, tile.z - skip);
+  }
+  const uint32_t ri = (tile.z + 15u) / 16u;
+  if (ri == 1u) moe_gemm_tile<GATE_UP, 1>(m, tile, As);
+  else if (RMAX == 2 || ri == 2u) moe_gemm_tile<GATE_UP, 2>(m, tile, As);
+  if constexpr (RMAX > 2) {
+    if (ri == 3u) moe_gemm_tile<GATE_UP, 3>(m, tile, As);
+    else if (ri == 4u) moe_gemm_tile<GATE_UP, 4>(m, tile, As);
+  }
+  if constexpr (RMAX > 4) {
+    if (ri == 5u) moe_gemm_tile<GATE_UP, 5>(m, tile, As);
+    else if (ri > 5u) moe_gemm_tile<GATE_UP, 6>(m, tile, As);
+  }
+}
+
 // resid[t][n] += the slot-ordered combine of row t's pair outputs (moe_down_kernel's epilogue,
 // moe_ref.h:144-152): sum_k rne(rne(d_k) w_k) in slot order, + rne(rne(d_shared) s)
+// Eight columns per thread, the slots' pieces loaded together: bound by the pair outputs' bytes
+// (2048 rows x 9 x 2048: 75 MB; 16 us, 30 with a column per thread).
 __global__ __launch_bounds__(256) void moe_combine_kernel(const uint32_t* __restrict__ route,
                                                           const uint16_t* __restrict__ d, uint16_t* __restrict__ resid,
-                                                          uint32_t top_k, uint32_t hidden) {
-  const uint32_t t = blockIdx.y, n = blockIdx.x * 256u + threadIdx.x;
-  if (n >= hidden) return;
+                                                          uint32_t T, uint32_t top_k, uint32_t hidden) {
+  const uint32_t h8 = hidden / 8u, i = blockIdx.x * 256u + threadIdx.x, t = i / h8, n = 8u * (i - t * h8);
+  if (t >= T) return;
   const uint32_t* row = route + (size_t)t * kMoeRouteWords;
   const uint32_t slots = top_k + 1;
   const uint16_t* dp = d + (size_t)t * slots * hidden + n;
-  float sum = 0.f;
-  for (uint32_t k = 0; k < top_k; ++k) {
-    const float wk = __builtin_bit_cast(float, row[kMoeW + k]);
-    sum += h2f(f2h(h2f(dp[(size_t)k * hidden]) * wk));
-  }
-  const uint16_t r_b = f2h(sum);
+  h8_any* rp = reinterpret_cast<h8_any*>(resid + (size_t)t * hidden + n);
+  u4_t v[9];
+#pragma unroll
+  for (uint32_t k = 0; k < 9; ++k) v[k] = *reinterpret_cast<const h8_any*>(dp + (size_t)min(k, top_k) * hidden);
+  const u4_t rv = *rp;
+  float wk[8];
+#pragma unroll
+  for (uint32_t k = 0; k < 8; ++k) wk[k] = __builtin_bit_cast(float, row[kMoeW + k]);
   const float sg = __builtin_bit_cast(float, row[kMoeSG]);
-  const uint16_t sh_b = f2h(h2f(dp[(size_t)top_k * hidden]) * sg);
-  const uint16_t o_b = f2h(h2f(r_b) + h2f(sh_b));
-  uint16_t* rp = resid + (size_t)t * hidden + n;
-  *rp = f2h(h2f(*rp) + h2f(o_b));
+  u4_t o;
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q) {
+    uint32_t half[2];
+#pragma unroll
+    for (uint32_t c = 0; c < 2; ++c) {
+      auto at = [&](const u4_t& u) { return h2f((uint16_t)(u[q] >> (16u * c))); };
+      float sum = 0.f;
+#pragma unroll
+      for (uint32_t k = 0; k < 8; ++k)
+        if (k < top_k) sum += h2f(f2h(at(v[k]) * wk[k]));
+      // (v[8]: slot top_k, as every piece from top_k on)
+      const uint16_t r_b = f2h(sum), sh_b = f2h(at(v[8]) * sg);
+      const uint16_t o_b = f2h(h2f(r_b) + h2f(sh_b));
+      half[c] = f2h(at(rv) + h2f(o_b));
+    }
+    o[q] = half[0] | (half[1] << 16);
+  }
+  *rp = o;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1281,18 +1339,31 @@ int mi_moe_prefill(const uint32_t* route, const uint16_t* x, const uint32_t* gu_
       reinterpret_cast<uintptr_t>(dn_blocks) % 4)
     return mi_fail(MI_ERR_ARG, "moe_prefill: tiles, x and h need 16-byte, gu_blocks and dn_blocks 4-byte alignment");
   const uint32_t slots = top_k + 1, P = T * slots;
-  const uint32_t max_tiles = (P + kMoeRows - 1u) / kMoeRows + experts + 1u;
+  // the tile's most 16-row blocks by the mean pairs per expert (256 experts, top 8, 2048 -> 512; the whole
+  // block in us at 2 / 4 / 6): 10 pairs 156 / 161 / 185, 16: 178 / 182 / 207, 32: 254 / 227 / 249,
+  // 47: 336 / 273 / 295, 64: 415 / 352 / 345
+  const uint32_t mean = T * top_k / experts, rmax = mean <= 20u ? 2u : mean <= 52u ? 4u : 6u;
+  const uint32_t tile_rows = rmax == 6u ? 96u : 64u;
+  const uint32_t max_tiles = (P + tile_rows - 1u) / tile_rows + experts + 1u;
   const size_t gu_block = (size_t)(2u * inter / 16u) * (hidden / GBK) * kMoeTile;
   const size_t dn_block = (size_t)(hidden / 16u) * (inter / GBK) * kMoeTile;
   hipStream_t st = (hipStream_t)stream;
   u4_t* tl = reinterpret_cast<u4_t*>(tiles);
-  moe_group_kernel<<<1, 1024, 0, st>>>(route, T, experts, top_k, list, tl, tiles_n);
-  moe_gemm_kernel<true><<<dim3(2u * inter / 256u, max_tiles), 256, 0, st>>>(tl, tiles_n, list, gu_blocks, gu_block,
-                                                                            x, T, h, nullptr, slots, hidden,
-                                                                            2u * inter);
-  moe_gemm_kernel<false><<<dim3(hidden / 256u, max_tiles), 256, 0, st>>>(tl, tiles_n, list, dn_blocks, dn_block, h,
-                                                                          P, nullptr, d, slots, inter, hidden);
-  moe_combine_kernel<<<dim3(hidden / 256u, T), 256, 0, st>>>(route, d, resid, top_k, hidden);
+  moe_group_kernel<<<1, 1024, 0, st>>>(route, T, experts, top_k, tile_rows, list, tl, tiles_n);
+  const MoeGemm up{tl, tiles_n, list, gu_blocks, x, h, nullptr, gu_block, T, slots, hidden, 2u * inter};
+  const MoeGemm down{tl, tiles_n, list, dn_blocks, h, nullptr, d, dn_block, P, slots, inter, hidden};
+  const dim3 up_grid(2u * inter / 256u, max_tiles, rmax == 2u ? 2u : 1u), down_grid(hidden / 256u, max_tiles, up_grid.z);
+  if (rmax == 2u) {
+    moe_gemm_kernel<true, 2><<<up_grid, 256, 0, st>>>(up);
+    moe_gemm_kernel<false, 2><<<down_grid, 256, 0, st>>>(down);
+  } else if (rmax == 4u) {
+    moe_gemm_kernel<true, 4><<<up_grid, 256, 0, st>>>(up);
+    moe_gemm_kernel<false, 4><<<down_grid, 256, 0, st>>>(down);
+  } else {
+    moe_gemm_kernel<true, 6><<<up_grid, 256, 0, st>>>(up);
+    moe_gemm_kernel<false, 6><<<down_grid, 256, 0, st>>>(down);
+  }
+  moe_combine_kernel<<<(T * (hidden / 8u) + 255u) / 256u, 256, 0, st>>>(route, d, resid, T, top_k, hidden);
   return mi_hip((int)hipGetLastError(), "moe_prefill");
 }
 
