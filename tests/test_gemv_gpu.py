@@ -124,3 +124,22 @@ def test_cfg1_gemv_fp16_out():
     assert np.all(np.abs(y - twin) <= 2e-3 * np.abs(twin) + 1e-3 * np.abs(twin).max())
     # fp16 output: N2 widened by the final fp16 rounding (half an ulp of the result)
     assert np.all(np.abs(y - ref[0]) <= np.ldexp(bound[0], -16) + np.abs(ref[0]) * 2.0 ** -11 + 1e-7)
+
+
+@pytest.mark.parametrize("S,M,N,off", [(1, 1, 64, 0), (15, 3, 7, 0), (16, 1, 65535, 0), (17, 2, 32768, 0), (33, 2, 32768, 1),
+                                       (2, 1, 65538, 1)])
+def test_fold_partials_in_slice_order(S, M, N, off):
+    """The fold over one, under, exactly and over 16 slices, one and four outputs per thread, partials
+    one float off 16 bytes: bitwise the ascending fp32 sums from 0, and their f16 rounding."""
+    rng = np.random.default_rng(S * N)
+    part = rng.standard_normal((S, M, N)).astype(np.float32)
+    buf = np.zeros(S * M * N + 1, np.float32)
+    buf[off:off + S * M * N] = part.ravel()
+    want = np.zeros((M, N), np.float32)
+    for s in range(S):
+        want = want + part[s]
+    d, o16, o32 = dev(buf), empty((M, N), np.uint16), empty((M, N), np.float32)
+    mi.call("mi_fold_partials", ptr(d) + 4 * off, ptr(o16), ptr(o32), S, M, N, stream())
+    sync()
+    assert np.array_equal(host(o32, np.uint32), want.view(np.uint32))
+    assert np.array_equal(host(o16, np.uint16), O.f32_to_f16_bits(want))
