@@ -305,9 +305,7 @@ __device__ __forceinline__ void qkv_consumer(const float* partials, uint32_t M, 
     float acc;
     if constexpr (EPL == 4) acc = (sq[0] + sq[2]) + (sq[1] + sq[3]);
     else acc = sq[0] + sq[1];
-#pragma unroll
-    for (int st = 32; st > 0; st >>= 1) acc += __shfl_down(acc, st, 64);
-    const float tot = __shfl(acc, 0, 64);
+    const float tot = wave_tree64(acc);
     const float rstd = 1.0f / sqrtf(tot / (float)HD + epi.qk_eps);
 #pragma unroll
     for (uint32_t k = 0; k < EPL; ++k) nv[k] = act_round(xf[k] * rstd * wn[k], epi.act);
@@ -337,38 +335,6 @@ __device__ __forceinline__ void qkv_consumer(const float* partials, uint32_t M, 
     else
       epi.kv_k[crow * epi.row_stride + h * epi.head_stride + e] = act_enc(out, epi.act);
   }
-}
-
-// sum_{g < n} p[g] from +0 in ascending g, p in LDS: the words read 32 / 16 / 4 at a time in
-// 16-byte reads (p 16-byte aligned, n % 4 == 0), so the chain of adds waits on the LDS a few
-// times rather than once per pair of words
-__device__ __forceinline__ float lds_seq_sum(const float* p, uint32_t n) {
-  float tot = 0.f;
-  uint32_t g = 0;
-  const f4_t* p4 = reinterpret_cast<const f4_t*>(p);
-  auto add4 = [&](const f4_t& v) {
-    tot += v[0];
-    tot += v[1];
-    tot += v[2];
-    tot += v[3];
-  };
-  for (; g + 32u <= n; g += 32u) {
-    f4_t v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = p4[g / 4u + j];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) add4(v[j]);
-  }
-  if (g + 16u <= n) {
-    f4_t v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = p4[g / 4u + j];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) add4(v[j]);
-    g += 16u;
-  }
-  for (; g < n; g += 4u) add4(p4[g / 4u]);
-  return tot;
 }
 
 // MR: row capacity (1, 2, 3, 4 or 16); U: k-groups whose loads are issued together; EPI: epilogue;
@@ -635,7 +601,7 @@ __global__ __launch_bounds__(256, (MR == 16 && U == 1 ? 6 : 1)) void gemv_w4a16_
     if (!epi.sums_out) w_pre = epi.next_w[n0 + lane];  // (the split form has no norm weights)
   }
   constexpr int kFoldBuf = fold_buf<MR, EPI>();
-  __shared__ float s_fold[kFoldBuf];
+  __shared__ __align__(16) float s_fold[kFoldBuf];
   const uint32_t t = threadIdx.x;
   {
     // sum_s partials[s][row][n] from 0.f in ascending s, polled in rounds of `per_round`
@@ -683,10 +649,7 @@ __global__ __launch_bounds__(256, (MR == 16 && U == 1 ? 6 : 1)) void gemv_w4a16_
       epi.resid[(size_t)row * N + n0 + lane] = rb;
       const float v = res_widen(rb, epi.act);
       red[1][row][lane] = v;
-      float a = __builtin_fmaf(v, v, 0.f);
-#pragma unroll
-      for (int st = 32; st > 0; st >>= 1) a += __shfl_down(a, st, 64);
-      a = publishable(__shfl(a, 0, 64));
+      const float a = publishable(wave_tree64(__builtin_fmaf(v, v, 0.f)));
       if (epi.sums_out) {  // the next launch forms the norm
         if (lane == 0) epi.sums_out[(size_t)row * ntiles + tile] = a;
         continue;
@@ -709,7 +672,10 @@ __global__ __launch_bounds__(256, (MR == 16 && U == 1 ? 6 : 1)) void gemv_w4a16_
       if (t < nr) {
         const float* ss = s_fold + t * ntiles;
         float tot = 0.f;
-        for (uint32_t g = 0; g < ntiles; ++g) tot += ss[g];
+        if (ntiles % 4u == 0)  // (every row's sums then start on 16 bytes)
+          tot = lds_seq_sum(ss, ntiles);
+        else
+          for (uint32_t g = 0; g < ntiles; ++g) tot += ss[g];
         s_rstd[r0 + t] = 1.0f / sqrtf(tot / (float)N + epi.eps);
       }
       __syncthreads();

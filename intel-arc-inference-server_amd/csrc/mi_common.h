@@ -147,6 +147,57 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
 }
 
+// The 64-lane pairwise tree v[i] += v[i + st], st = 32 .. 1, whose root lands in lane 0, on the vector
+// ALUs: st = 32 and 16 by lane swaps of v with itself (halves, then rows of 16), 8 .. 1 by DPP row
+// shifts. Lane 0 adds exactly the pairs that __shfl_down would give it, without an LDS round trip per
+// step; every lane gets the root.
+__device__ __forceinline__ float wave_tree64(float v) {
+  float a = v, b = v;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  a = a + b;
+  b = a;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  v = a + b;
+  v += dpp_f<0x108>(v);  // row_shl:8, 4, 2, 1: lane i of a row of 16 gets lane i + st
+  v += dpp_f<0x104>(v);
+  v += dpp_f<0x102>(v);
+  v += dpp_f<0x101>(v);
+  return lane_f(v, 0);
+}
+// sum_{g < n} p[g] from +0 in ascending g, p in LDS: the words read 32 / 16 / 4 at a time in
+// 16-byte reads (p 16-byte aligned), so the chain of adds waits on the LDS a few times rather
+// than once per word (80 words: about 3 us as a loop of single reads, under 1 so)
+__device__ __forceinline__ float lds_seq_sum(const float* p, uint32_t n) {
+  float tot = 0.f;
+  uint32_t g = 0;
+  const f4_t* p4 = reinterpret_cast<const f4_t*>(p);
+  auto add4 = [&](const f4_t& v) {
+    tot += v[0];
+    tot += v[1];
+    tot += v[2];
+    tot += v[3];
+  };
+  for (; g + 32u <= n; g += 32u) {
+    f4_t v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = p4[g / 4u + j];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) add4(v[j]);
+  }
+  if (g + 16u <= n) {
+    f4_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = p4[g / 4u + j];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) add4(v[j]);
+    g += 16u;
+  }
+  for (; g + 4u <= n; g += 4u) add4(p4[g / 4u]);
+  for (; g < n; ++g) tot += p[g];
+  return tot;
+}
+
+
 // Orders LDS between the lanes of one wave: lanes that hand data to each other through LDS
 // need it between the writes and the reads (and before the next writes). Without it the
 // compiler may keep a lane's earlier LDS value in a register (another lane's store is a data

@@ -482,21 +482,12 @@ __device__ void down_norm_consumer(const DownNorm& dnm, uint32_t m, uint32_t hid
     rv[u] = 0.f;
     if (c < nch) {
       rv[u] = h2f(sres[c * 64u + lane]);
-      float a = __builtin_fmaf(rv[u], rv[u], 0.f);
-#pragma unroll
-      for (int st = 32; st > 0; st >>= 1) a += __shfl_down(a, st, 64);
+      const float a = wave_tree64(__builtin_fmaf(rv[u], rv[u], 0.f));
       if (lane == 0) s_chunk[c] = a;
     }
   }
   __syncthreads();
-  __shared__ float s_rstd;
-  if (t == 0) {
-    float tot = 0.f;
-    for (uint32_t c = 0; c < nch; ++c) tot += s_chunk[c];
-    s_rstd = 1.0f / sqrtf(tot / (float)hidden + dnm.eps);
-  }
-  __syncthreads();
-  const float r = s_rstd;
+  const float r = 1.0f / sqrtf(lds_seq_sum(s_chunk, nch) / (float)hidden + dnm.eps);
   if (t == 0 && dnm.rstd) dnm.rstd[m] = r;
 #pragma unroll
   for (uint32_t u = 0; u < kCh; ++u) {
@@ -513,7 +504,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const uint32_t* __restric
                                                        uint32_t inter, uint32_t M, DownNorm dnm) {
   extern __shared__ uint32_t s_w[];  // [slots][G][kHalfU32]
   __shared__ __align__(16) float s_h[kMaxSlotsInter / 64 * kXs];
-  __shared__ float s_t[9][8][16];  // [slot][column][group], inter <= 1024
+  __shared__ __align__(16) float s_t[9][8][16];  // [slot][column][group], inter <= 1024
   __shared__ float s_d[9][8];
   if (dnm.x && blockIdx.y == M) {  // the norm row (uniform)
     if (blockIdx.x < M)

@@ -1168,9 +1168,7 @@ __global__ __launch_bounds__(256) void prep_rows_kernel(const float* __restrict_
     float acc;
     if constexpr (EPL == 4) acc = (sq[0] + sq[2]) + (sq[1] + sq[3]);
     else acc = sq[0] + sq[1];
-#pragma unroll
-    for (int st = 32; st > 0; st >>= 1) acc += __shfl_down(acc, st, 64);
-    const float tot = __shfl(acc, 0, 64);
+    const float tot = wave_tree64(acc);
     const float rstd = 1.0f / sqrtf(tot / (float)HD + eps);
 #pragma unroll
     for (uint32_t k = 0; k < EPL; ++k) nv[k] = h2f(f2h(xf[k] * rstd * wn[k]));
