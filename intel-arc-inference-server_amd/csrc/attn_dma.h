@@ -32,11 +32,21 @@
 //           l % 16, dims 8 (l / 16) + 32 kk; int8 widened exactly to f16), B = q in f16 high
 //           and low parts;
 //   softmax per head over the 16 positions, online across the wave's groups (fp32);
-//   P V     O^T = V^T W^T (v_mfma_f32_16x16x16_f16) per 16-dim tile: A = V^T read from LDS
+//   P V     O^T = V^T W^T (v_mfma_f32_16x16x16_f16, two groups: 16x16x32) per 16-dim tile: A = V^T read from LDS
 //           with gfx950's transposing reads - ds_read_b64_tr_b16 gives lane (i, g) dim i of
 //           positions 4 g .. 4 g + 3 (f16); ds_read_b64_tr_b8 gives the same for two tiles at
 //           once (int8, widened exactly to f16) - and B = the weights (int8: times the row's V
 //           scale) in f16 high and low parts.
+// What bounds it: at long contexts HBM, but only while the vector work stays below it: two waves
+// per SIMD issue, per int8 group of 128 dims, 80 instructions to widen K and V alone. So what a
+// step can take from outside its loop it does: a lane's load offsets are formed once, the scales'
+// halves are chosen by two uniform shifts, the masks are formed only in a block's last step (or
+// where rows end), f16 parts take two instructions per value, a tile without rows is skipped,
+// and two int8 groups share one 16x16x32 product per tile for P V. At short ones latency: the row
+// split and the block test divide once, and the merge reads and writes 16 bytes per thread.
+// One row at 131072 int8 keys of 8 heads 59.5 -> 54.7 us (5.0 TB/s), at 40000 23.1 -> 20.5; at 65000
+// f16 keys 56.8 -> 54.2; 16 rows at 30000 int8 keys 77.7 -> 63.9; 4 rows at 4099 f16 keys 15.1 -> 13.0;
+// int8 rows of 256 at 100000 keys of 2 heads 41.4 -> 36.6.
 // Each wave's online softmax takes its groups in ascending order, NG groups per step, and the
 // waves merge in wave order; the results are checked against attn_decode_v2's restatement and
 // fp64 attention.
@@ -89,6 +99,15 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
 
+// two fp32 values as f16 pairs, high and low parts (the remainder v - h is exact in fp32: one fma
+// that reads the f16 value directly, with neg1 = -1, which the compiler may not know to be -1 - it
+// would make the fma a conversion and a subtraction)
+__device__ __forceinline__ void f16_parts(float v0, float v1, float neg1, uint32_t& hi, uint32_t& lo) {
+  const h2_t h = __builtin_convertvector((f2_t{v0, v1}), h2_t);
+  const float l0 = __builtin_fmaf((float)h.x, neg1, v0), l1 = __builtin_fmaf((float)h.y, neg1, v1);
+  hi = h2_bits(h);
+  lo = h2_bits(__builtin_convertvector((f2_t{l0, l1}), h2_t));
+}
 template <uint32_t NB, uint32_t DG>
 __device__ __forceinline__ void wait_group(uint32_t after) {  // after: groups issued after it
   if (after == 0) wait_vm<0>();
@@ -110,16 +129,21 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
   // one (f16 rows of 128 measured faster with one, the ring prefetching the next group); the same
   // for every CT, since the step's rounding depends on it
   constexpr uint32_t NG = HD == 128 && KV8 ? 2u : 1u;
-  // slots per wave: several tiles take the fewest (a multiple of NG) that hold the merge, which
-  // leaves LDS for the tiles' q
+  // QREG: each wave holds the B operands of q itself (one tile: no LDS read of them per group, and
+  // less LDS); else they are staged in LDS once and read per group (two tiles' operands in registers
+  // would leave two work-groups per CU, not three: 4 rows of 40 heads at 4099 keys 12.9 -> 16.9 us)
+  constexpr bool QREG = CT == 1;
+  // slots per wave: several tiles whose q takes LDS have the fewest (a multiple of NG) that hold
+  // the merge
   constexpr uint32_t NBMIN = (RED + 4u * SLOT - 1u) / (4u * SLOT);
-  constexpr uint32_t NB = CT == 1 ? C::NB : (NBMIN + NG - 1u) / NG * NG;
+  constexpr uint32_t NB = QREG ? C::NB : (NBMIN + NG - 1u) / NG * NG;
   constexpr uint32_t RING = 4u * NB * SLOT;
   static_assert(RING >= RED, "merge area");
+  constexpr uint32_t MT = RING >= CT * RED ? CT : 1u;  // tiles merged at once
   __shared__ __align__(16) unsigned char s_ring[RING];
-  __shared__ float st_m[4][16], st_l[4][16], st_f[4][16], st_hm[16], st_hs[16];
+  __shared__ float st_m[4][16 * MT], st_l[4][16 * MT], st_f[4][16 * MT], st_hm[16 * MT], st_hs[16 * MT];
   __shared__ uint32_t s_grow[kMaxBlockGroups];
-  __shared__ h8_t s_q[CT][2][KK][64];
+  __shared__ h8_t s_q[QREG ? 1 : CT][2][QREG ? 1 : KK][QREG ? 1 : 64];
   // FP: the new K/V rows (f16), the roped q of the GQA heads and the waves' normed rows. At
   // rows of 256 the last two live in the ring (LDS is short), which the fused form then starts
   // to load only after its prologue; at rows of 128 they have arrays of their own and the ring's
@@ -145,31 +169,30 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
   // this work-group's rows [r_lo, r_hi): the list's rows split where the block size changes
   // (row b on; the size is non-decreasing in the row and, rounded to 64 positions of
   // ceil(len / tgt), changes at most once over 64 consecutive rows), then RPW at a time
-  uint32_t r_lo, r_hi;
+  uint32_t r_lo, r_hi, s;
   if constexpr (RPW == 1) {
     r_lo = zg;
     r_hi = zg + 1u;
     if (zg >= n_act) return;
   } else {
-    const uint32_t s0 = v2_ppw(row_len(0), a.tgt);
-    uint32_t b = n_act;
-    for (uint32_t r = 1; r < n_act; ++r)
-      if (v2_ppw(row_len(r), a.tgt) != s0) {
-        b = r;
-        break;
-      }
+    // (row r's size is row 0's, s0, while its keys are at most s0 tgt: no division per row)
+    if (n_act == 0) return;
+    s = v2_ppw(row_len(0), a.tgt);
+    const uint64_t cap = (uint64_t)s * a.tgt;
+    const uint32_t b = row_len(n_act - 1u) <= cap ? n_act : (uint32_t)cap - pos;
     const uint32_t za = (b + RPW - 1u) / RPW;
     r_lo = zg < za ? zg * RPW : b + (zg - za) * RPW;
     r_hi = min(r_lo + RPW, zg < za ? b : n_act);
     if (r_lo >= r_hi) return;
+    if (zg >= za) s = v2_ppw(row_len(r_lo), a.tgt);
   }
   const uint32_t m = r_lo;  // the fused prep's row (RPW = 1)
   const uint32_t L = row_len(r_hi - 1u);
-  const uint32_t s = v2_ppw(L, a.tgt);
-  uint32_t nb = (L - 1) / s + 1;
-  if (nb > a.tgt) nb = a.tgt;
-  if (blk >= nb) return;
+  if constexpr (RPW == 1) s = v2_ppw(L, a.tgt);
+  if ((uint64_t)blk * s >= L) return;  // s tgt >= L: at most tgt blocks
   const uint32_t p_begin = blk * s, p_end = min(p_begin + s, L);
+  // every column's row sees the block's positions below pe_all
+  const uint32_t pe_all = min(p_begin + s, row_len(r_lo));
   // this lane's column 16 ct + qi of each tile: its row, and the row's end in the block
   // (p_begin: no column, or the row ends before the block)
   uint32_t crow[CT], pe_col[CT];
@@ -179,6 +202,7 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     crow[ct] = r_lo + c / GQA;
     pe_col[ct] = c < NC && crow[ct] < r_hi ? max(min(p_begin + s, row_len(crow[ct])), p_begin) : p_begin;
   }
+  const uint32_t ncols = (r_hi - r_lo) * GQA;  // the live columns
   const uint32_t ng = (p_end - p_begin + 15u) / 16u;
   const uint32_t ngw = wave < ng ? (ng - wave + 3u) / 4u : 0u;  // this wave's groups
 
@@ -193,6 +217,21 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
   const uint32_t ring_lds = lds_addr(ring);
   auto swz = [](uint32_t r) -> uint32_t { return (r ^ (r >> 3)) & (CPR - 1u); };
 
+  // The lanes' parts of a group's load addresses, formed once: load i's row offset and column
+  // (min(r, glast) rsb = min(r rsb, glast rsb)), and the scale row's offset (rb is a multiple of
+  // 16, so it does not reach the word alignment).
+  uint32_t ro[C::NI], co[C::NI];
+#pragma unroll
+  for (uint32_t i = 0; i < C::NI; ++i) {
+    const uint32_t r = (64u * i + lane) / CPR;
+    ro[i] = r * (uint32_t)rsb;
+    co[i] = 16u * (((64u * i + lane) % CPR) ^ swz(r));
+  }
+  uintptr_t sc_base = 0;
+  const size_t sc_row = (lane & 15u) * a.sc_row_stride;
+  if constexpr (KV8 == 1)
+    sc_base = reinterpret_cast<uintptr_t>(((lane & 16u) ? a.v_scale : a.k_scale) + (size_t)j * a.sc_head_stride);
+
   // issue this wave's group number tw (gi = wave + 4 tw, first cache row rb) into slot tw % NB
   auto issue = [&](uint32_t tw, uint32_t rb) {
     const uint32_t gi = wave + 4u * tw;
@@ -204,17 +243,14 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     lds_reads_done();
 #pragma unroll
     for (uint32_t i = 0; i < C::NI; ++i) {
-      const uint32_t sidx = 64u * i + lane, r = sidx / CPR, c = (sidx % CPR) ^ swz(sidx / CPR);
-      const uint32_t voff = min(r, glast) * (uint32_t)rsb + 16u * c;
+      const uint32_t voff = min(ro[i], glast * (uint32_t)rsb) + co[i];
       dma16(slot + 1024u * i, kg, voff);
       dma16(slot + GB + 1024u * i, vg, voff);
     }
     if constexpr (KV8 == 1) {
-      const uint32_t r = min(lane & 15u, glast);
-      const uint16_t* sb = (lane & 16u) ? a.v_scale : a.k_scale;
-      const size_t e = (size_t)(rb + r) * a.sc_row_stride + (size_t)j * a.sc_head_stride;
-      const uintptr_t ad = reinterpret_cast<uintptr_t>(sb + e) & ~(uintptr_t)3;
-      dma4(slot + 2u * GB, reinterpret_cast<const void*>(ad));
+      const size_t lrow = (lane & 15u) <= glast ? sc_row : glast * a.sc_row_stride;
+      const uintptr_t ad = (sc_base + 2u * lrow) & ~(uintptr_t)3;
+      dma4(slot + 2u * GB, reinterpret_cast<const void*>(ad + 2u * ((size_t)rb * a.sc_row_stride)));
     }
   };
   // The first NB groups, their rows straight from the page table (all its loads first, one wait
@@ -241,12 +277,12 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     }
   };
   if constexpr (kEarly) issue_first();
-  // q of the GQA heads (plain form: wave 0 loads it)
+  // q of the GQA heads (plain form: every wave with QREG, else wave 0)
   f4_t qv[CT][FP ? 1u : 2u * KK];
   if constexpr (!FP) {
 #pragma unroll
     for (uint32_t ct = 0; ct < CT; ++ct)
-      if (wave == 0 && pe_col[ct] > p_begin) {
+      if ((QREG || wave == 0) && pe_col[ct] > p_begin) {
         const float* qp = a.attn_q + ((size_t)crow[ct] * a.q_heads + j * GQA + (16u * ct + qi) % GQA) * HD + 8 * qq;
 #pragma unroll
         for (uint32_t kk = 0; kk < KK; ++kk) {
@@ -389,8 +425,11 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
       a.ctrl_w[CTRL_DEBUG] = 0xDEAD0002u;  // attn_prep's flag: the row's position is past the cache
     lds_barrier();
   }
-  // q as the MFMA B operand (f16 high and low parts), staged by wave 0
-  if (wave == 0) {
+  float neg1 = -1.0f;
+  asm volatile("" : "+v"(neg1));
+  // q as the MFMA B operand (f16 high and low parts), with QREG in registers, else staged by wave 0
+  h8_t qh[QREG ? CT : 1][QREG ? KK : 1], ql[QREG ? CT : 1][QREG ? KK : 1];
+  if (QREG || wave == 0) {
 #pragma unroll
     for (uint32_t ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -409,15 +448,22 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = 0.f;
       }
-      h8_t hi, lo;
+      u4_t hw, lw;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const half_t h = (half_t)v[e];
-        hi[e] = h;
-        lo[e] = (half_t)(v[e] - (float)h);
+      for (int e = 0; e < 4; ++e) {
+        uint32_t h2, l2;
+        f16_parts(v[2 * e], v[2 * e + 1], neg1, h2, l2);
+        hw[e] = h2;
+        lw[e] = l2;
       }
-      s_q[ct][0][kk][lane] = hi;
-      s_q[ct][1][kk][lane] = lo;
+      const h8_t hi = __builtin_bit_cast(h8_t, hw), lo = __builtin_bit_cast(h8_t, lw);
+      if constexpr (QREG) {
+        qh[ct][kk] = hi;
+        ql[ct][kk] = lo;
+      } else {
+        s_q[ct][0][kk][lane] = hi;
+        s_q[ct][1][kk][lane] = lo;
+      }
     }
   }
   wait_vm<0>();   // (the compiler's waits above have seen to this already)
@@ -437,9 +483,15 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
 #pragma unroll
     for (uint32_t tt = 0; tt < NT; ++tt) acc[ct][tt] = f4_t{0.f, 0.f, 0.f, 0.f};
   }
-  // the scales' halves: an element's word half is bit 1 of its address
-  const uint32_t kpar0 = (uint32_t)(((uintptr_t)a.k_scale >> 1) + (size_t)j * a.sc_head_stride);
-  const uint32_t vpar0 = (uint32_t)(((uintptr_t)a.v_scale >> 1) + (size_t)j * a.sc_head_stride);
+  // the scales' halves: an element's word half is bit 1 of its address. A group's first row is a
+  // multiple of 16 and a lane's rows are 4 qq + r, so only r's parity counts: uniform shifts.
+  uint32_t ksh[2], vsh[2];
+#pragma unroll
+  for (uint32_t r = 0; r < 2; ++r) {
+    const uint32_t e = j * (uint32_t)a.sc_head_stride + r * (uint32_t)a.sc_row_stride;
+    ksh[r] = 16u * (((uint32_t)((uintptr_t)a.k_scale >> 1) + e) & 1u);
+    vsh[r] = 16u * (((uint32_t)((uintptr_t)a.v_scale >> 1) + e) & 1u);
+  }
   // the max over the four lanes l % 16 + 16 k that hold one head's scores: v_permlane16_swap
   // and v_permlane32_swap of x with a copy of itself leave rows (0, 0, 2, 2) / (1, 1, 3, 3) and
   // halves (lo, lo) / (hi, hi) in the two registers (VALU, no LDS round trip). Written as
@@ -452,6 +504,7 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     return fmaxf(b0, b1);
   };
   static_assert(NB % NG == 0, "ring");
+  typedef float f4a_t __attribute__((ext_vector_type(4), aligned(4)));
   typedef int v2i_t __attribute__((ext_vector_type(2)));
   typedef short v4s_t __attribute__((ext_vector_type(4)));
   constexpr uint32_t NTR = KV8 ? NT / 2 : NT;  // transposing reads per group
@@ -540,26 +593,28 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
         vw[u][0] = v4.x; vw[u][1] = v4.y; vw[u][2] = v4.z; vw[u][3] = v4.w;
       }
     }
+    // whether every row sees all of the step's positions: no masks then (columns that hold no
+    // row form values that nothing reads)
+    const bool full = (NG == 1 || has1) && p0g[NG - 1] + 16u <= pe_all;
     // the int8 rows' score and V scales (shared by the tiles)
     float rsc[NG][4], vsv[NG][4];
 #pragma unroll
-    for (uint32_t u = 0; u < NG; ++u) {
-      uint32_t rb = 0;
-      if constexpr (KV8 == 1) rb = group_row(wave + 4u * (u && has1 ? tw + 1 : tw));
+    for (uint32_t u = 0; u < NG; ++u)
 #pragma unroll
       for (uint32_t r = 0; r < 4; ++r) {
         rsc[u][r] = qscale;
         vsv[u][r] = 1.0f;
         if constexpr (KV8 == 1) {
-          const uint32_t rr = glen[u] ? min(4u * qq + r, glen[u] - 1u) : 0u;
-          const uint32_t er = (uint32_t)((size_t)(rb + rr) * a.sc_row_stride);
-          rsc[u][r] = qscale * h2f((uint16_t)(((er + kpar0) & 1u) ? kw[u][r] >> 16 : kw[u][r] & 0xFFFFu));
-          vsv[u][r] = h2f((uint16_t)(((er + vpar0) & 1u) ? vw[u][r] >> 16 : vw[u][r] & 0xFFFFu));
+          rsc[u][r] = qscale * h2f((uint16_t)(kw[u][r] >> ksh[r & 1u]));
+          vsv[u][r] = h2f((uint16_t)(vw[u][r] >> vsh[r & 1u]));
+          // (a row past the group's end holds its last row's word, whose other half is no scale of
+          // this head: its weight is 0, so any finite scale will do; its score is masked)
+          if (!full) vsv[u][r] = 4u * qq + r < glen[u] ? vsv[u][r] : 0.f;
         }
       }
-    }
 #pragma unroll
     for (uint32_t ct = 0; ct < CT; ++ct) {
+      if (16u * ct >= ncols) break;  // uniform: no row in this tile
       // scores S^T[position 4 qq + r][column 16 ct + qi]: the f16 high and low parts of q on
       // two chains
       f4_t dh[NG], dl[NG];
@@ -570,30 +625,46 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
 #pragma unroll
         for (uint32_t u = 0; u < NG; ++u) {
           const h8_t k8 = KV8 ? chunk_h8<1>(kc[u][kk]) : kh[u][kk];
-          dh[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, s_q[ct][0][kk][lane], dh[u], 0, 0, 0);
-          dl[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, s_q[ct][1][kk][lane], dl[u], 0, 0, 0);
+          h8_t b0, b1;
+          if constexpr (QREG) {
+            b0 = qh[ct][kk];
+            b1 = ql[ct][kk];
+          } else {
+            b0 = s_q[ct][0][kk][lane];
+            b1 = s_q[ct][1][kk][lane];
+          }
+          dh[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, b0, dh[u], 0, 0, 0);
+          dl[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, b1, dl[u], 0, 0, 0);
         }
       float sc[NG][4];
+#pragma unroll
+      for (uint32_t u = 0; u < NG; ++u)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) sc[u][r] = (dh[u][r] + dl[u][r]) * rsc[u][r];
+      bool colive = true;  // a column none of whose positions are in these groups keeps its state
+      if (!full) {
+        colive = p0g[0] < pe_col[ct];
+#pragma unroll
+        for (uint32_t u = 0; u < NG; ++u)
+#pragma unroll
+          for (uint32_t r = 0; r < 4; ++r)
+            sc[u][r] = 4u * qq + r < glen[u] && p0g[u] + 4u * qq + r < pe_col[ct] ? sc[u][r] : -INFINITY;
+      }
       float mx = -INFINITY;
 #pragma unroll
       for (uint32_t u = 0; u < NG; ++u)
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) {
-          sc[u][r] = 4u * qq + r < glen[u] && p0g[u] + 4u * qq + r < pe_col[ct] ? (dh[u][r] + dl[u][r]) * rsc[u][r]
-                                                                                : -INFINITY;
-          mx = fmaxf(mx, sc[u][r]);
-        }
+        for (uint32_t r = 0; r < 4; ++r) mx = fmaxf(mx, sc[u][r]);
       mx = head_max(mx);
-      // a column none of whose positions are in these groups keeps its state
-      const bool colive = p0g[0] < pe_col[ct];
       const float m_new = colive ? fmaxf(m_run[ct], mx) : m_run[ct];
+      const float m_sub = colive ? m_new : 0.f;  // a column that keeps its state: weights exp2(-inf) = 0
       const float alpha = colive ? __builtin_amdgcn_exp2f(m_run[ct] - m_new) : 1.0f;  // 0 on the first group
       float w[NG][4];
       float wsum = 0.f;
 #pragma unroll
       for (uint32_t u = 0; u < NG; ++u) {
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) w[u][r] = colive ? __builtin_amdgcn_exp2f(sc[u][r] - m_new) : 0.f;
+        for (uint32_t r = 0; r < 4; ++r) w[u][r] = __builtin_amdgcn_exp2f(sc[u][r] - m_sub);
         wsum += (w[u][0] + w[u][1]) + (w[u][2] + w[u][3]);
       }
       l_run[ct] = __builtin_fmaf(l_run[ct], alpha, wsum);
@@ -602,38 +673,53 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
 #pragma unroll
         for (uint32_t tt = 0; tt < NT; ++tt) acc[ct][tt] *= alpha;
       }
-      // B operands: the weights (int8: times the row's V scale), f16 high and low parts
-      h4_t bh[NG], bl[NG];
+      // B operands: the weights (int8: times the row's V scale), f16 high and low parts (the
+      // remainder is exact in fp32)
+      uint32_t bh[NG][2], bl[NG][2];
 #pragma unroll
       for (uint32_t u = 0; u < NG; ++u)
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) {
-          const float wv = w[u][r] * vsv[u][r];
-          const half_t h = (half_t)wv;
-          bh[u][r] = h;
-          bl[u][r] = (half_t)(wv - (float)h);
+        for (uint32_t r = 0; r < 4; r += 2) {
+          float v0 = w[u][r] * vsv[u][r], v1 = w[u][r + 1] * vsv[u][r + 1];
+          asm("" : "+v"(v0), "+v"(v1));  // rounded to fp32 first
+          f16_parts(v0, v1, neg1, bh[u][r / 2], bl[u][r / 2]);
         }
-      // P V per 16-dim tile
+      // P V per 16-dim tile. Two groups per step: one product over their 32 positions (lane (i, g)
+      // holds positions 4 g .. 4 g + 3 of the first, then of the second)
+      if constexpr (KV8 == 0) {
+        const h4_t wh = __builtin_bit_cast(h4_t, (u2_t{bh[0][0], bh[0][1]}));
+        const h4_t wl = __builtin_bit_cast(h4_t, (u2_t{bl[0][0], bl[0][1]}));
+        static_assert(KV8 == 1 || NG == 1, "f16 rows: one group per step");
 #pragma unroll
-      for (uint32_t i = 0; i < NTR; ++i) {
+        for (uint32_t i = 0; i < NTR; ++i) {
+          acc[ct][i] = __builtin_amdgcn_mfma_f32_16x16x16f16(av[0][i], wh, acc[ct][i], 0, 0, 0);
+          acc[ct][i] = __builtin_amdgcn_mfma_f32_16x16x16f16(av[0][i], wl, acc[ct][i], 0, 0, 0);
+        }
+      } else {
 #pragma unroll
-        for (uint32_t u = 0; u < NG; ++u) {
-          if constexpr (KV8 == 0) {
-            acc[ct][i] = __builtin_amdgcn_mfma_f32_16x16x16f16(av[u][i], bh[u], acc[ct][i], 0, 0, 0);
-            acc[ct][i] = __builtin_amdgcn_mfma_f32_16x16x16f16(av[u][i], bl[u], acc[ct][i], 0, 0, 0);
+        for (uint32_t i = 0; i < NTR; ++i) {
+          h8_t vt[NG];  // the group's two tiles' V^T
+#pragma unroll
+          for (uint32_t u = 0; u < NG; ++u) vt[u] = chunk_h8<1>({u2_t{(uint32_t)raw[u][i].x, (uint32_t)raw[u][i].y}});
+          if constexpr (NG == 2) {
+            const h8_t wh = __builtin_bit_cast(h8_t, (u4_t{bh[0][0], bh[0][1], bh[1][0], bh[1][1]}));
+            const h8_t wl = __builtin_bit_cast(h8_t, (u4_t{bl[0][0], bl[0][1], bl[1][0], bl[1][1]}));
+#pragma unroll
+            for (uint32_t e = 0; e < 2; ++e) {
+              const h8_t av8 = e == 0 ? __builtin_shufflevector(vt[0], vt[NG - 1], 0, 1, 2, 3, 8, 9, 10, 11)
+                                      : __builtin_shufflevector(vt[0], vt[NG - 1], 4, 5, 6, 7, 12, 13, 14, 15);
+              acc[ct][2 * i + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av8, wh, acc[ct][2 * i + e], 0, 0, 0);
+              acc[ct][2 * i + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av8, wl, acc[ct][2 * i + e], 0, 0, 0);
+            }
           } else {
-            const h2_t bias = {(half_t)1152.0f, (half_t)1152.0f};
-            const uint32_t x0 = (uint32_t)raw[u][i].x ^ 0x80808080u, x1 = (uint32_t)raw[u][i].y ^ 0x80808080u;
-            const uint32_t hi = 0x64646464u;
-            const h2_t p0 = as_h2(__builtin_amdgcn_perm(hi, x0, 0x04010400u)) - bias;
-            const h2_t p1 = as_h2(__builtin_amdgcn_perm(hi, x0, 0x04030402u)) - bias;
-            const h2_t p2 = as_h2(__builtin_amdgcn_perm(hi, x1, 0x04010400u)) - bias;
-            const h2_t p3 = as_h2(__builtin_amdgcn_perm(hi, x1, 0x04030402u)) - bias;
-            const h4_t a0 = h4_t{p0[0], p0[1], p1[0], p1[1]}, a1 = h4_t{p2[0], p2[1], p3[0], p3[1]};
-            acc[ct][2 * i] = __builtin_amdgcn_mfma_f32_16x16x16f16(a0, bh[u], acc[ct][2 * i], 0, 0, 0);
-            acc[ct][2 * i] = __builtin_amdgcn_mfma_f32_16x16x16f16(a0, bl[u], acc[ct][2 * i], 0, 0, 0);
-            acc[ct][2 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1, bh[u], acc[ct][2 * i + 1], 0, 0, 0);
-            acc[ct][2 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1, bl[u], acc[ct][2 * i + 1], 0, 0, 0);
+            const h4_t wh = __builtin_bit_cast(h4_t, (u2_t{bh[0][0], bh[0][1]}));
+            const h4_t wl = __builtin_bit_cast(h4_t, (u2_t{bl[0][0], bl[0][1]}));
+            const h4_t a0 = __builtin_shufflevector(vt[0], vt[0], 0, 1, 2, 3);
+            const h4_t a1 = __builtin_shufflevector(vt[0], vt[0], 4, 5, 6, 7);
+            acc[ct][2 * i] = __builtin_amdgcn_mfma_f32_16x16x16f16(a0, wh, acc[ct][2 * i], 0, 0, 0);
+            acc[ct][2 * i] = __builtin_amdgcn_mfma_f32_16x16x16f16(a0, wl, acc[ct][2 * i], 0, 0, 0);
+            acc[ct][2 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1, wh, acc[ct][2 * i + 1], 0, 0, 0);
+            acc[ct][2 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1, wl, acc[ct][2 * i + 1], 0, 0, 0);
           }
         }
       }
@@ -645,27 +731,29 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
   }
   wait_vm<0>();
   lds_barrier();  // every wave is done with its ring, which the merge reuses
-  // merge the four waves per tile of columns: M = max m_w, f_w = exp(m_w - M), sum and acc
-  // weighted by f_w in wave order (the state's max in natural units: max * ln 2)
-  float* red = reinterpret_cast<float*>(s_ring);  // [4][16][HD]
-  const uint32_t ncols = (r_hi - r_lo) * GQA;      // the live columns
+  // merge the four waves, MT tiles of columns at a time: M = max m_w, f_w = exp(m_w - M), sum and
+  // acc weighted by f_w in wave order (the state's max in natural units: max * ln 2)
+  float* red = reinterpret_cast<float*>(s_ring);  // [4][16 MT][HD]
 #pragma unroll
-  for (uint32_t ct = 0; ct < CT; ++ct) {
-    const uint32_t nlc = ncols > 16u * ct ? min(ncols - 16u * ct, 16u) : 0u;  // this tile's
+  for (uint32_t ct0 = 0; ct0 < CT; ct0 += MT) {
+    const uint32_t nlc = ncols > 16u * ct0 ? min(ncols - 16u * ct0, 16u * MT) : 0u;  // these tiles'
     if (nlc == 0) break;  // uniform
-    if (ct) lds_barrier();  // the previous tile's merge is done with red and the st arrays
-    const float mr = m_run[ct] * 0.6931471805599453f;
-    float l = l_run[ct] + __shfl_xor(l_run[ct], 16, 64);
-    l = l + __shfl_xor(l, 32, 64);
-    if (qq == 0) {
-      st_m[wave][qi] = mr;
-      st_l[wave][qi] = l;
-    }
-    if (qi < nlc) {
+    if (ct0) lds_barrier();  // the previous merge is done with red and the st arrays
 #pragma unroll
-      for (uint32_t tt = 0; tt < NT; ++tt)
+    for (uint32_t c1 = 0; c1 < MT; ++c1) {
+      const uint32_t ct = ct0 + c1, col = 16u * c1 + qi;
+      const float mr = m_run[ct] * 0.6931471805599453f;
+      float l = l_run[ct] + __shfl_xor(l_run[ct], 16, 64);
+      l = l + __shfl_xor(l, 32, 64);
+      if (qq == 0) {
+        st_m[wave][col] = mr;
+        st_l[wave][col] = l;
+      }
+      if (col < nlc) {
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) red[(wave * 16u + qi) * HD + 16u * tt + 4u * qq + r] = acc[ct][tt][r];
+        for (uint32_t tt = 0; tt < NT; ++tt)
+          *reinterpret_cast<f4_t*>(red + (wave * 16u * MT + col) * HD + 16u * tt + 4u * qq) = acc[ct][tt];
+      }
     }
     lds_barrier();
     if (t < nlc) {
@@ -683,15 +771,21 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
       st_hs[t] = sm;
     }
     lds_barrier();
-    for (uint32_t idx = t; idx < nlc * HD; idx += 256u) {
-      const uint32_t g = idx / HD, dd = idx % HD, c = 16u * ct + g, row = r_lo + c / GQA;
+    // four dims per thread
+    for (uint32_t idx = t; idx < nlc * (HD / 4u); idx += 256u) {
+      const uint32_t g = idx / (HD / 4u), dd = 4u * (idx % (HD / 4u)), c = 16u * ct0 + g, row = r_lo + c / GQA;
       // a row whose keys end before this block has no partial here
       if (blk * s >= row_len(row)) continue;
-      float v = 0.f;
+      f4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (uint32_t w2 = 0; w2 < 4; ++w2) v = __builtin_fmaf(red[(w2 * 16u + g) * HD + dd], st_f[w2][g], v);
+      for (uint32_t w2 = 0; w2 < 4; ++w2) {
+        const f4_t x = *reinterpret_cast<const f4_t*>(red + (w2 * 16u * MT + g) * HD + dd);
+        const float f = st_f[w2][g];
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) v[e] = __builtin_fmaf(x[e], f, v[e]);
+      }
       float* out = a.attn_part + (((size_t)(j * GQA + c % GQA) * a.tgt + blk) * a.M + row) * (HD + 2);
-      *as_global(out + 2 + dd) = v;
+      *as_global(reinterpret_cast<f4a_t*>(out + 2 + dd)) = v;
       if (dd == 0) {
         out[0] = st_hm[g];
         out[1] = st_hs[g];

@@ -106,6 +106,36 @@ def test_decode_every_gqa_and_block_length(QH, KVH, HD, Lm, tgt, pos):
     check_close(got[0].reshape(QH, HD), want)
 
 
+@pytest.mark.parametrize("KVH,HD", [(3, 128), (2, 128), (3, 256)])
+@pytest.mark.parametrize("M,pos", [(1, 0), (1, 16), (3, 29), (4, 62), (7, 250), (2, 1000)])
+def test_scales_by_row_and_head_at_any_parity(KVH, HD, M, pos):
+    """int8 scales stored [row][head] from a base that is not word aligned (odd and even strides: a
+    4-byte load holds another head's or the next row's scale in its other half), NaN in every row the
+    step does not see: the bits of the [head][row] layout. The lists end inside a group, a step of two
+    groups and a block, and cross a change of the block size."""
+    QH, Lm, tgt = 5 * KVH, 1088, 4
+    sh = O.attn_shape(QH, KVH, HD)
+    k, v, ks, vs = make_kv(1, KVH, Lm, HD, pos + HD)
+    q = np.random.default_rng(pos).standard_normal((M, QH, HD)).astype(np.float32)
+    want, pw = gpu_attention(sh, q, 1, k, v, ks, vs, pos, M, tgt)
+    nan = np.uint16(0x7E00)
+
+    def interleave(s):
+        w = np.full(1 + Lm * KVH, nan, np.uint16)
+        w[1:].reshape(Lm, KVH)[:pos + M] = s[:, :pos + M].T
+        return dev(w)
+
+    ctrl, part = ctrl_dev(pos, M), empty((QH, tgt, M, HD + 2), np.float32)
+    out = dev(np.full((M, QH * HD), 0xFFFF, np.uint16))
+    dk, dv, dq, dks, dvs = dev(k), dev(v), dev(q), interleave(ks), interleave(vs)
+    shp = mi.shape_ref(sh)
+    mi.call("mi_attn_decode", ptr(ctrl), ptr(dq), 1, ptr(dk), ptr(dv), ptr(dks) + 2, ptr(dvs) + 2, HD, Lm * HD,
+            KVH, 1, None, 0, Lm, ptr(part), M, tgt, shp, stream())
+    mi.call("mi_attn_reduce", ptr(ctrl), ptr(part), None, ptr(out), M, tgt, Lm, shp, stream())
+    sync()
+    assert np.array_equal(host(out, np.uint16), want)
+
+
 @pytest.mark.parametrize("kind", [0, 1])
 def test_long_context_paged_bitwise(kind):
     """BASELINE config 3 shape (40 q / 8 kv, hd 128) at L = 32768, 64-token pages in a
