@@ -178,12 +178,12 @@ __device__ void route_compute(const float* lg, uint32_t* s_row, uint32_t E, uint
     const auto fmax_op = [](float a, float b) { return fmaxf(a, b); };
     const auto add_op = [](float a, float b) { return a + b; };
     const float mloc = levels(v[0], v[1], v[2], v[3], fmax_op);
-    const float mx = __shfl(wave_tree(lane < n0 ? mloc : -INFINITY, n0, fmax_op), 0, 64);
+    const float mx = n0 == 64u ? wave_max(mloc) : __shfl(wave_tree(lane < n0 ? mloc : -INFINITY, n0, fmax_op), 0, 64);
     float ex[4];
 #pragma unroll
     for (uint32_t u = 0; u < 4; ++u) ex[u] = lane + 64u * u < E ? expf(v[u] - mx) : 0.f;
     const float sloc = levels(ex[0], ex[1], ex[2], ex[3], add_op);
-    const float sum = __shfl(wave_tree(lane < n0 ? sloc : 0.f, n0, add_op), 0, 64);
+    const float sum = n0 == 64u ? wave_tree64(sloc) : __shfl(wave_tree(lane < n0 ? sloc : 0.f, n0, add_op), 0, 64);
 #pragma unroll
     for (uint32_t u = 0; u < 4; ++u) {
       const uint32_t j = lane + 64u * u;
@@ -271,62 +271,74 @@ __device__ __forceinline__ u4_t half_piece(const uint32_t* tile, uint32_t ch, ui
   return load_stream16(tile + off);
 }
 
-// LDS floats per 64-element group of a staged activation row: 4 of padding, so the groups
-// that the lanes of one wave read together start in different banks
-constexpr uint32_t kXs = 68;
+// A layout-1 row is 64 contiguous bytes, half of which is each half tile's: the two work-groups
+// of a tile are 8 apart in the grid, so the same XCD's L2 serves both. i: the work-group's index
+// over a multiple of 16 half tiles.
+__device__ __forceinline__ void half_of(uint32_t i, uint32_t& tile, uint32_t& ch) {
+  tile = i / 16u * 8u + i % 8u;
+  ch = i / 8u % 2u;
+}
 
-// dst[g * kXs + k % 64] = h2f(src[k]) for k < n, g = k / 64 (n a multiple of 8, src 16-byte
-// aligned), from u4_t pieces already loaded: v[u] holds piece threadIdx.x + 256 u
-template <int PER>
-__device__ __forceinline__ void put_f16(float* dst, const u4_t (&v)[PER], uint32_t n) {
+// f16 words in LDS per 64-element group of a staged activation row: 8 of padding, so the groups
+// that the lanes of one wave read together start in different banks
+constexpr uint32_t kXs = 72;
+
+// dst[g * kXs + k % 64] = src[k] for k < n, g = k / 64 (n a multiple of 8, src 16-byte
+// aligned), from u4_t pieces already loaded: v[u] holds piece threadIdx.x + NT u
+template <int PER, uint32_t NT>
+__device__ __forceinline__ void put_f16(uint16_t* dst, const u4_t (&v)[PER], uint32_t n) {
   const uint32_t n8 = n / 8u;
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const uint32_t i = threadIdx.x + 256u * u;
-    if (i < n8) {
-      const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-      float* d = dst + (i / 8u) * kXs + (i % 8u) * 8u;
-#pragma unroll
-      for (uint32_t j = 0; j < 8; ++j) d[j] = h2f((uint16_t)(w[j / 2] >> (16 * (j % 2))));
-    }
+    const uint32_t i = threadIdx.x + NT * u;
+    if (i < n8) *reinterpret_cast<u4_t*>(dst + (i / 8u) * kXs + (i % 8u) * 8u) = v[u];
   }
 }
 // (every load unconditional, pieces past n re-reading the last: a load under a branch leaves
 // its value in a register that the branch's join copies, and the copy waits for it at once)
-template <int PER>
+template <int PER, uint32_t NT>
 __device__ __forceinline__ void get_f16(u4_t (&v)[PER], const uint16_t* src, uint32_t n) {
   const uint32_t n8 = n / 8u;
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const uint32_t i = min(threadIdx.x + 256u * u, n8 - 1u);
+    const uint32_t i = min(threadIdx.x + NT * u, n8 - 1u);
     v[u] = *reinterpret_cast<const u4_t*>(src + 8u * i);
   }
 }
 
 // One k-group's dot for column c < 8 of a staged half tile (moe_ref.h:98-116's tile_dot body):
 // sum over words j of (sum over nibbles i of (q - 8) * x) in ascending order, then * scale;
-// xs: the group's 64 activations (16-byte aligned), read four at a time
-__device__ __forceinline__ float half_term(const uint32_t* ht, uint32_t c, const float* __restrict__ xs) {
+// xs: the group's 64 activations in f16 (16-byte aligned), read eight at a time. The nibbles
+// become f16 pairs (bits under an exponent of 1024, minus 1032) and a product of two f16 values
+// is exact in fp32, so one fma per product is the multiply and the add: 2.5 instructions per
+// weight for five (extract, subtract, convert, multiply, add), and half the LDS reads of x. A
+// token's launches are latency and these instructions, not bytes (256 experts, top 8, 2048 x 512:
+// gate||up 12.2 -> 9.9 us, down + norm 12.0 -> 9.9 with its wider work-groups; 8 rows' block 108 -> 90).
+__device__ __forceinline__ float half_term(const uint32_t* ht, uint32_t c, const uint16_t* __restrict__ xs) {
   uint32_t wd[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) wd[j] = ht[j * 8 + c];
   const uint16_t sc = reinterpret_cast<const uint16_t*>(ht + 64)[c];
-  const f4_t* x4 = reinterpret_cast<const f4_t*>(xs);
+  const u4_t* x8 = reinterpret_cast<const u4_t*>(xs);
+  const h2_t bias = {(half_t)1032.0f, (half_t)1032.0f};
   float g = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const f4_t lo = x4[2 * j], hi = x4[2 * j + 1];
-    const float xv[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    const u4_t xw = x8[j];
+    const h2_t xp[4] = {as_h2(xw.x), as_h2(xw.y), as_h2(xw.z), as_h2(xw.w)};
+    h2_t q[4];  // nibbles i and i + 4
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = as_h2(((wd[j] >> (4 * i)) & 0x000F000Fu) | 0x64006400u) - bias;
     float a = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) a += (float)((int)((wd[j] >> (4 * i)) & 0xFu) - 8) * xv[i];
+    for (int i = 0; i < 8; ++i) a = __builtin_fmaf((float)q[i & 3][i >> 2], (float)xp[i / 2][i & 1], a);
     g += a;
   }
   return g * h2f(sc);
 }
 
 // ---- gate||up + SiLU (moe.cl:335-381; twin moe_ref.h:154-168) ------------------------------
-// grid (slots * inter/8, M): work-group (slot, ib, ch) makes h[m][slot][16 ib + 8 ch .. + 7]
+// grid (slots * inter/8, M): work-group (slot, half_of's (ib, ch)) makes h[m][slot][16 ib + 8 ch .. + 7]
 // from half ch of the expert's gate tile 2 ib and up tile 2 ib + 1 (interleave16 columns).
 // Dynamic LDS: 2 G staged half tiles.
 // ROUTED: the work-group forms its row's route row itself from the router logits (every
@@ -343,16 +355,18 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(uint32_t* __restrict__
                                                           uint32_t top_k, uint32_t hidden,
                                                           uint32_t inter) {
   extern __shared__ uint32_t s_w[];  // [2][G][kHalfU32]
-  __shared__ __align__(16) float s_x[kMaxHidden / 64 * kXs];
+  __shared__ __align__(16) uint16_t s_x[kMaxHidden / 64 * kXs];
   __shared__ float s_t[2][8][kMaxGroups];
   __shared__ float s_r[2][8][kUpKs];
   __shared__ uint32_t s_row[ROUTED ? kRouteWords : 1];
   const uint32_t t = threadIdx.x, m = blockIdx.y;
-  const uint32_t nhb = inter / 8, slot = blockIdx.x / nhb, hb = blockIdx.x % nhb, ib = hb / 2, ch = hb % 2;
+  const uint32_t nhb = inter / 8, slot = blockIdx.x / nhb;
+  uint32_t ib, ch;
+  half_of(blockIdx.x % nhb, ib, ch);
   const uint32_t G = hidden / 64, slots = top_k + 1;
   constexpr int XP = kMaxHidden / 8 / 256;  // x pieces per thread
   u4_t xv[XP];
-  get_f16<XP>(xv, x + (size_t)m * hidden, hidden);
+  get_f16<XP, 256>(xv, x + (size_t)m * hidden, hidden);
   uint32_t e;
   if constexpr (ROUTED) {
     route_compute(logits + (size_t)m * router_n, s_row, E, top_k);
@@ -375,7 +389,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(uint32_t* __restrict__
         v[u] = half_piece(base + (size_t)tg * kTileU32, ch, k);
       }
     }
-    put_f16<XP>(s_x, xv, hidden);
+    put_f16<XP, 256>(s_x, xv, hidden);
 #pragma unroll
     for (uint32_t u = 0; u < kBatch; ++u) {
       const uint32_t i = t + 256u * u;
@@ -413,7 +427,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(uint32_t* __restrict__
 }
 
 // ---- down + combine + residual (moe.cl:383-470; twin moe_ref.h:140-177) ---------------------
-// grid (hidden/8, M): work-group (nb, ch) makes resid[m][16 nb + 8 ch .. + 7] from half ch of
+// grid (hidden/8, M): work-group half_of's (nb, ch) makes resid[m][16 nb + 8 ch .. + 7] from half ch of
 // every slot's down tile nb, combined in slot order. Dynamic LDS: slots * G staged half tiles.
 // The next RMSNorm in the same launch (DownNorm::x non-NULL): the grid has one more row of
 // work-groups, after every producer; work-group m of it is row m's norm. Each producer also
@@ -496,22 +510,28 @@ __device__ void down_norm_consumer(const DownNorm& dnm, uint32_t m, uint32_t hid
   }
 }
 
-__global__ __launch_bounds__(256) void moe_down_kernel(const uint32_t* __restrict__ route,
+// NT threads: 640 where there are more than 256 (slot, group, column) terms, which they make in
+// one turn up to 640 (9 slots of 512: 576) - a decode step has few work-groups per CU, so each
+// needs its own waves - else 256.
+template <uint32_t NT>
+__global__ __launch_bounds__(NT) void moe_down_kernel(const uint32_t* __restrict__ route,
                                                        const uint16_t* __restrict__ h,
                                                        const uint32_t* __restrict__ dn,
                                                        uint16_t* __restrict__ resid, uint32_t E,
                                                        uint32_t top_k, uint32_t hidden,
                                                        uint32_t inter, uint32_t M, DownNorm dnm) {
   extern __shared__ uint32_t s_w[];  // [slots][G][kHalfU32]
-  __shared__ __align__(16) float s_h[kMaxSlotsInter / 64 * kXs];
+  __shared__ __align__(16) uint16_t s_h[kMaxSlotsInter / 64 * kXs];
   __shared__ __align__(16) float s_t[9][8][16];  // [slot][column][group], inter <= 1024
   __shared__ float s_d[9][8];
-  if (dnm.x && blockIdx.y == M) {  // the norm row (uniform)
-    if (blockIdx.x < M)
+  if (dnm.x && blockIdx.y == M) {  // the norm row (uniform; its work-groups' first 256 threads)
+    if (blockIdx.x < M && threadIdx.x < 256u)
       down_norm_consumer(dnm, blockIdx.x, hidden, reinterpret_cast<uint32_t*>(s_h), &s_t[0][0][0]);
     return;
   }
-  const uint32_t t = threadIdx.x, m = blockIdx.y, nb = blockIdx.x / 2, ch = blockIdx.x % 2;
+  const uint32_t t = threadIdx.x, m = blockIdx.y;
+  uint32_t nb, ch;
+  half_of(blockIdx.x, nb, ch);
   const uint32_t G = inter / 64, slots = top_k + 1;
   const uint32_t* row = route + (size_t)m * kRouteWords;
   uint32_t ids[9];
@@ -525,17 +545,17 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const uint32_t* __restric
   const float sg = __builtin_bit_cast(float, row[R_SG]);
   uint16_t* rp = resid + (size_t)m * hidden + nb * 16 + ch * 8 + (t & 7u);
   const uint16_t r_old = *rp;  // (every lane: lanes 8.. read lane t % 8's element, unused)
-  constexpr int HP = kMaxSlotsInter / 8 / 256 + 1;  // h pieces per thread (<= 1152 pieces)
+  constexpr int HP = (kMaxSlotsInter / 8 + NT - 1) / NT;  // h pieces per thread (<= 1152 pieces)
   u4_t hv[HP];
-  get_f16<HP>(hv, h + (size_t)m * slots * inter, slots * inter);
+  get_f16<HP, NT>(hv, h + (size_t)m * slots * inter, slots * inter);
   {
     const size_t block = (size_t)(hidden / 16) * G * kTileU32;
     const uint32_t n4 = slots * G * kHalfU4;  // pieces: (slot, group g, piece k)
-    constexpr uint32_t kBatch = 10;           // 9 * 16 * 17 = 2448 pieces (inter <= 1024)
+    constexpr uint32_t kBatch = (2448 + NT - 1) / NT;  // 9 * 16 * 17 = 2448 pieces (inter <= 1024)
     u4_t v[kBatch];
 #pragma unroll
     for (uint32_t u = 0; u < kBatch; ++u) {
-      const uint32_t i = t + 256u * u;
+      const uint32_t i = t + NT * u;
       if (i < n4) {
         const uint32_t sg = i / kHalfU4, k = i - sg * kHalfU4, sl = sg / G, g = sg - sl * G;
         uint32_t eid = ids[0];
@@ -544,16 +564,16 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const uint32_t* __restric
         v[u] = half_piece(dn + (size_t)eid * block + ((size_t)nb * G + g) * kTileU32, ch, k);
       }
     }
-    put_f16<HP>(s_h, hv, slots * inter);
+    put_f16<HP, NT>(s_h, hv, slots * inter);
 #pragma unroll
     for (uint32_t u = 0; u < kBatch; ++u) {
-      const uint32_t i = t + 256u * u;
+      const uint32_t i = t + NT * u;
       if (i < n4) reinterpret_cast<u4_t*>(s_w)[i] = v[u];
     }
   }
   __syncthreads();
   const uint32_t tasks = slots * 8u * G;
-  for (uint32_t i = t; i < tasks; i += 256u) {
+  for (uint32_t i = t; i < tasks; i += NT) {
     const uint32_t slot = i / (8u * G), rem = i % (8u * G), g = rem / 8u, c = rem % 8u;
     s_t[slot][c][g] = half_term(s_w + ((size_t)slot * G + g) * kHalfU32, c, s_h + (slot * G + g) * kXs);
   }
@@ -588,6 +608,9 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const uint32_t* __restric
     }
   }
 }
+
+// moe_down_kernel's threads for its terms
+bool down_wide(uint32_t top_k, uint32_t inter) { return (top_k + 1) * (inter / 64) * 8 > 256; }
 
 int check_moe(uint32_t M, uint32_t E, uint32_t top_k, uint32_t hidden, uint32_t inter) {
   if (M == 0 || M > 16) return mi_fail(MI_ERR_SHAPE, "moe: M must be 1..16");
@@ -672,8 +695,12 @@ extern "C" int mi_moe_down(const uint32_t* route, const uint16_t* h, const uint3
   if (reinterpret_cast<uintptr_t>(dn_blocks) % 16 || reinterpret_cast<uintptr_t>(h) % 16)
     return mi_fail(MI_ERR_ARG, "moe_down: dn_blocks and h need 16-byte alignment");
   const size_t lds = size_t(top_k + 1) * (inter / 64) * kHalfU32 * 4;
-  moe_down_kernel<<<dim3(hidden / 8, M), 256, lds, static_cast<hipStream_t>(stream)>>>(
-      route, h, dn_blocks, resid, experts, top_k, hidden, inter, M, DownNorm{});
+  if (down_wide(top_k, inter))
+    moe_down_kernel<640><<<dim3(hidden / 8, M), 640, lds, static_cast<hipStream_t>(stream)>>>(
+        route, h, dn_blocks, resid, experts, top_k, hidden, inter, M, DownNorm{});
+  else
+    moe_down_kernel<256><<<dim3(hidden / 8, M), 256, lds, static_cast<hipStream_t>(stream)>>>(
+        route, h, dn_blocks, resid, experts, top_k, hidden, inter, M, DownNorm{});
   return mi_hip(static_cast<int>(hipGetLastError()), "moe_down launch");
 }
 
@@ -689,8 +716,12 @@ extern "C" int mi_moe_down_norm(const uint32_t* route, const uint16_t* h, const 
     return mi_fail(MI_ERR_ARG, "moe_down_norm: dn_blocks and h need 16-byte alignment");
   const size_t lds = size_t(top_k + 1) * (inter / 64) * kHalfU32 * 4;
   const DownNorm dnm{handoff, norm_w, x_out, rstd, eps, status, poll_limit ? poll_limit : kDnPollLimit, inject};
-  moe_down_kernel<<<dim3(hidden / 8, M + 1), 256, lds, static_cast<hipStream_t>(stream)>>>(
-      route, h, dn_blocks, resid, experts, top_k, hidden, inter, M, dnm);
+  if (down_wide(top_k, inter))
+    moe_down_kernel<640><<<dim3(hidden / 8, M + 1), 640, lds, static_cast<hipStream_t>(stream)>>>(
+        route, h, dn_blocks, resid, experts, top_k, hidden, inter, M, dnm);
+  else
+    moe_down_kernel<256><<<dim3(hidden / 8, M + 1), 256, lds, static_cast<hipStream_t>(stream)>>>(
+        route, h, dn_blocks, resid, experts, top_k, hidden, inter, M, dnm);
   return mi_hip(static_cast<int>(hipGetLastError()), "moe_down_norm launch");
 }
 

@@ -178,6 +178,32 @@ def test_gate_up_and_down_vs_oracle(moe256, M):
         assert f16_ulps(res_gpu[m], res_or).max() <= 2
 
 
+@pytest.mark.parametrize("K,inter", [(8, 128), (1, 1024), (3, 640), (8, 512), (8, 1024)])
+def test_down_terms_by_work_group_size(K, inter):
+    """The down launch's (slot, group, column) terms below, at and above one turn of 256 and of 640
+    threads: bitwise the oracle's split dots and combine, every column."""
+    hidden, M = 512, 2
+    mo = Moe(11, E=16, hidden=hidden, inter=inter, router_n=32, top_k=K)
+    rng = np.random.default_rng(K + inter)
+    lg = rng.standard_normal((M, mo.router_n)).astype(np.float32)
+    h = O.f32_to_f16_bits(rng.standard_normal((M, K + 1, inter)).astype(np.float32))
+    resid = O.f32_to_f16_bits(rng.standard_normal((M, hidden)).astype(np.float32))
+    route, dl, dh, dr = empty((M, ROUTE_WORDS), np.uint32), dev(lg), dev(h), dev(resid)
+    mi.call("mi_moe_route", ptr(dl), ptr(route), M, mo.E, K, mo.router_n, stream())
+    mi.call("mi_moe_down", ptr(route), ptr(dh), ptr(mo.d_dn), ptr(dr), M, mo.E, K, hidden, inter, stream())
+    sync()
+    rows, got = host(route, np.uint32), host(dr, np.uint16)
+    for m in range(M):
+        r = route_struct_from_row(rows[m], K)
+        for n in range(hidden):
+            d = np.empty(K + 1, np.float32)
+            for slot in range(K + 1):
+                blk = C.c_void_p(mo.dn.ctypes.data + 4 * (r.ids[slot] if slot < K else mo.E) * mo.dn_block)
+                d[slot] = O.lib().orc_moe_split_dot(F16, 1, blk, None, inter, hidden, n,
+                                                    O._p(np.ascontiguousarray(h[m, slot])), 2)
+            assert int(got[m, n]) == int(O.lib().orc_moe_combine(F16, O._p(d), C.byref(r), K, int(resid[m, n]))), n
+
+
 @pytest.mark.parametrize("E,hidden,inter,M", [(256, 2048, 512, 1), (256, 2048, 512, 3), (16, 512, 128, 2)])
 def test_routed_gate_up_is_route_then_gate_up(E, hidden, inter, M):
     """mi_moe_gate_up_routed (routing inside the gate||up launch) writes the route rows and h
