@@ -486,7 +486,7 @@ int mi_embed_rows(const uint32_t* ids, const uint16_t* embed, uint16_t* resid, u
  * shared expert last); resid [T][hidden] f16 += the slot-ordered combine (moe_ref.h:144-152).
  * Workspace: list [T (top_k + 1)] u32, tiles [(T (top_k + 1) + 63) / 64 + experts + 1] x 4 u32
  * (16-byte aligned), tiles_n [1], h [T (top_k + 1)][inter] f16, d [T (top_k + 1)][hidden] f16.
- * Each expert's pairs run through the int4 MFMA tile in 64-row tiles, so the per-pair values
+ * Each expert's pairs run through the int4 MFMA tile in tiles of up to 96 rows, so the per-pair values
  * round like mi_gemm_w4a16 (one f16 rounding per weight), not like the decode kernels. T <= 2048. */
 int mi_moe_prefill(const uint32_t* route, const uint16_t* x, const uint32_t* gu_blocks,
                    const uint32_t* dn_blocks, uint16_t* resid, uint32_t T, uint32_t experts,
