@@ -1230,17 +1230,21 @@ static int cu_count(uint32_t* cus, const char* name) {
   return 0;
 }
 
-// The work-group shape of the GEMM: rows per tile 16 ri, k parts ks (or the few-rows kernel). All but
-// the 128-row tile run one work-group of 8 waves per CU, so a launch takes ceil(work-groups / CUs)
-// rounds; a round's time over 80 k-groups (K = 5120), measured on a 256-CU part, is the table's
-// `cost` (us x 10), what a launch adds to it `over`. The rule takes the shape with the least sum.
+// The work-group shape of the GEMM: rows per tile 16 ri, k parts ks (or the few-rows kernel). A
+// launch takes ceil(work-groups / CUs) rounds; the rule takes the shape with the least
+//   launch + rounds (round + K / 64 step),
+// a round's own cost being the pipeline's fill, the parts' merge and the epilogue: it decides for
+// short K over many rounds, where the 4-wave shapes (two work-groups per CU, so one's ends run
+// beside the other's products) win. The three ns were fitted to 118 shapes of 150..2048 rows on a
+// 256-CU part (within 15 % of 9 in 10; the choice 0.2 % off the best shape on average); the
+// few-rows ones are from K = 5120. 772 x 1728 -> 29952 125 -> 110 us by the round's cost; a 96-row tile of
+// 4 waves would be better still for some (546 x 1344 -> 16896: 53 us, 46 with it).
 // Measured (us, the one 4-wave kernel of 64..128-row tiles before / this rule's choice; K -> N):
 //   5120 -> 7168: 8 rows 65.5 / 11.3 (few, 16 rows), 64: 66.4 / 20.9 (few, 32), 100: 67.6 / 27.5 (few, 64),
 //   200: 67.5 / 36 (32 x 256), 333: 68.6 / 41 (48), 500: 69.2 / 45 (64), 777: 83.4 / 63 (96),
 //   1500: 140 / 119 (96), 2048: 169 / 155 (128);
 //   17408 -> 5120: 8 rows 218 / 26, 64: 220 / 48, 333: 220 / 110, 777: 267 / 190, 2048: 414 / 368;
 //   12864 -> 2816: 8 rows 160 / 19, 64: 162 / 26, 1024: 168 / 101.
-// (The 128-row tile, 4 waves and two work-groups per CU, loses to the others until it needs fewer rounds.)
 struct GemmPick {
   bool few;
   uint32_t ri, ks;
@@ -1248,17 +1252,19 @@ struct GemmPick {
 static GemmPick pick_gemm(uint32_t T, uint32_t K, uint32_t N, uint32_t cus) {
   static constexpr struct {
     GemmPick p;
-    uint32_t cost, over;
-  } kShapes[] = {{{true, 1, 8}, 110, 20},  {{true, 2, 8}, 160, 20},  {{true, 4, 8}, 240, 20},
-                 {{false, 1, 2}, 270, 40}, {{false, 2, 2}, 330, 40}, {{false, 3, 2}, 390, 40},
-                 {{false, 4, 2}, 450, 40}, {{false, 6, 2}, 640, 40}, {{false, 8, 1}, 775, 40}};
+    int64_t launch, round, step;  // ns
+  } kShapes[] = {{{true, 1, 8}, 0, 2000, 138},       {{true, 2, 8}, 0, 2000, 200},
+                 {{true, 4, 8}, 0, 2000, 300},       {{false, 1, 2}, 3370, 1640, 309},
+                 {{false, 2, 2}, 2430, 2800, 361},   {{false, 3, 2}, -320, 6160, 436},
+                 {{false, 4, 2}, -1660, 8080, 493},  {{false, 6, 2}, -3680, 11630, 608},
+                 {{false, 8, 1}, 6190, 2770, 875}};
   GemmPick best{false, 8, 1};
-  uint64_t least = ~0ull;
+  int64_t least = INT64_MAX;
   for (const auto& s : kShapes) {
     const uint64_t rows = (T + 16u * s.p.ri - 1u) / (16u * s.p.ri);
     if (rows > 65535u) continue;  // the grid's limit
     const uint64_t wg = rows * (s.p.few ? N / 64u : (N + 255u) / 256u);
-    const uint64_t t = (wg + cus - 1u) / cus * s.cost * (K / GBK) + 80ull * s.over;
+    const int64_t t = s.launch + (int64_t)((wg + cus - 1u) / cus) * (s.round + (int64_t)(K / GBK) * s.step);
     if (t < least) {
       least = t;
       best = s.p;
