@@ -870,10 +870,15 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
   }
 
   // m_run: the column's reference exponent. It is raised to the largest c s seen only when that
-  // exceeds it by more than kSlack (weights up to 2^kSlack lose nothing in fp32 or in the f16 high
-  // and low parts), so after a few keys the accumulators are hardly ever rescaled and the maximum
-  // over the column's four lanes hardly ever formed
-  constexpr float kNoKey = -1e30f, kSlack = 8.f;
+  // exceeds it by more than kSlack (the threshold of FlashAttention-4's conditional rescaling; f16 rows:
+  // weights up to 2^kSlack lose nothing in fp32 or in the f16 high and low parts), so after a few keys
+  // the accumulators are hardly ever rescaled and the maximum over the column's four lanes hardly ever
+  // formed. An int8 row's weight becomes f16 times its V scale, which passes f16's 65504 from a scale
+  // of 256 on: a lane with a scale above kSlackScale among its eight keys takes no slack, so its
+  // weights stay within 1 (c_up, c_dn: the largest c s rounded up) and no scale overflows (seven
+  // instructions per 32 keys: 777 rows over 3778 keys 127.1 -> 127.7 us).
+  constexpr float kNoKey = -1e30f, kSlack = 8.f, kSlackScale = 255.f;
+  const float c_up = KV8 ? c * 1.0000002384f : c, c_dn = KV8 ? c * 0.9999997616f : c;
   float m_run[CT], l_run[CT];
   f4_t acc[CT][NT];
 #pragma unroll
@@ -914,6 +919,12 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
           vscale[g] = *reinterpret_cast<const f4_t*>(s.vs + 32u * ks + 16u * g + 4u * qq);
         }
       }
+      float slack = kSlack;
+      if constexpr (KV8 == 1) {  // (the largest of the lane's eight keys' scales, whose weights it forms)
+        auto abs3 = [](float x, float y, float z) { return max3(fabsf(x), fabsf(y), fabsf(z)); };
+        const f4_t v0 = vscale[0], v1 = vscale[1];
+        if (max3(abs3(v0[0], v0[1], v0[2]), abs3(v0[3], v1[0], v1[1]), abs3(v1[2], v1[3], v1[3])) > kSlackScale) slack = 0.f;
+      }
       const bool masked = g0 + 31u > a.pos0 + t0;  // uniform: some column does not see every key
       u4_t bh[CT], bl[CT];
 #pragma unroll
@@ -929,8 +940,9 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
           for (uint32_t e = 0; e < 8; ++e)
             w[e] = g0 + 16u * (e / 4) + 4u * qq + e % 4 <= lim[ct] ? w[e] : -INFINITY;
         }
-        const float mx = max3(max3(w[0], w[1], w[2]), max3(w[3], w[4], w[5]), max3(w[6], w[7], w[7])) * c;
-        if (__ballot(mx > m_run[ct] + kSlack)) {
+        float mx = max3(max3(w[0], w[1], w[2]), max3(w[3], w[4], w[5]), max3(w[6], w[7], w[7]));
+        mx *= mx > 0.f ? c_up : c_dn;
+        if (__ballot(mx > m_run[ct] + slack)) {
           const float m_new = fmaxf(m_run[ct], col_max(mx));
           const float alpha = __builtin_amdgcn_exp2f(m_run[ct] - m_new);
           m_run[ct] = m_new;

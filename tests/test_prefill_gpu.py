@@ -288,6 +288,50 @@ def test_attn_prefill_work_group_shapes_vs_fp64(QH, KVH, HD, T, pos0, int8):
         assert np.all(err <= bound), (h, (err / bound).max())
 
 
+# keys in one part and in two, 64 columns per work-group; the key counts end inside an iteration
+@pytest.mark.parametrize("T,pos0", [(5, 259), (100, 301), (1030, 231)])
+@pytest.mark.parametrize("big", [255, 256, 300, 8000, 65504])
+def test_attn_prefill_int8_large_v_scales(T, pos0, big):
+    """V scales up to f16's largest under scores that rise by 7.9 in log2 units after the first 128
+    keys (a weight times its V scale must stay an f16 value), every third key's scale large, against
+    fp64 attention on the fp32 rotated output (the f16 one overflows by itself)."""
+    QH, KVH, HD, keys = 16, 2, 256, pos0 + T
+    sh = O.attn_shape(QH, KVH, HD)
+    rng = np.random.default_rng(T)
+    u = rng.choice([-1, 1], (KVH, 1, HD)) * rng.integers(64, 120, (KVH, 1, HD))
+    k8 = (u + rng.integers(-3, 4, (KVH, keys, HD))).astype(np.int8)
+    v8 = rng.integers(-127, 128, (KVH, keys, HD)).astype(np.int8)
+    rise = np.clip((np.arange(keys) - 128) / 32, 0.002, 1) * 7.9 / np.log2(np.e)
+    ks = O.f32_to_f16_bits(np.tile((0.05 * rise / rise[-1]).astype(np.float32), (KVH, 1)))
+    vs = O.f32_to_f16_bits(np.where(np.arange(keys) % 3 == 0, big, 0.03)[None].repeat(KVH, 0).astype(np.float32))
+    # q along u, so that the last keys' score is rise[-1]
+    gain = rise[-1] / (0.05 * np.square(u.astype(np.float64)).sum(-1) * float(sh.scale))
+    q = (np.repeat((u[:, 0] * gain).astype(np.float32), QH // KVH, 0)[None] * np.linspace(0.97, 1, T)[:, None, None]).astype(np.float32)
+    print(f"attn_prefill_kv8 V scale {big} T={T} pos0={pos0}", flush=True)
+    keep = [dev(a) for a in (q, k8, v8, ks, vs)]
+    rot, out = empty((T, QH, HD), np.float32), empty((T, QH * HD), np.uint16)
+    mi.call("mi_attn_prefill_kv8", *[ptr(a) for a in keep], HD, keys * HD, 1, keys, None, 0, T, pos0, mi.shape_ref(sh),
+            ptr(rot), ptr(out), stream())
+    sync()
+    got = host(rot, np.float32).reshape(T, QH, HD).astype(np.float64)
+    assert np.isfinite(got).all()
+    hidden = np.arange(keys)[None, :] > pos0 + np.arange(T)[:, None]
+    for h in range(0, QH, QH // KVH):
+        j = h // (QH // KVH)
+        kh = k8[j] * O.f16_bits_to_f32(ks[j]).astype(np.float64)[:, None]
+        vh = v8[j] * O.f16_bits_to_f32(vs[j]).astype(np.float64)[:, None]
+        s = q[:, h].astype(np.float64) @ kh.T * float(sh.scale)
+        s[hidden] = -np.inf
+        w = np.exp(s - s.max(-1, keepdims=True))
+        w /= w.sum(-1, keepdims=True)
+        # test_attn_prefill_work_group_shapes_vs_fp64's bound
+        ds = 2.0 ** -21 * np.where(hidden, 0, np.abs(q[:, h]).astype(np.float64) @ np.abs(kh).T * float(sh.scale))
+        bound = (2 * ds.max(-1, keepdims=True) + 2.0 ** -20) * (w @ np.abs(vh))
+        bound += 8 * 2.0 ** -25 / 3 ** 0.5 * np.sqrt(~hidden @ np.square(v8[j].astype(np.float64)))
+        err = np.abs(got[:, h] - w @ vh)
+        assert np.all(err <= bound), (h, (err / bound).max())
+
+
 def test_attn_prefill_paged_bitwise():
     sh = O.attn_shape(40, 8, 128)
     Lm, P, T, pos0 = 512, 64, 50, 300
