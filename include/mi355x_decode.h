@@ -442,7 +442,11 @@ int mi_moe_down_norm(const uint32_t* route, const uint16_t* h, const uint32_t* d
                      uint32_t* handoff, uint32_t* status, uint32_t poll_limit, uint32_t inject, void* stream);
 
 /* ---- the chunked prefill's kernels (src/kernels/prefill: pf_gemm_q4.cl, pf_flash_attn.cl,
- * pf_embed.cl) ---- */
+ * pf_embed.cl) ----
+ * The order of a sum follows the launch's shape: T, K and N for the GEMMs, T, pos0 and the heads
+ * for the attention. The same call gives the same bits; a row computed among fewer or more rows (a
+ * prompt cut into other chunks) may differ in the last bits. A row's bits do not depend on what
+ * the other rows hold. */
 /* out [T][N] fp32 = x [T][K] f16 . W (int4 GPTQ g64 layout 0) on the matrix cores, with
  * w = f16((q - 8) * scale) (the reference's prefill rounds the same product to bf16,
  * pf_dequant_slab.cl). 64 | K, 128 | N. */
@@ -603,7 +607,8 @@ int mi_engine_ingest(mi_engine* e, const uint32_t* ids, uint32_t n);
  * cache holds those positions and cur_token is the argmax of the last position's logits, as
  * mi_engine_ingest of the same ids leaves them (up to the two paths' roundings). MoE layers run
  * their expert kernels over the chunk's rows in slices; the int8 cache takes attn_prep_kv8's
- * rows and mi_attn_prefill_kv8. Refused: no ids, chunk above the cap, an id outside the
+ * rows and mi_attn_prefill_kv8. The kernels' sum orders follow the rows per launch, so other
+ * chunk sizes give other last bits. Refused: no ids, chunk above the cap, an id outside the
  * vocabulary, past the cache. Allocates its scratch on the first call (and for a larger chunk). */
 int mi_engine_prefill(mi_engine* e, const uint32_t* ids, uint32_t n, uint32_t chunk);
 int mi_engine_read_ctrl(mi_engine* e, uint32_t* out /* MI_CTRL_WORDS */);

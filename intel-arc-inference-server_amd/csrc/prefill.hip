@@ -942,8 +942,10 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
         }
         float mx = max3(max3(w[0], w[1], w[2]), max3(w[3], w[4], w[5]), max3(w[6], w[7], w[7]));
         mx *= mx > 0.f ? c_up : c_dn;
-        if (__ballot(mx > m_run[ct] + slack)) {
-          const float m_new = fmaxf(m_run[ct], col_max(mx));
+        if (const uint64_t over = __ballot(mx > m_run[ct] + slack)) {
+          // (each column by its own four lanes, whatever its neighbours need)
+          const uint32_t o = (uint32_t)over | (uint32_t)(over >> 32);
+          const float cm = col_max(mx), m_new = ((o | o >> 16) >> qi) & 1u ? fmaxf(m_run[ct], cm) : m_run[ct];
           const float alpha = __builtin_amdgcn_exp2f(m_run[ct] - m_new);
           m_run[ct] = m_new;
           l_run[ct] *= alpha;

@@ -332,6 +332,38 @@ def test_attn_prefill_int8_large_v_scales(T, pos0, big):
         assert np.all(err <= bound), (h, (err / bound).max())
 
 
+@pytest.mark.parametrize("QH,KVH,HD,T,pos0,int8", [
+    (40, 8, 128, 6, 123, 0), (40, 8, 128, 65, 0, 0), (40, 8, 128, 810, 0, 0), (16, 2, 256, 33, 95, 0),
+    (16, 2, 256, 9, 119, 1), (16, 2, 256, 1030, 31, 1)])
+def test_attn_prefill_columns_do_not_depend_on_their_neighbours(QH, KVH, HD, T, pos0, int8):
+    """A (row, head)'s bits are the same whatever the other rows and heads of its work-group hold: half
+    of them, drawn at random, with 30 times the q, whose maxima rise where the others' do not."""
+    sh = O.attn_shape(QH, KVH, HD)
+    keys = pos0 + T
+    rng = np.random.default_rng(T)
+    q = rng.standard_normal((T, QH, HD)).astype(np.float32)
+    loud = rng.random((T, QH)) < 0.5
+    print(f"attn_prefill neighbours {QH}/{KVH}x{HD} T={T} pos0={pos0} int8={int8}", flush=True)
+
+    def run(q):
+        if not int8:
+            return prefill_attention(sh, q, k16, v16, T, pos0)
+        rot, out = empty((T, QH, HD), np.float32), empty((T, QH * HD), np.uint16)
+        mi.call("mi_attn_prefill_kv8", *[ptr(a) for a in [dev(q), *keep]], HD, keys * HD, 1, keys, None, 0, T, pos0,
+                mi.shape_ref(sh), ptr(rot), ptr(out), stream())
+        sync()
+        return host(out, np.uint16)
+
+    if int8:
+        keep = [dev(rng.integers(-127, 128, (KVH, keys, HD)).astype(np.int8)) for _ in range(2)]
+        keep += [dev(O.f32_to_f16_bits(rng.uniform(0.005, 0.05, (KVH, keys)).astype(np.float32))) for _ in range(2)]
+    else:
+        k16, v16 = (O.f32_to_f16_bits(rng.standard_normal((KVH, keys, HD)).astype(np.float32)) for _ in range(2))
+    a = run(q).reshape(T, QH, HD)
+    b = run(np.where(loud[..., None], 30 * q, q).astype(np.float32)).reshape(T, QH, HD)
+    assert np.array_equal(a[~loud], b[~loud])
+
+
 def test_attn_prefill_paged_bitwise():
     sh = O.attn_shape(40, 8, 128)
     Lm, P, T, pos0 = 512, 64, 50, 300
