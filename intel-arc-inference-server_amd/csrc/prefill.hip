@@ -98,6 +98,7 @@ __device__ __forceinline__ u4_t dequant_scaled(uint32_t w, h2_t s2, const DqCons
 
 // outputs are stored in pieces of several elements at the elements' own alignment
 typedef f4_t f4_any __attribute__((aligned(4)));
+typedef uint32_t h2_any __attribute__((aligned(2)));
 typedef u2_t h4_any __attribute__((aligned(2)));
 typedef u4_t h8_any __attribute__((aligned(2)));
 
@@ -126,27 +127,30 @@ __device__ __forceinline__ void pin(h8_t (&f)[N]) {
   for (uint32_t j = 0; j < N; ++j) asm volatile("" : "+v"(f[j]));
   __builtin_amdgcn_sched_barrier(0);
 }
-__device__ __forceinline__ uint16_t swiglu16(float g, float u) {
-  const uint16_t g_b = f2h(g), u_b = f2h(u);
-  return f2h(h2f(f2h(silu_f32(h2f(g_b)))) * h2f(u_b));
-}
+__device__ __forceinline__ uint32_t f16_pair(float x, float y) { return (uint32_t)f2h(x) | ((uint32_t)f2h(y) << 16); }
 
 // The lane's four adjacent columns ncol .. + 3 of one row. SILU: the columns are gate||up in the
-// interleave16 order, so the up values of a gate lane (fr & 4 == 0) are four lanes on; it writes h
-// [T][N/2] f16 = rne(rne(silu(rne(g))) * rne(u)) (the arithmetic of prep_silu_mul, prep.cl:384)
-// instead of the fp32 output. Every lane of the row's 16 calls it; `store`: the row and column exist.
+// interleave16 order, so a gate lane (fr & 4 == 0) and the lane four on hold the gate and the up
+// values of the same four outputs; it writes h [T][N/2] f16 = rne(rne(silu(rne(g))) * rne(u)) (the
+// arithmetic of prep_silu_mul, prep.cl:384) instead of the fp32 output. The two lanes swap a pair of f16
+// values and form two outputs each: four on the gate lane alone would leave half the lanes idle in
+// the exponentials and divisions (64 -> 20096 at 1868 rows, nearly all epilogue, 52 -> 37 us; 1088 ->
+// 25344 at 1542 137 -> 115; 5120 -> 34816 at 2048 693 -> 659). Every lane of the row's 16 calls it; `store`: the row and column exist.
 template <bool SILU>
 __device__ __forceinline__ void store_row4(f4_t v, bool store, float* out, uint16_t* h_out, uint32_t row, uint32_t ncol,
                                            uint32_t N) {
   if constexpr (SILU) {
-    uint16_t h[4];
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) h[j] = swiglu16(v[j], dpp_f<0x104>(v[j]));  // row_shl:4
-    if (store && !(ncol & 16u)) {
-      const uint32_t n = ncol / 32u * 16u + ncol % 16u;
-      *reinterpret_cast<h4_any*>(h_out + (size_t)row * (N / 2) + n) =
-          u2_t{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-    }
+    const bool up = ncol & 16u;
+    const uint32_t p01 = f16_pair(v[0], v[1]), p23 = f16_pair(v[2], v[3]);
+    const uint32_t own = up ? p23 : p01, send = up ? p01 : p23;
+    // (row_shl:4 into the gate lanes, row_shr:4 into the up lanes)
+    const int from = __builtin_amdgcn_update_dpp(0, (int)send, 0x104, 0xF, 0x5, true);
+    const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(from, (int)send, 0x114, 0xF, 0xA, true);
+    const uint32_t g = up ? got : own, u = up ? own : got;
+    const float s0 = h2f(f2h(silu_f32(h2f((uint16_t)g)))), s1 = h2f(f2h(silu_f32(h2f((uint16_t)(g >> 16)))));
+    const uint32_t n = ncol / 32u * 16u + ncol % 16u + (up ? 2u : 0u);
+    if (store)
+      *reinterpret_cast<h2_any*>(h_out + (size_t)row * (N / 2) + n) = f16_pair(s0 * h2f((uint16_t)u), s1 * h2f((uint16_t)(u >> 16)));
   } else {
     if (store) *reinterpret_cast<f4_any*>(out + (size_t)row * N + ncol) = v;
   }
