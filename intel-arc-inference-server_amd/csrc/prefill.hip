@@ -157,9 +157,12 @@ __device__ __forceinline__ void store_row4(f4_t v, bool store, float* out, uint1
 }
 
 // Tile: 16 RI rows x 256 columns, 4 waves of 16 RI x 64 per K part. KS = 2: 8 waves, waves 4 .. 7 the
-// second half of the k-groups, the halves added at the end through LDS. DA / DB: k-groups of
-// activations / weights in flight in registers ahead of the one multiplied.
-template <bool SILU, uint32_t RI, uint32_t KS, uint32_t DA>
+// second half of the k-groups, the halves added at the end through LDS. DA: k-groups of activations in
+// flight in registers ahead of the one multiplied (of weights two). ODD: a part has an odd number of
+// groups, the last of which follows the loop over pairs (a second group of zeros instead took a fifth
+// of the time at K = 64, 5 % at 1344; a branch for it inside the loop costs the waits their exact
+// counts, 3 to 10 % at K = 5120, and the code after the loop alone 3 % at 333 rows, hence a kernel each).
+template <bool SILU, uint32_t RI, uint32_t KS, uint32_t DA, bool ODD>
 __global__ __launch_bounds__(256 * KS, 2) void gemm_w4a16_kernel(const uint32_t* __restrict__ qweight,
                                                                  const uint16_t* __restrict__ scales,
                                                                  const uint16_t* __restrict__ x,
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_w4a16_kernel(const uint32_t*
   dequant_half(b_st[0], 0, dq, bf[0]);
   pin(bf[0]);
   lds_barrier();
-  for (uint32_t it0 = 0; it0 < n_it; it0 += 2u) {
+  for (uint32_t it0 = 0; it0 + (ODD ? 1u : 0u) < n_it; it0 += 2u) {
 #pragma unroll
     for (uint32_t u = 0; u < 2u; ++u) {
       const uint32_t g = g0 + it0 + u;
@@ -266,6 +269,23 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_w4a16_kernel(const uint32_t*
       store_a(u ^ 1u, a_st[(u + 1u) % DA]);  // the other buffer was last read before the previous barrier
       lds_barrier();
     }
+  }
+  if constexpr (ODD) {  // the last group
+#pragma unroll
+    for (uint32_t ks = 0; ks < 2; ++ks) {
+      if (ks) {
+        dequant_half(b_st[0], 1, dq, bf[1]);
+        pin(bf[1]);
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < RI; ++i) {
+        const h8_t af = *reinterpret_cast<const h8_t*>(&sm.As[kp][0][16u * i + fr][32u * ks + 8u * fq]);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[ks][j], acc[i][j], 0, 0, 0);
+      }
+    }
+    if constexpr (KS > 1) lds_barrier();  // (the merge reuses the staged activations)
   }
   if constexpr (KS > 1) {  // the second half's sums through LDS (the staged activations are done with)
     if (kp) {
@@ -1310,8 +1330,10 @@ static int launch_gemm(const char* name, const uint32_t* qweight, const uint16_t
   hipStream_t st = (hipStream_t)stream;
   const GemmPick p = pick_gemm(T, K, N, cus);
   const dim3 grid(p.few ? N / 64u : (N + 255u) / 256u, (T + 16u * p.ri - 1u) / (16u * p.ri));
-#define MI_GEMM(RI, KS, DA) \
-  gemm_w4a16_kernel<SILU, RI, KS, DA><<<grid, 256 * KS, 0, st>>>(qweight, scales, x, out, h, T, K, N)
+  const bool odd = (K / GBK + p.ks - 1u) / p.ks & 1u;  // k-groups per part
+#define MI_GEMM(RI, KS, DA)                                                                                    \
+  if (odd) gemm_w4a16_kernel<SILU, RI, KS, DA, true><<<grid, 256 * KS, 0, st>>>(qweight, scales, x, out, h, T, K, N); \
+  else gemm_w4a16_kernel<SILU, RI, KS, DA, false><<<grid, 256 * KS, 0, st>>>(qweight, scales, x, out, h, T, K, N)
 #define MI_GEMM_FEW(RI, D) \
   gemm_w4a16_few_kernel<SILU, RI, 8, D><<<grid, 512, 0, st>>>(qweight, scales, x, out, h, T, K, N)
   switch ((p.few ? 100u : 10u * p.ks) + p.ri) {
