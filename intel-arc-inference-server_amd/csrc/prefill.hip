@@ -12,8 +12,8 @@
 // layout 0). The contraction is a dense GEMM here (2 T K N flops over K N / 2 weight bytes):
 // MFMA-bound from some hundred rows, bound by the weights' stream and its latency below.
 //   * each wave has 16 RI rows x 64 columns = RI x 4 v_mfma_f32_16x16x32_f16 tiles; 4 waves side by
-//     side make tiles of 16 RI x 256 (RI 8: 128 rows per weight unpacked). Where a launch would
-//     leave CUs with one such work-group or none, RI is smaller and 8 waves split the k-groups in
+//     side make tiles of 16 RI x 256 (RI 4, 6 or 8: up to 128 rows per weight unpacked). Where a launch
+//     would leave CUs with one such work-group or none, 8 waves split the k-groups of 16 .. 96 rows in
 //     two parts, or (few rows) 8 waves split the k-groups of a 64-column tile (pick_gemm);
 //   * one 64-deep k-group per iteration (one scale per column). The activations go through LDS,
 //     double-buffered (the next group's rows are loaded into registers while the current group
@@ -29,10 +29,9 @@
 //     (k0,k4)(k1,k5)(k2,k6)(k3,k7) inside each 8-k chunk, so the products pair up;
 //   * fp32 accumulation in MFMA order, the k parts' sums added in ascending k. A column's order
 //     therefore depends on the shape that the rule takes, that is on T, K and N.
-// Measured at 2048 rows (MI355X, us before / now): gate||up + SwiGLU 5120 -> 34816 714 / 678 (1.08 PFLOP/s;
-// the library's plain f16 product of these sizes 1.17), q||k||v 5120 -> 7168 167 / 147, down 17408 -> 5120
-// 406 / 359; a product of the matrix cores takes twice its issue time even so, since the clock falls under
-// it (1.93 GHz at 1.0 PFLOP/s by the counters).
+// gate||up + SwiGLU 5120 -> 34816 at 2048 rows 739 -> 672 us (1.09 PFLOP/s; the library's plain f16 product
+// of these sizes 1.17; the other sizes stand at pick_gemm): a product of the matrix cores takes twice its
+// issue time even so, since the clock falls under it.
 //
 // attn_prefill_kernel: causal GQA attention of T query rows at positions pos0 .. pos0+T-1 over
 // the cache rows [0, pos0 + t] (the chunk's own rows written by attn_prep before it), f16 or the
@@ -1268,21 +1267,23 @@ static int cu_count(uint32_t* cus, const char* name) {
   return 0;
 }
 
-// The work-group shape of the GEMM: rows per tile 16 ri, k parts ks (or the few-rows kernel). A
-// launch takes ceil(work-groups / CUs) rounds; the rule takes the shape with the least
-//   launch + rounds (round + K / 64 step),
-// a round's own cost being the pipeline's fill, the parts' merge and the epilogue: it decides for
-// short K over many rounds, where the 4-wave shapes (two work-groups per CU, so one's ends run
-// beside the other's products) win. The three ns were fitted to 118 shapes of 150..2048 rows on a
-// 256-CU part (within 15 % of 9 in 10; the choice 0.2 % off the best shape on average); the
-// few-rows ones are from K = 5120. 772 x 1728 -> 29952 125 -> 110 us by the round's cost; a 96-row tile of
-// 4 waves would be better still for some (546 x 1344 -> 16896: 53 us, 46 with it).
-// Measured (us, the one 4-wave kernel of 64..128-row tiles before / this rule's choice; K -> N):
-//   5120 -> 7168: 8 rows 65.5 / 11.3 (few, 16 rows), 64: 66.4 / 20.9 (few, 32), 100: 67.6 / 27.5 (few, 64),
-//   200: 67.5 / 36 (32 x 256), 333: 68.6 / 41 (48), 500: 69.2 / 45 (64), 777: 83.4 / 63 (96),
-//   1500: 140 / 119 (96), 2048: 169 / 155 (128);
-//   17408 -> 5120: 8 rows 218 / 26, 64: 220 / 48, 333: 220 / 110, 777: 267 / 190, 2048: 414 / 368;
-//   12864 -> 2816: 8 rows 160 / 19, 64: 162 / 26, 1024: 168 / 101.
+// The work-group shape of the GEMM: rows per tile 16 ri, k parts ks (or the few-rows kernel). A CU's
+// work-groups are r = ceil(work-groups / CUs); the rule takes the shape with the least
+//   launch + (r / 2) (pair + K / 64 pair_step) + (r % 2) (round + K / 64 step).
+// Two 4-wave work-groups share a CU (pair: one's ends and waits run beside the other's products), the
+// others run one after the other (pair = 2 round); a round's own cost is the pipeline's fill, the
+// parts' merge and the epilogue. The ns were fitted on a 256-CU part to every shape's times at 888 random
+// sizes (8..2048 rows, K 64..17408, N 512..57344, plain and SwiGLU): the choice is 0.5 % off the best
+// shape on average (fitted to two thirds of them, 0.6 % on the rest), 24 % at most, at a few us.
+// Measured (us, the 4-wave kernel of 64..128-row tiles with 4-byte weight loads / this rule's choice; K -> N):
+//   5120 -> 7168: 8 rows 65.6 / 12.1 (few, 16 rows), 64: 65.9 / 20.7 (few, 32), 100: 66.8 / 27.1 (few, 64),
+//   200: 66.8 / 32.9 (32 x 256), 333: 67.2 / 38.2 (48), 500: 68.3 / 44.3 (64), 777: 84.8 / 59.1 (96),
+//   1500: 128 / 111 (96 in one part), 2048: 163 / 141 (128);
+//   17408 -> 5120: 8 rows 217 / 26.6, 64: 218 / 48.2, 333: 222 / 105, 777: 268 / 170, 2048: 421 / 363;
+//   12864 -> 2816: 8 rows 161 / 20.2, 64: 161 / 26.2, 1024: 183 / 105;
+//   SwiGLU: 1344 -> 16896 at 546 rows 41.9 / 38.5, 1600 -> 32128 at 270 53.0 / 39.1, 1728 -> 29952 at 772 112 / 104.
+// The geometric mean over 250 other sizes from K = 512 on is 2.4, none slower; below K = 448 nine of 83 are,
+// by 3 to 12 % (at most 2 us: a round's ends are nearly all of them).
 struct GemmPick {
   bool few;
   uint32_t ri, ks;
@@ -1290,19 +1291,21 @@ struct GemmPick {
 static GemmPick pick_gemm(uint32_t T, uint32_t K, uint32_t N, uint32_t cus) {
   static constexpr struct {
     GemmPick p;
-    int64_t launch, round, step;  // ns
-  } kShapes[] = {{{true, 1, 8}, 0, 2000, 138},       {{true, 2, 8}, 0, 2000, 200},
-                 {{true, 4, 8}, 0, 2000, 300},       {{false, 1, 2}, 3370, 1640, 309},
-                 {{false, 2, 2}, 2430, 2800, 361},   {{false, 3, 2}, -320, 6160, 436},
-                 {{false, 4, 2}, -1660, 8080, 493},  {{false, 6, 2}, -3680, 11630, 608},
-                 {{false, 8, 1}, 6190, 2770, 875}};
+    int64_t launch, pair, pair_step, round, step;  // ns
+  } kShapes[] = {{{true, 1, 8}, 1899, 5116, 186, 2558, 93}, {{true, 2, 8}, 1392, 9904, 238, 4952, 119},
+                 {{true, 4, 8}, 0, 10230, 412, 5115, 206}, {{false, 1, 2}, 3203, 1614, 484, 807, 242},
+                 {{false, 2, 2}, 3793, 2156, 700, 1078, 350}, {{false, 3, 2}, 1186, 8206, 832, 4103, 416},
+                 {{false, 4, 2}, 558, 10852, 998, 5426, 499}, {{false, 6, 2}, 0, 13074, 1294, 6537, 647},
+                 {{false, 4, 1}, 3373, 4409, 934, 1666, 585}, {{false, 6, 1}, 1048, 7432, 1254, 4493, 738},
+                 {{false, 8, 1}, 1189, 13167, 1452, 6702, 926}};
   GemmPick best{false, 8, 1};
   int64_t least = INT64_MAX;
   for (const auto& s : kShapes) {
     const uint64_t rows = (T + 16u * s.p.ri - 1u) / (16u * s.p.ri);
     if (rows > 65535u) continue;  // the grid's limit
     const uint64_t wg = rows * (s.p.few ? N / 64u : (N + 255u) / 256u);
-    const int64_t t = s.launch + (int64_t)((wg + cus - 1u) / cus) * (s.round + (int64_t)(K / GBK) * s.step);
+    const int64_t r = (int64_t)((wg + cus - 1u) / cus), G = K / GBK;
+    const int64_t t = s.launch + r / 2 * (s.pair + G * s.pair_step) + r % 2 * (s.round + G * s.step);
     if (t < least) {
       least = t;
       best = s.p;
@@ -1345,6 +1348,8 @@ static int launch_gemm(const char* name, const uint32_t* qweight, const uint16_t
     case 23: MI_GEMM(3, 2, 2); break;
     case 24: MI_GEMM(4, 2, 2); break;
     case 26: MI_GEMM(6, 2, 1); break;
+    case 14: MI_GEMM(4, 1, 2); break;
+    case 16: MI_GEMM(6, 1, 1); break;
     default: MI_GEMM(8, 1, 1); break;
   }
 #undef MI_GEMM

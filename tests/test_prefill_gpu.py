@@ -43,9 +43,7 @@ def dequant16(qw, sc):
     return ((q.astype(np.float32) - 8) * s).astype(np.float16).astype(np.float64)
 
 
-# the shapes take all four work-group tiles on a 256-CU part (N % 256 != 0: 128 x 128; small
-# grids: 64 x 256; T = 2000, N = 5120: 96 x 256; T = 1000, N = 14336: 128 x 256), with ragged T
-# and odd group counts
+# small and large grids, a last column tile of 128 (N % 256 != 0), ragged T, odd group counts
 @pytest.mark.parametrize("T,K,N", [(1, 256, 128), (3, 64, 256), (9, 320, 384), (37, 1024, 384), (130, 2048, 256),
                                    (256, 5120, 512), (1000, 192, 14336), (2000, 64, 5120)])
 def test_gemm_vs_fp64(T, K, N):
@@ -64,9 +62,8 @@ def test_gemm_vs_fp64(T, K, N):
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
 
 
-# the launch rule's work-group shapes on a 256-CU part, in its order (16, 32, 64 rows with the k-groups
-# over 8 waves; 16 .. 96 rows x 256 columns in two k parts; 128 rows): full and ragged rows, odd group
-# counts, fewer groups than waves or parts, a last tile of 128 columns
+# the launch rule's work-group shapes on a 256-CU part, with those of the list below: full and ragged
+# rows, odd group counts, fewer groups than waves or parts, a last tile of 128 columns
 @pytest.mark.parametrize("T,K,N", [(16, 448, 384), (5, 64, 128), (17, 576, 7296), (64, 320, 7168), (33, 64, 7168),
                                    (100, 832, 7168), (16, 1856, 34816), (11, 2112, 34944), (30, 1856, 34816),
                                    (48, 1856, 34816), (35, 2112, 34944), (64, 1856, 34816), (511, 1088, 7296),
@@ -89,6 +86,16 @@ def test_gemm_work_group_shapes(T, K, N):
     over = np.abs(got - xf @ w) / bound
     assert np.all(over <= 1), over.max()
     assert np.array_equal(host(h, np.uint16), host(hw, np.uint16))
+
+
+# k parts of an even number of groups for each number of rows, then the rest of the rule's shapes: 64, 96 and
+# 128 rows in one part, 96 in two, 32 and 64 with the k-groups over 8 waves
+@pytest.mark.parametrize("T,K,N", [(17, 192, 9472), (17, 192, 34816), (129, 192, 14464), (50, 768, 34816), (79, 768, 34816),
+                                   (50, 128, 34816), (50, 64, 34944), (64, 192, 34816), (79, 128, 34816), (95, 64, 34944),
+                                   (850, 384, 14464), (333, 448, 34816), (79, 832, 34816), (50, 832, 34816), (17, 1536, 9472),
+                                   (17, 1600, 9472), (33, 2048, 9472), (33, 2112, 9472)])
+def test_gemm_work_group_shapes_more(T, K, N):
+    test_gemm_work_group_shapes(T, K, N)
 
 
 def test_gemm_outputs_at_their_own_alignment():
