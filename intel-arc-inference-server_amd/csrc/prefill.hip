@@ -1388,10 +1388,16 @@ int mi_moe_prefill(const uint32_t* route, const uint16_t* x, const uint32_t* gu_
       reinterpret_cast<uintptr_t>(dn_blocks) % 4)
     return mi_fail(MI_ERR_ARG, "moe_prefill: tiles, x and h need 16-byte, gu_blocks and dn_blocks 4-byte alignment");
   const uint32_t slots = top_k + 1, P = T * slots;
-  // the tile's most 16-row blocks by the mean pairs per expert (256 experts, top 8, 2048 -> 512; the whole
-  // block in us at 2 / 4 / 6): 10 pairs 156 / 161 / 185, 16: 178 / 182 / 207, 32: 254 / 227 / 249,
-  // 47: 336 / 273 / 295, 64: 415 / 352 / 345
-  const uint32_t mean = T * top_k / experts, rmax = mean <= 20u ? 2u : mean <= 52u ? 4u : 6u;
+  // The tile's most 16-row blocks by the mean pairs per expert. Measured at 2 / 4 / 6 (us, the whole block, pairs
+  // spread evenly): 256 experts, top 8, 2048 -> 512: 8 pairs 114 / 120 / 141, 16: 125 / 129 / 152, 32: 188 / 153 / 176,
+  // 46: 248 / 186 / 202, 64: 309 / 242 / 230; ten other shapes of 16..256 experts cross at 16..24 and 48..72. Six
+  // blocks pay where one tile then holds an expert's pairs (32 experts, top 8, 2048 -> 512: 80 pairs 69 / 61 at 4 / 6,
+  // 96: 71 / 63). From there to 140 both take two tiles, and those of four blocks have more waves in flight (112: 71 / 90,
+  // 128: 73 / 91; tiles of 64 rows in the kernel before: 85, 87). Beyond, six save a tile, which pays where a tile
+  // works long (hidden x inter 2^21 on: 64 experts, top 8, 3072 -> 768 at 176: 278 / 260; 32 experts, 2048 -> 512: 89 / 96).
+  const uint32_t mean = T * top_k / experts;
+  const bool one96 = mean > 52u && mean <= 96u, long96 = mean > 140u && hidden * inter >= 1u << 21;
+  const uint32_t rmax = mean <= 20u ? 2u : one96 || long96 ? 6u : 4u;
   const uint32_t tile_rows = rmax == 6u ? 96u : 64u;
   const uint32_t max_tiles = (P + tile_rows - 1u) / tile_rows + experts + 1u;
   const size_t gu_block = (size_t)(2u * inter / 16u) * (hidden / GBK) * kMoeTile;

@@ -375,10 +375,10 @@ def test_moe_prefill_matches_decode_kernels(T, bad):
 # rows), with random routes and with every row on the same experts (whole tiles and remainders)
 @pytest.mark.parametrize("T,K,skew", [(16, 1, False), (40, 8, False), (42, 8, False), (42, 8, True), (104, 8, False),
                                       (104, 7, True), (107, 8, False), (97, 8, True), (193, 5, True), (129, 8, True)])
-def test_moe_prefill_tile_shapes(T, K, skew):
+def test_moe_prefill_tile_shapes(T, K, skew, H=512, I=128):
     """mi_moe_prefill's row tiles against the oracle of the prefill block (rel 2e-3, as
     test_moe_prefill_matches_decode_kernels), the pairs' list the stable sort by expert."""
-    E, H, I = 16, 512, 128
+    E = 16
     mo = Moe(5, E=E, top_k=K, hidden=H, inter=I, router_n=32)
     rng = np.random.default_rng(T + K)
     x = O.f32_to_f16_bits(rng.standard_normal((T, H)).astype(np.float32))
@@ -403,6 +403,12 @@ def test_moe_prefill_tile_shapes(T, K, skew):
     assert np.all(np.abs(got - want) <= 2e-3 * np.abs(want) + 2e-3 * np.abs(want).max())
     ex = np.concatenate([rt[:, :K].astype(np.int64), np.full((T, 1), E)], axis=1).ravel()
     assert np.array_equal(host(lst, np.uint32), np.argsort(ex, kind="stable").astype(np.uint32))
+
+
+# the rule's other edges: 96 / 97 pairs, and 140 / 141 with hidden x inter below 2^21 and at it
+@pytest.mark.parametrize("T,H,I", [(192, 512, 128), (194, 512, 128), (282, 512, 128), (280, 2048, 1024), (282, 2048, 1024)])
+def test_moe_prefill_tile_shapes_above_96_pairs(T, H, I):
+    test_moe_prefill_tile_shapes(T, 8, False, H, I)
 
 
 @pytest.mark.parametrize("M,K,N,ksplit", [(64, 64, 16, 8), (65, 128, 80, 4), (71, 1088, 272, 8), (100, 576, 48, 1),
