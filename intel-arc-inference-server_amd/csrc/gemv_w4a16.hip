@@ -724,11 +724,13 @@ __global__ __launch_bounds__(256, (MR == 16 && U == 1 ? 6 : 1)) void gemv_w4a16_
 }
 
 // out[m][n] (fp16 or fp32) = sum over s ascending of partials[s][m][n], from 0.f. V adjacent outputs
-// per thread, the loads of up to 16 slices together (a slice past S re-reads the last and is not
-// added), so a fold takes one memory round trip per 16 slices rather than one per slice: bound by
-// the partials' bytes at many rows (10 x 16 x 34816 floats, 22 MB: 7.0 -> 5.6 us), by that round
-// trip at one.
-template <int V>
+// per thread, the loads of B slices together (a slice past S re-reads the last and is not added), so a
+// fold takes one memory round trip per B slices rather than one per slice: bound by the partials'
+// bytes at many rows (10 x 16 x 34816 floats, 22 MB: 7.0 -> 5.6 us), by that round trip at one. B follows
+// S (launch_fold): with 16 for every S a linear of few k-groups lost to its re-read slices what the round
+// trips gave (with its GEMV, one slice at a time / 16 / this: 7 rows of 1856 -> 25344 10.0 / 10.8 / 10.0, 16 of 512 ->
+// 34816 8.95 / 9.5 / 8.4, 14 of 2752 -> 7360 11.4 / 12.2 / 11.4; one row of 17408 -> 5120 18.6 / 12.6 / 12.3).
+template <int V, int B>
 __global__ __launch_bounds__(256) void fold_partials_kernel(const float* __restrict__ partials,
                                                             uint16_t* __restrict__ out16,
                                                             float* __restrict__ out32,
@@ -736,7 +738,6 @@ __global__ __launch_bounds__(256) void fold_partials_kernel(const float* __restr
   typedef float fv_t __attribute__((ext_vector_type(V), aligned(4)));
   const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * V;
   if (i >= MN) return;
-  constexpr uint32_t B = 16;
   float t[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) t[k] = 0.f;
@@ -755,6 +756,25 @@ __global__ __launch_bounds__(256) void fold_partials_kernel(const float* __restr
     if (out16) out16[i + k] = f2h(t[k]);
     if (out32) out32[i + k] = t[k];
   }
+}
+
+template <int V>
+void launch_fold(const float* partials, uint16_t* out16, float* out32, uint32_t S, uint32_t MN, hipStream_t st) {
+  const uint32_t wg = (MN / V + 255u) / 256u;
+  // the fewest round trips of at most 16 slices, equally long (up to one slice re-read per trip)
+  const uint32_t trips = (S + 15u) / 16u, b = (S + trips - 1u) / trips;
+#define MI_FOLD(B) fold_partials_kernel<V, B><<<wg, 256, 0, st>>>(partials, out16, out32, S, MN)
+  switch ((b + 1u) / 2u) {
+    case 1: if (b == 1u) MI_FOLD(1); else MI_FOLD(2); break;
+    case 2: MI_FOLD(4); break;
+    case 3: MI_FOLD(6); break;
+    case 4: MI_FOLD(8); break;
+    case 5: MI_FOLD(10); break;
+    case 6: MI_FOLD(12); break;
+    case 7: MI_FOLD(14); break;
+    default: MI_FOLD(16); break;
+  }
+#undef MI_FOLD
 }
 
 __global__ __launch_bounds__(256) void handoff_init_kernel(uint32_t* __restrict__ p, size_t n) {
@@ -964,8 +984,8 @@ extern "C" int mi_fold_partials(const float* partials, uint16_t* out_f16, float*
   // four outputs per thread where that still gives every CU a few waves, else one
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (MN % 4u == 0 && MN >= 65536u)
-    fold_partials_kernel<4><<<(MN / 4u + 255u) / 256u, 256, 0, st>>>(partials, out_f16, out_f32, S, MN);
+    launch_fold<4>(partials, out_f16, out_f32, S, MN, st);
   else
-    fold_partials_kernel<1><<<(MN + 255u) / 256u, 256, 0, st>>>(partials, out_f16, out_f32, S, MN);
+    launch_fold<1>(partials, out_f16, out_f32, S, MN, st);
   return mi_hip((int)hipGetLastError(), "fold_partials launch");
 }

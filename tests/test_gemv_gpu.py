@@ -143,3 +143,10 @@ def test_fold_partials_in_slice_order(S, M, N, off):
     sync()
     assert np.array_equal(host(o32, np.uint32), want.view(np.uint32))
     assert np.array_equal(host(o16, np.uint16), O.f32_to_f16_bits(want))
+
+
+# every batch length, for one and four outputs per thread, with and without a slice past S in the last batch
+@pytest.mark.parametrize("N", [65, 65536])
+@pytest.mark.parametrize("S", [2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 18, 19, 27, 34])
+def test_fold_partials_batch_lengths(S, N):
+    test_fold_partials_in_slice_order(S, 1, N, 0)
