@@ -387,6 +387,52 @@ def test_attn_prefill_paged_bitwise():
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("P", [16, 64])
+@pytest.mark.parametrize("QH,KVH,HD,T,pos0,int8", [
+    (40, 8, 128, 6, 123, 0), (40, 8, 128, 64, 0, 0), (40, 8, 128, 7, 185, 0), (40, 8, 128, 810, 0, 0), (16, 2, 256, 5, 59, 0),
+    (16, 2, 256, 33, 95, 0), (16, 2, 256, 1030, 0, 0), (16, 2, 256, 1, 0, 1), (16, 2, 256, 9, 119, 1), (16, 2, 256, 1030, 31, 1),
+    (24, 4, 256, 37, 290, 1)])
+def test_attn_prefill_work_group_shapes_paged_bitwise(QH, KVH, HD, T, pos0, int8, P):
+    """Each work-group shape through a permuted page table, keys ending inside a page: bitwise the
+    contiguous cache. Every row that no key has holds NaN (int8: NaN scales)."""
+    sh = O.attn_shape(QH, KVH, HD)
+    keys = pos0 + T
+    npg = -(-keys // P) + 3
+    rng = np.random.default_rng(T + pos0 + P)
+    pages = rng.permutation(npg).astype(np.uint32)
+    phys = (pages[:, None] * P + np.arange(P)).ravel()[:keys]
+    q = rng.standard_normal((T, QH, HD)).astype(np.float32)
+    print(f"attn_prefill paged {QH}/{KVH}x{HD} T={T} pos0={pos0} int8={int8} P={P}", flush=True)
+
+    def paged(a, fill):
+        b = np.full((KVH, npg * P) + a.shape[2:], fill, a.dtype)
+        b[:, phys] = a
+        return b
+
+    if int8:
+        kv = [rng.integers(-127, 128, (KVH, keys, HD)).astype(np.int8) for _ in range(2)]
+        sc = [O.f32_to_f16_bits(rng.uniform(0.005, 0.05, (KVH, keys)).astype(np.float32)) for _ in range(2)]
+
+        def run(kv, sc, Lm, pages, P):
+            keep = [dev(a) for a in (q, *kv, *sc)]
+            rot, out, dpg = empty((T, QH, HD), np.float32), empty((T, QH * HD), np.uint16), dev(pages)
+            mi.call("mi_attn_prefill_kv8", *[ptr(a) for a in keep], HD, Lm * HD, 1, Lm, ptr(dpg), P, T, pos0, mi.shape_ref(sh),
+                    ptr(rot), ptr(out), stream())
+            sync()
+            return host(out, np.uint16), host(rot, np.uint32)
+
+        want = run(kv, sc, keys, None, 0)
+        got = run([paged(a, 127) for a in kv], [paged(a, 0x7E00) for a in sc], npg * P, pages, P)
+        assert np.array_equal(got[1], want[1])
+        got, want = got[0], want[0]
+    else:
+        k, v = (O.f32_to_f16_bits(rng.standard_normal((KVH, keys, HD)).astype(np.float32)) for _ in range(2))
+        want = prefill_attention(sh, q, k, v, T, pos0)
+        got = prefill_attention(sh, q, paged(k, 0x7E00), paged(v, 0x7E00), T, pos0, pages, P)
+    assert np.array_equal(got, want)
+    assert np.isfinite(O.f16_bits_to_f32(want)).all()
+
+
 def kv_rows(eng, p0, n):
     d = eng.desc
     k = eng.to_host(mi.T_KV_K, 0, np.uint16).reshape(d.layers, d.kv_heads, d.max_len, d.head_dim)
