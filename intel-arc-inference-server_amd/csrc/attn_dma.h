@@ -99,15 +99,6 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
 
-// two fp32 values as f16 pairs, high and low parts (the remainder v - h is exact in fp32: one fma
-// that reads the f16 value directly, with neg1 = -1, which the compiler may not know to be -1 - it
-// would make the fma a conversion and a subtraction)
-__device__ __forceinline__ void f16_parts(float v0, float v1, float neg1, uint32_t& hi, uint32_t& lo) {
-  const h2_t h = __builtin_convertvector((f2_t{v0, v1}), h2_t);
-  const float l0 = __builtin_fmaf((float)h.x, neg1, v0), l1 = __builtin_fmaf((float)h.y, neg1, v1);
-  hi = h2_bits(h);
-  lo = h2_bits(__builtin_convertvector((f2_t{l0, l1}), h2_t));
-}
 template <uint32_t NB, uint32_t DG>
 __device__ __forceinline__ void wait_group(uint32_t after) {  // after: groups issued after it
   if (after == 0) wait_vm<0>();
@@ -139,9 +130,8 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
   constexpr uint32_t NB = QREG ? C::NB : (NBMIN + NG - 1u) / NG * NG;
   constexpr uint32_t RING = 4u * NB * SLOT;
   static_assert(RING >= RED, "merge area");
-  constexpr uint32_t MT = RING >= CT * RED ? CT : 1u;  // tiles merged at once
   __shared__ __align__(16) unsigned char s_ring[RING];
-  __shared__ float st_m[4][16 * MT], st_l[4][16 * MT], st_f[4][16 * MT], st_hm[16 * MT], st_hs[16 * MT];
+  __shared__ float st_m[4][16], st_l[4][16], st_f[4][16], st_hm[16], st_hs[16];
   __shared__ uint32_t s_grow[kMaxBlockGroups];
   __shared__ h8_t s_q[QREG ? 1 : CT][2][QREG ? 1 : KK][QREG ? 1 : 64];
   // FP: the new K/V rows (f16), the roped q of the GQA heads and the waves' normed rows. At
@@ -492,15 +482,12 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     ksh[r] = 16u * (((uint32_t)((uintptr_t)a.k_scale >> 1) + e) & 1u);
     vsh[r] = 16u * (((uint32_t)((uintptr_t)a.v_scale >> 1) + e) & 1u);
   }
-  // the max over the four lanes l % 16 + 16 k that hold one head's scores: v_permlane16_swap
-  // and v_permlane32_swap of x with a copy of itself leave rows (0, 0, 2, 2) / (1, 1, 3, 3) and
-  // halves (lo, lo) / (hi, hi) in the two registers (VALU, no LDS round trip). Written as
-  // assembly: the compiler's builtin for these swaps dropped the second result here.
+  // the max over the four lanes l % 16 + 16 k that hold one head's scores
   auto head_max = [](float x) {
     float a0 = x, a1 = x;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a0), "+v"(a1));
+    lane_swap16(a0, a1);
     float b0 = fmaxf(a0, a1), b1 = b0;
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(b0), "+v"(b1));
+    lane_swap32(b0, b1);
     return fmaxf(b0, b1);
   };
   static_assert(NB % NG == 0, "ring");
@@ -731,29 +718,25 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
   }
   wait_vm<0>();
   lds_barrier();  // every wave is done with its ring, which the merge reuses
-  // merge the four waves, MT tiles of columns at a time: M = max m_w, f_w = exp(m_w - M), sum and
+  // merge the four waves, a tile of columns at a time: M = max m_w, f_w = exp(m_w - M), sum and
   // acc weighted by f_w in wave order (the state's max in natural units: max * ln 2)
-  float* red = reinterpret_cast<float*>(s_ring);  // [4][16 MT][HD]
+  float* red = reinterpret_cast<float*>(s_ring);  // [4][16][HD]
 #pragma unroll
-  for (uint32_t ct0 = 0; ct0 < CT; ct0 += MT) {
-    const uint32_t nlc = ncols > 16u * ct0 ? min(ncols - 16u * ct0, 16u * MT) : 0u;  // these tiles'
+  for (uint32_t ct = 0; ct < CT; ++ct) {
+    const uint32_t nlc = ncols > 16u * ct ? min(ncols - 16u * ct, 16u) : 0u;  // this tile's
     if (nlc == 0) break;  // uniform
-    if (ct0) lds_barrier();  // the previous merge is done with red and the st arrays
+    if (ct) lds_barrier();  // the previous tile's merge is done with red and the st arrays
+    const float mr = m_run[ct] * 0.6931471805599453f;
+    float l = l_run[ct] + __shfl_xor(l_run[ct], 16, 64);
+    l = l + __shfl_xor(l, 32, 64);
+    if (qq == 0) {
+      st_m[wave][qi] = mr;
+      st_l[wave][qi] = l;
+    }
+    if (qi < nlc) {
 #pragma unroll
-    for (uint32_t c1 = 0; c1 < MT; ++c1) {
-      const uint32_t ct = ct0 + c1, col = 16u * c1 + qi;
-      const float mr = m_run[ct] * 0.6931471805599453f;
-      float l = l_run[ct] + __shfl_xor(l_run[ct], 16, 64);
-      l = l + __shfl_xor(l, 32, 64);
-      if (qq == 0) {
-        st_m[wave][col] = mr;
-        st_l[wave][col] = l;
-      }
-      if (col < nlc) {
-#pragma unroll
-        for (uint32_t tt = 0; tt < NT; ++tt)
-          *reinterpret_cast<f4_t*>(red + (wave * 16u * MT + col) * HD + 16u * tt + 4u * qq) = acc[ct][tt];
-      }
+      for (uint32_t tt = 0; tt < NT; ++tt)
+        *reinterpret_cast<f4_t*>(red + (wave * 16u + qi) * HD + 16u * tt + 4u * qq) = acc[ct][tt];
     }
     lds_barrier();
     if (t < nlc) {
@@ -773,13 +756,13 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     lds_barrier();
     // four dims per thread
     for (uint32_t idx = t; idx < nlc * (HD / 4u); idx += 256u) {
-      const uint32_t g = idx / (HD / 4u), dd = 4u * (idx % (HD / 4u)), c = 16u * ct0 + g, row = r_lo + c / GQA;
+      const uint32_t g = idx / (HD / 4u), dd = 4u * (idx % (HD / 4u)), c = 16u * ct + g, row = r_lo + c / GQA;
       // a row whose keys end before this block has no partial here
       if (blk * s >= row_len(row)) continue;
       f4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (uint32_t w2 = 0; w2 < 4; ++w2) {
-        const f4_t x = *reinterpret_cast<const f4_t*>(red + (w2 * 16u * MT + g) * HD + dd);
+        const f4_t x = *reinterpret_cast<const f4_t*>(red + (w2 * 16u + g) * HD + dd);
         const float f = st_f[w2][g];
 #pragma unroll
         for (uint32_t e = 0; e < 4; ++e) v[e] = __builtin_fmaf(x[e], f, v[e]);

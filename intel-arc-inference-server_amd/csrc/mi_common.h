@@ -147,16 +147,26 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
 }
 
+// v_permlane16_swap and v_permlane32_swap of a and b: with a == b they leave rows (0, 0, 2, 2) / (1, 1, 3, 3)
+// and halves (lo, lo) / (hi, hi) in the two registers, no LDS round trip. Written as assembly: the
+// compiler's builtin for these swaps dropped the second result here.
+__device__ __forceinline__ void lane_swap16(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void lane_swap32(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+
 // The 64-lane pairwise tree v[i] += v[i + st], st = 32 .. 1, whose root lands in lane 0, on the vector
 // ALUs: st = 32 and 16 by lane swaps of v with itself (halves, then rows of 16), 8 .. 1 by DPP row
 // shifts. Lane 0 adds exactly the pairs that __shfl_down would give it, without an LDS round trip per
 // step; every lane gets the root.
 __device__ __forceinline__ float wave_tree64(float v) {
   float a = v, b = v;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  lane_swap32(a, b);
   a = a + b;
   b = a;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  lane_swap16(a, b);
   v = a + b;
   v += dpp_f<0x108>(v);  // row_shl:8, 4, 2, 1: lane i of a row of 16 gets lane i + st
   v += dpp_f<0x104>(v);
@@ -164,6 +174,7 @@ __device__ __forceinline__ float wave_tree64(float v) {
   v += dpp_f<0x101>(v);
   return lane_f(v, 0);
 }
+
 // sum_{g < n} p[g] from +0 in ascending g, p in LDS: the words read 32 / 16 / 4 at a time in
 // 16-byte reads (p 16-byte aligned), so the chain of adds waits on the LDS a few times rather
 // than once per word (80 words: about 3 us as a loop of single reads, under 1 so)
@@ -197,6 +208,15 @@ __device__ __forceinline__ float lds_seq_sum(const float* p, uint32_t n) {
   return tot;
 }
 
+// two fp32 values as f16 pairs, high and low parts (v_cvt_pk_f16_f32 rounds to nearest; the
+// remainder v - h is exact in fp32: one v_fma_mix_f32 with neg1 = -1, which the compiler may not
+// know to be -1 - it would make the fma a conversion and a subtraction)
+__device__ __forceinline__ void f16_parts(float v0, float v1, float neg1, uint32_t& hi, uint32_t& lo) {
+  const h2_t h = __builtin_convertvector((f2_t{v0, v1}), h2_t);
+  const float l0 = __builtin_fmaf((float)h.x, neg1, v0), l1 = __builtin_fmaf((float)h.y, neg1, v1);
+  hi = h2_bits(h);
+  lo = h2_bits(__builtin_convertvector((f2_t{l0, l1}), h2_t));
+}
 
 // Orders LDS between the lanes of one wave: lanes that hand data to each other through LDS
 // need it between the writes and the reads (and before the next writes). Without it the

@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_w4a16_kernel(const uint32_t*
 // weights and its activations (in the A operand's own layout, from L2) D groups ahead. The waves'
 // sums are added through LDS in ascending k.
 template <bool SILU, uint32_t RI, uint32_t KW, uint32_t D>
-__global__ __launch_bounds__(64 * KW, KW > 8 ? 4 : 2) void gemm_w4a16_few_kernel(
+__global__ __launch_bounds__(64 * KW, 2) void gemm_w4a16_few_kernel(
     const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ x,
     float* __restrict__ out, uint16_t* __restrict__ h_out, uint32_t T, uint32_t K, uint32_t N) {
   constexpr uint32_t BM = 16u * RI;
@@ -407,8 +407,8 @@ __global__ __launch_bounds__(64 * KW, KW > 8 ? 4 : 2) void gemm_w4a16_few_kernel
 // ---------------------------------------------------------------------------------------------
 // The decode kernels take one row at a time through every expert it routes to, which for a
 // chunk reads each expert's weights once per routed row. Here the chunk's (row, slot) pairs are
-// grouped by expert first (moe_group_kernel), so each expert's weights stream once per 64 of
-// its pairs through the MFMA tile of gemm_w4a16_kernel (moe_gemm_kernel: layout-1 weights,
+// grouped by expert first (moe_group_kernel), so each expert's weights stream once per 32, 64 or
+// 96 of its pairs through the MFMA tile of gemm_w4a16_kernel (moe_gemm_kernel: layout-1 weights,
 // gathered activation rows, scattered outputs), and the slot-ordered combine with the residual
 // (moe.cl:383-470's epilogue, moe_ref.h:144-152) runs per row afterwards.
 constexpr uint32_t kMoeRouteWords = 32, kMoeW = 8, kMoeSG = 16;  // the route row (moe.cl:49-56)
@@ -716,7 +716,7 @@ struct PrefillAttnArgs {
   uint32_t page, T, pos0, q_heads;
   float scale;
   // KV8: fp16 row scales at row * sc_row_stride + head * sc_head_stride, and the output in
-  // the cache's rotated basis, fp32 [T][q_heads][HD], for the un-rotation pass
+  // the output in the cache's rotated basis, fp32 [T][q_heads][HD]
   const uint16_t* k_scale;
   const uint16_t* v_scale;
   size_t sc_row_stride, sc_head_stride;
@@ -736,35 +736,17 @@ __device__ __forceinline__ u4_t widen_i8x8(uint32_t x0, uint32_t x1) {
               h2_bits(as_h2(__builtin_amdgcn_perm(hi, x1, 0x04030402u)) - bias)};
 }
 
-// The max over the four lanes l % 16 + 16 k that hold one column's scores: v_permlane16_swap and
-// v_permlane32_swap of x with a copy of itself leave rows (0, 0, 2, 2) / (1, 1, 3, 3) and halves
-// (lo, lo) / (hi, hi) in the two registers (no LDS round trip; assembly as in csrc/attn_dma.h).
-__device__ __forceinline__ void swap16(float& a0, float& a1) {
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a0), "+v"(a1));
-}
-__device__ __forceinline__ void swap32(float& a0, float& a1) {
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a0), "+v"(a1));
-}
 // (v_maximum3_f32: fmaxf would quieten each operand first, an instruction per operand)
 __device__ __forceinline__ float max3(float x, float y, float z) {
   return __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y), z);
 }
+// the max over the four lanes l % 16 + 16 k that hold one column's scores
 __device__ __forceinline__ float col_max(float x) {
   float a0 = x, a1 = x;
-  swap16(a0, a1);
+  lane_swap16(a0, a1);
   float b0 = __builtin_elementwise_maximum(a0, a1), b1 = b0;
-  swap32(b0, b1);
+  lane_swap32(b0, b1);
   return __builtin_elementwise_maximum(b0, b1);
-}
-
-// two fp32 values as f16 pairs, high and low parts (v_cvt_pk_f16_f32 rounds to nearest; the
-// remainder v - h is exact in fp32: one v_fma_mix_f32 with neg1 = -1, which the compiler may not
-// know to be -1 - it would make the fma a conversion and a subtraction)
-__device__ __forceinline__ void split_pair(float v0, float v1, float neg1, uint32_t& hi, uint32_t& lo) {
-  const h2_t h = __builtin_convertvector((f2_t{v0, v1}), h2_t);
-  const float l0 = __builtin_fmaf((float)h.x, neg1, v0), l1 = __builtin_fmaf((float)h.y, neg1, v1);
-  hi = h2_bits(h);
-  lo = h2_bits(__builtin_convertvector((f2_t{l0, l1}), h2_t));
 }
 
 // 8 consecutive elements of a cache row as loaded, and as f16
@@ -788,7 +770,7 @@ struct KvPiece<1> {
 // taking the column tiles of w % 4 and the keys 32 (w / 4) .. of each 32 NS-key iteration (the NS
 // partial results of a column merge through LDS at the end, in ascending key part).
 template <int HD, int GQA, int KV8, int NC, int CT, int NS>
-__global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_prefill_kernel(PrefillAttnArgs a) {
+__global__ __launch_bounds__(64 * NC * NS, 2) void attn_prefill_kernel(PrefillAttnArgs a) {
   constexpr uint32_t KK = HD / 32, NT = HD / 16;
   constexpr uint32_t COLS = 16 * CT * NC, RB = COLS / GQA;  // columns and rows per work-group
   constexpr uint32_t KB = 32 * NS;                      // keys per iteration
@@ -883,10 +865,10 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
       const f4_t q1 = *reinterpret_cast<const f4_t*>(qp + 32u * kk + 4) * sgn;
       u4_t h, l;
       uint32_t hh, ll;
-      split_pair(q0.x, q0.y, neg1, hh, ll); h.x = hh; l.x = ll;
-      split_pair(q0.z, q0.w, neg1, hh, ll); h.y = hh; l.y = ll;
-      split_pair(q1.x, q1.y, neg1, hh, ll); h.z = hh; l.z = ll;
-      split_pair(q1.z, q1.w, neg1, hh, ll); h.w = hh; l.w = ll;
+      f16_parts(q0.x, q0.y, neg1, hh, ll); h.x = hh; l.x = ll;
+      f16_parts(q0.z, q0.w, neg1, hh, ll); h.y = hh; l.y = ll;
+      f16_parts(q1.x, q1.y, neg1, hh, ll); h.z = hh; l.z = ll;
+      f16_parts(q1.z, q1.w, neg1, hh, ll); h.w = hh; l.w = ll;
       qh[ct][kk] = __builtin_bit_cast(h8_t, h);
       ql[ct][kk] = __builtin_bit_cast(h8_t, l);
     }
@@ -983,10 +965,10 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
           for (uint32_t e = 0; e < 8; ++e) w[e] *= vscale[e / 4][e % 4];
         }
         uint32_t hh, ll;
-        split_pair(w[0], w[1], neg1, hh, ll); bh[ct].x = hh; bl[ct].x = ll;
-        split_pair(w[2], w[3], neg1, hh, ll); bh[ct].y = hh; bl[ct].y = ll;
-        split_pair(w[4], w[5], neg1, hh, ll); bh[ct].z = hh; bl[ct].z = ll;
-        split_pair(w[6], w[7], neg1, hh, ll); bh[ct].w = hh; bl[ct].w = ll;
+        f16_parts(w[0], w[1], neg1, hh, ll); bh[ct].x = hh; bl[ct].x = ll;
+        f16_parts(w[2], w[3], neg1, hh, ll); bh[ct].y = hh; bl[ct].y = ll;
+        f16_parts(w[4], w[5], neg1, hh, ll); bh[ct].z = hh; bl[ct].z = ll;
+        f16_parts(w[6], w[7], neg1, hh, ll); bh[ct].w = hh; bl[ct].w = ll;
       }
       // O^T += V^T P^T: the products' 32 k are the keys 4 qq + e of the two groups, which is how
       // the lanes hold the weights; V^T of 4 keys comes from one transposing read (lane 4 jj + h
@@ -1021,9 +1003,9 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
 #pragma unroll
   for (uint32_t ct = 0; ct < CT; ++ct) {
     float a0 = l_run[ct], a1 = l_run[ct];
-    swap16(a0, a1);
+    lane_swap16(a0, a1);
     float b0 = a0 + a1, b1 = b0;
-    swap32(b0, b1);
+    lane_swap32(b0, b1);
     l[ct] = b0 + b1;
   }
   if constexpr (NS > 1) {
@@ -1084,9 +1066,9 @@ __global__ __launch_bounds__(64 * NC * NS, CT * HD > 256 ? 1 : 2) void attn_pref
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) {
           float a0 = y2[r], a1 = y2[r];
-          swap16(a0, a1);
+          lane_swap16(a0, a1);
           float b0 = (qq & 1u) ? a0 - a1 : a0 + a1, b1 = b0;
-          swap32(b0, b1);
+          lane_swap32(b0, b1);
           y2[r] = (qq & 2u) ? b0 - b1 : b0 + b1;
         }
         acc[ct][tt] = y2;
@@ -1122,17 +1104,27 @@ void launch_prefill_gqa(const PrefillAttnArgs& a, uint32_t kv_heads, uint32_t cu
   // 175 in one part; 333 rows over 1333: 32 / 44), but not for 64 keys or fewer (64 rows at position
   // 0: 6.6 / 7.4, int8 12.4 / 14.9); up to 32 columns at rows of 128 two column tiles and the keys in
   // four parts (3 rows over 8003: 77 / 131; 6 over 506: 11.1 / 13.5).
-  constexpr int CT = HD == 128 ? 2 : 1;
-  constexpr uint32_t RB = 64 * CT / GQA, R1 = 64 / GQA;
-  const uint32_t wide = kv_heads * ((a.T + RB - 1) / RB), narrow = kv_heads * ((a.T + R1 - 1) / R1);
-  if (CT > 1 && wide > cus)
-    attn_prefill_kernel<HD, GQA, KV8, 4, CT, 1><<<dim3(kv_heads, (a.T + RB - 1) / RB), 256, 0, st>>>(a);
-  else if (narrow > cus || a.pos0 + a.T <= 64)
-    attn_prefill_kernel<HD, GQA, KV8, 4, 1, 1><<<dim3(kv_heads, (a.T + R1 - 1) / R1), 256, 0, st>>>(a);
-  else if (HD == 128 && a.T * GQA <= 32)
-    attn_prefill_kernel<HD, GQA, KV8, 2, 1, (HD == 128 ? 4 : 2)><<<dim3(kv_heads, 1), (HD == 128 ? 512 : 256), 0, st>>>(a);
-  else
-    attn_prefill_kernel<HD, GQA, KV8, 4, 1, 2><<<dim3(kv_heads, (a.T + R1 - 1) / R1), 512, 0, st>>>(a);
+  constexpr uint32_t R1 = 64 / GQA;
+  const uint32_t narrow = (a.T + R1 - 1) / R1;
+  if constexpr (HD == 128) {
+    constexpr uint32_t R2 = 128 / GQA;
+    const uint32_t wide = (a.T + R2 - 1) / R2;
+    if (kv_heads * wide > cus) {
+      attn_prefill_kernel<HD, GQA, KV8, 4, 2, 1><<<dim3(kv_heads, wide), 256, 0, st>>>(a);
+      return;
+    }
+  }
+  if (kv_heads * narrow > cus || a.pos0 + a.T <= 64) {
+    attn_prefill_kernel<HD, GQA, KV8, 4, 1, 1><<<dim3(kv_heads, narrow), 256, 0, st>>>(a);
+    return;
+  }
+  if constexpr (HD == 128) {
+    if (a.T * GQA <= 32) {
+      attn_prefill_kernel<HD, GQA, KV8, 2, 1, 4><<<dim3(kv_heads, 1), 512, 0, st>>>(a);
+      return;
+    }
+  }
+  attn_prefill_kernel<HD, GQA, KV8, 4, 1, 2><<<dim3(kv_heads, narrow), 512, 0, st>>>(a);
 }
 
 template <int HD, int KV8>
