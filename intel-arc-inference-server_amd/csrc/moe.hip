@@ -524,7 +524,9 @@ __global__ __launch_bounds__(NT) void moe_down_kernel(const uint32_t* __restrict
   __shared__ __align__(16) uint16_t s_h[kMaxSlotsInter / 64 * kXs];
   __shared__ __align__(16) float s_t[9][8][16];  // [slot][column][group], inter <= 1024
   __shared__ float s_d[9][8];
-  if (dnm.x && blockIdx.y == M) {  // the norm row (uniform; its work-groups' first 256 threads)
+  // the norm row: its work-groups' first 256 threads (whole waves: the others end here, and an ended
+  // wave no longer counts at the consumer's barriers)
+  if (dnm.x && blockIdx.y == M) {
     if (blockIdx.x < M && threadIdx.x < 256u)
       down_norm_consumer(dnm, blockIdx.x, hidden, reinterpret_cast<uint32_t*>(s_h), &s_t[0][0][0]);
     return;
@@ -639,7 +641,11 @@ extern "C" int mi_gemv_f16w(const uint16_t* w_tiled, const uint16_t* x, float* o
   if (reinterpret_cast<uintptr_t>(x) % 16) return mi_fail(MI_ERR_ARG, "gemv_f16w: x needs 16-byte alignment");
   hipStream_t st = static_cast<hipStream_t>(stream);
   // 8 rows per work-group: the 2048-row router of 272 columns 73 us (4 rows 88; 16 rows 86, whose 640
-  // work-groups leave the second of two rounds a quarter full)
+  // work-groups leave the second of two rounds a quarter full). From 64 rows on (us, one row per work-group /
+  // this; 16 slices): 2048 x 272 48 rows 9.2 / 12.4, 64 11.2 / 12.5, 96 14.6 / 12.5, 256 30 / 12.5; 4096 x 144 64
+  // rows 14.6 / 21.7, 128 21.8 / 21.8, 256 35 / 21.8; 2048 x 80 64 rows 6.1 / 12.4, 256 11.4 / 12.5, 384 16 / 12.5;
+  // 2048 x 2048 8 rows 9.4 / 12.4, 16 16 / 12.5, 64 54 / 12.8. They cross at 900 to 1400 of the one-row kernel's
+  // work-groups, so the line at 64 rows is early for narrow routers and late for wide linears.
   constexpr uint32_t R = 8;
   if (M >= 64)
     gemv_f16w_rows_kernel<R><<<dim3((N + 63) / 64, (M + R - 1) / R), 64 * ksplit, 0, st>>>(w_tiled, x, out, M, K, N,
