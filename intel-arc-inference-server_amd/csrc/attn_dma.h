@@ -601,7 +601,10 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
       }
 #pragma unroll
     for (uint32_t ct = 0; ct < CT; ++ct) {
-      if (16u * ct >= ncols) break;  // uniform: no row in this tile
+      // no row in this tile (uniform). One tile always has one, and at f16 rows the branch that is never
+      // taken held loads back (one row of 16 / 2 heads of 256 at 30000 keys 22.2 -> 21.4 us, of 8 / 1 at 65000 30.0 -> 27.9);
+      // int8 rows are slower without it (31.2 -> 31.6) and keep it.
+      if ((CT > 1 || KV8 == 1) && 16u * ct >= ncols) break;
       // scores S^T[position 4 qq + r][column 16 ct + qi]: the f16 high and low parts of q on
       // two chains
       f4_t dh[NG], dl[NG];
