@@ -157,6 +157,15 @@ __device__ __forceinline__ void lane_swap32(float& a, float& b) {
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
 }
 
+// four pairs at once: they share the wait states on either side
+#define MI_SWAP4(ROWS)                                                                                          \
+  asm volatile("s_nop 1\n\tv_permlane" ROWS "_swap_b32 %0, %4\n\tv_permlane" ROWS "_swap_b32 %1, %5\n\t"       \
+               "v_permlane" ROWS "_swap_b32 %2, %6\n\tv_permlane" ROWS "_swap_b32 %3, %7\n\ts_nop 1"           \
+               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]))
+__device__ __forceinline__ void lane_swap16(float (&a)[4], float (&b)[4]) { MI_SWAP4("16"); }
+__device__ __forceinline__ void lane_swap32(float (&a)[4], float (&b)[4]) { MI_SWAP4("32"); }
+#undef MI_SWAP4
+
 // The 64-lane pairwise tree v[i] += v[i + st], st = 32 .. 1, whose root lands in lane 0, on the vector
 // ALUs: st = 32 and 16 by lane swaps of v with itself (halves, then rows of 16), 8 .. 1 by DPP row
 // shifts. Lane 0 adds exactly the pairs that __shfl_down would give it, without an LDS round trip per

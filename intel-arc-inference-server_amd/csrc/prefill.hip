@@ -1055,22 +1055,24 @@ __global__ __launch_bounds__(64 * NC * NS, 2) void attn_prefill_kernel(PrefillAt
         for (uint32_t tt = 0; tt < NT; ++tt) *reinterpret_cast<f4_any*>(a.out_rot + o + 16u * tt) = acc[ct][tt];
       }
       // FWHT(s * y): the stages h = 1 .. 128 in order, the pair (i, i + h) becoming (a + c, a - c):
-      // h = 1, 2 inside the four values, 4 and 8 across the lane groups, 16 .. 128 across the tiles
+      // h = 1, 2 inside the four values, 4 and 8 across the lane groups (four swaps together: apart, their
+      // wait states took 0.6 us of a few rows' 9.4), 16 .. 128 across the tiles
 #pragma unroll
       for (uint32_t tt = 0; tt < NT; ++tt) {
         f4_t y;
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) y[r] = kv8_flip(acc[ct][tt][r], kv8_sign_neg(16u * tt + 4u * qq + r));
         const f4_t y1 = {y[0] + y[1], y[0] - y[1], y[2] + y[3], y[2] - y[3]};
-        f4_t y2 = {y1[0] + y1[2], y1[1] + y1[3], y1[0] - y1[2], y1[1] - y1[3]};
+        float u0[4] = {y1[0] + y1[2], y1[1] + y1[3], y1[0] - y1[2], y1[1] - y1[3]}, u1[4], v0[4], v1[4];
 #pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) {
-          float a0 = y2[r], a1 = y2[r];
-          lane_swap16(a0, a1);
-          float b0 = (qq & 1u) ? a0 - a1 : a0 + a1, b1 = b0;
-          lane_swap32(b0, b1);
-          y2[r] = (qq & 2u) ? b0 - b1 : b0 + b1;
-        }
+        for (uint32_t r = 0; r < 4; ++r) u1[r] = u0[r];
+        lane_swap16(u0, u1);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) v0[r] = v1[r] = (qq & 1u) ? u0[r] - u1[r] : u0[r] + u1[r];
+        lane_swap32(v0, v1);
+        f4_t y2;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) y2[r] = (qq & 2u) ? v0[r] - v1[r] : v0[r] + v1[r];
         acc[ct][tt] = y2;
       }
 #pragma unroll
