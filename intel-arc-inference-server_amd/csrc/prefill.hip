@@ -49,9 +49,9 @@
 //     buffer after the products: one barrier per iteration, no wait for the load's latency;
 //   * the accumulators follow the running maximum only when it has risen by more than 2^8, the
 //     f16 parts come from v_cvt_pk_f16_f32 and v_fma_mix_f32.
-// Measured (MI355X, 40 / 8 heads of 128, 2048 rows): 180 -> 86 us, 500 TFLOP/s of attention products
-// or 1.0 PFLOP/s with the low parts (45 % of the matrix cores' time at 98 us, counters); 16 / 2 heads of 256,
-// int8, 777 rows at position 3001: 375 -> 126 us; one step per 16 keys on 16x16x16 products before.
+// Measured (MI355X, 40 / 8 heads of 128, 2048 rows): 180 -> 84 us, 510 TFLOP/s of attention products or 1.0 PFLOP/s
+// with the low parts (45 % of the matrix cores' cycles at 2.4 GHz, counters); 16 / 2 heads of 256, int8, 777 rows at
+// position 3001: 375 -> 129 us; one step per 16 keys on 16x16x16 products before.
 #include <algorithm>
 #include <string>
 
