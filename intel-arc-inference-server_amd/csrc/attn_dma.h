@@ -491,7 +491,9 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
     return fmaxf(b0, b1);
   };
   static_assert(NB % NG == 0, "ring");
+  // (a template argument would drop the partials' own 4-byte alignment)
   typedef float f4a_t __attribute__((ext_vector_type(4), aligned(4)));
+  typedef f4a_t __attribute__((address_space(1)))* f4a_g;
   typedef int v2i_t __attribute__((ext_vector_type(2)));
   typedef short v4s_t __attribute__((ext_vector_type(4)));
   constexpr uint32_t NTR = KV8 ? NT / 2 : NT;  // transposing reads per group
@@ -771,7 +773,7 @@ __device__ __forceinline__ void attn_block_dma(const AttnDecodeArgs& a, uint32_t
         for (uint32_t e = 0; e < 4; ++e) v[e] = __builtin_fmaf(x[e], f, v[e]);
       }
       float* out = a.attn_part + (((size_t)(j * GQA + c % GQA) * a.tgt + blk) * a.M + row) * (HD + 2);
-      *as_global(reinterpret_cast<f4a_t*>(out + 2 + dd)) = v;
+      *(f4a_g)(as_global(out) + 2 + dd) = v;
       if (dd == 0) {
         out[0] = st_hm[g];
         out[1] = st_hs[g];

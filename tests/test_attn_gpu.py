@@ -246,6 +246,28 @@ def test_rows_paged_bitwise_contiguous(kind, QH, KVH, HD):
         assert np.array_equal(one[0], b[m]), m
 
 
+@pytest.mark.parametrize("kind,QH,KVH,HD,M", [(0, 40, 8, 128, 1), (1, 40, 8, 128, 4), (0, 16, 2, 256, 3)])
+def test_partials_at_their_own_alignment(kind, QH, KVH, HD, M):
+    """attn_part one float off 16 bytes: the same partials, and nothing beside them."""
+    Lm, tgt, pos = 512, 4, 300
+    sh = O.attn_shape(QH, KVH, HD)
+    k, v, ks, vs = make_kv(kind, KVH, Lm, HD, 7)
+    n = QH * tgt * M * (HD + 2)
+    ctrl, shp = ctrl_dev(pos, M), mi.shape_ref(sh)
+    keep = [dev(a) for a in (np.random.default_rng(7).standard_normal((M, QH, HD)).astype(np.float32), k, v, ks, vs)]
+    got = []
+    for off in (0, 1):
+        part = dev(np.zeros(n + 8, np.float32))
+        print(f"attn partials kind={kind} HD={HD} M={M} off={off}", flush=True)
+        mi.call("mi_attn_decode", ptr(ctrl), ptr(keep[0]), kind, *[ptr(a) for a in keep[1:]], HD, Lm * HD, 1, Lm, None, 0, Lm,
+                ptr(part) + 4 * off, M, tgt, shp, stream())
+        sync()
+        got.append(host(part, np.uint32))
+    assert got[0][:n].any()
+    assert np.array_equal(got[1][1:n + 1], got[0][:n])
+    assert got[1][0] == 0 and not got[1][n + 1:].any()
+
+
 def test_reduce_matches_oracle_merge_on_device_partials():
     """attn_reduce_v2's merge on the GPU's own partials: within 1 fp16 ulp of the oracle's
     sequential merge (the device forms the same sum with a common max; exp differs by <= 1
